@@ -65,6 +65,7 @@ struct fs2d_handle {
     void* sort_buf = nullptr;    // the density scatter's sorted path (scatter_sort_bytes), on the first advect
     void* render_buf = nullptr;  // device staging of the visual output, grown on demand
     size_t render_bytes = 0;
+    HostStage stage;             // host transfers (fs2d_transfer.hip)
     struct MgLevel {
         int n, R, P;
         float *p, *t, *b;  // iterate, its ping-pong partner, right-hand side
@@ -694,18 +695,6 @@ int advance(fs2d_handle* h, float diff, float visc, float dt) {
     return rc;
 }
 
-int copy_in(fs2d_handle* h, float* dst, const float* src, hipMemcpyKind kind) {
-    const size_t row = sizeof(float) * h->R;
-    FS2D_HIP(h, hipMemcpy2DAsync(dst, sizeof(float) * h->P, src, row, row, h->R, kind, h->stream));
-    return FS2D_OK;
-}
-
-int copy_out(fs2d_handle* h, float* dst, const float* src, hipMemcpyKind kind) {
-    const size_t row = sizeof(float) * h->R;
-    FS2D_HIP(h, hipMemcpy2DAsync(dst, row, src, sizeof(float) * h->P, row, h->R, kind, h->stream));
-    return FS2D_OK;
-}
-
 bool field_ok(int field) { return field >= FS2D_FIELD_DENSITY && field <= FS2D_FIELD_VELOCITY_V; }
 
 // Exceptions thrown on the host (allocation in plan building, maps and
@@ -828,6 +817,7 @@ int fs2d_hip_destroy(fs2d_handle* h) {
     if (h->res_sums) (void)hipFree(h->res_sums);
     if (h->render_buf) (void)hipFree(h->render_buf);
     if (h->sort_buf) (void)hipFree(h->sort_buf);
+    stage_free(h->stage);
     for (auto& L : h->mg)
         for (float* q : {L.p, L.t, L.b})
             if (q) (void)hipFree(q);
@@ -849,11 +839,12 @@ void* fs2d_hip_stream(fs2d_handle* h) { return h ? static_cast<void*>(h->stream)
 
 static int fs2d_hip_upload_impl(fs2d_handle* h, const float* rho, const float* u, const float* v) {
     if (!h || !rho || !u || !v) return fail(h, FS2D_ERR_ARGUMENT, "fs2d_hip_upload: NULL argument");
-    int rc;
+    RowCopies c;
+    c.add(rho, h->rho());
+    c.add(u, h->u());
+    c.add(v, h->v());
     h->speed_valid = false;
-    if ((rc = copy_in(h, h->rho(), rho, hipMemcpyHostToDevice))) return rc;
-    if ((rc = copy_in(h, h->u(), u, hipMemcpyHostToDevice))) return rc;
-    if ((rc = copy_in(h, h->v(), v, hipMemcpyHostToDevice))) return rc;
+    FS2D_HIP(h, stage_in(h->stage, h->stream, c, h->R, h->P));
     FS2D_HIP(h, hipStreamSynchronize(h->stream));
     return FS2D_OK;
 }
@@ -864,11 +855,13 @@ int fs2d_hip_upload(fs2d_handle* h, const float* rho, const float* u, const floa
 
 static int fs2d_hip_upload_device_impl(fs2d_handle* h, const float* rho, const float* u, const float* v) {
     if (!h || !rho || !u || !v) return fail(h, FS2D_ERR_ARGUMENT, "fs2d_hip_upload_device: NULL argument");
-    int rc;
+    RowCopies c;
+    c.add(rho, h->rho());
+    c.add(u, h->u());
+    c.add(v, h->v());
     h->speed_valid = false;
-    if ((rc = copy_in(h, h->rho(), rho, hipMemcpyDeviceToDevice))) return rc;
-    if ((rc = copy_in(h, h->u(), u, hipMemcpyDeviceToDevice))) return rc;
-    return copy_in(h, h->v(), v, hipMemcpyDeviceToDevice);
+    FS2D_HIP(h, launch_copy_rows(h->stream, c, h->R, h->R, h->P));
+    return FS2D_OK;
 }
 
 int fs2d_hip_upload_device(fs2d_handle* h, const float* rho, const float* u, const float* v) {
@@ -879,14 +872,12 @@ static int fs2d_hip_set_sources_impl(fs2d_handle* h, const float* rs, const floa
     if (!h) return fail(h, FS2D_ERR_ARGUMENT, "fs2d_hip_set_sources: NULL handle");
     const float* src[3] = {rs, us, vs};
     const int dst[3] = {F_RS, F_US, F_VS};
+    RowCopies c;
     for (int i = 0; i < 3; ++i) {
-        if (src[i]) {
-            int rc = copy_in(h, h->f[dst[i]], src[i], hipMemcpyHostToDevice);
-            if (rc) return rc;
-        } else {
-            FS2D_HIP(h, launch_fill(h->stream, h->f[dst[i]], 0u, h->field_bytes / 4));
-        }
+        if (src[i]) c.add(src[i], h->f[dst[i]]);
+        else FS2D_HIP(h, launch_fill(h->stream, h->f[dst[i]], 0u, h->field_bytes / 4));
     }
+    FS2D_HIP(h, stage_in(h->stage, h->stream, c, h->R, h->P));
     FS2D_HIP(h, hipStreamSynchronize(h->stream));
     return FS2D_OK;
 }
@@ -930,11 +921,11 @@ int fs2d_hip_sync(fs2d_handle* h) {
 
 static int fs2d_hip_download_impl(fs2d_handle* h, float* rho, float* u, float* v) {
     if (!h) return fail(h, FS2D_ERR_ARGUMENT, "fs2d_hip_download: NULL handle");
-    int rc;
-    if (rho && (rc = copy_out(h, rho, h->rho(), hipMemcpyDeviceToHost))) return rc;
-    if (u && (rc = copy_out(h, u, h->u(), hipMemcpyDeviceToHost))) return rc;
-    if (v && (rc = copy_out(h, v, h->v(), hipMemcpyDeviceToHost))) return rc;
-    FS2D_HIP(h, hipStreamSynchronize(h->stream));
+    RowCopies c;
+    if (rho) c.add(h->rho(), rho);
+    if (u) c.add(h->u(), u);
+    if (v) c.add(h->v(), v);
+    FS2D_HIP(h, stage_out(h->stage, h->stream, c, h->R, h->P));
     return FS2D_OK;
 }
 
@@ -944,10 +935,11 @@ int fs2d_hip_download(fs2d_handle* h, float* rho, float* u, float* v) {
 
 static int fs2d_hip_download_device_impl(fs2d_handle* h, float* rho, float* u, float* v) {
     if (!h) return fail(h, FS2D_ERR_ARGUMENT, "fs2d_hip_download_device: NULL handle");
-    int rc;
-    if (rho && (rc = copy_out(h, rho, h->rho(), hipMemcpyDeviceToDevice))) return rc;
-    if (u && (rc = copy_out(h, u, h->u(), hipMemcpyDeviceToDevice))) return rc;
-    if (v && (rc = copy_out(h, v, h->v(), hipMemcpyDeviceToDevice))) return rc;
+    RowCopies c;
+    if (rho) c.add(h->rho(), rho);
+    if (u) c.add(h->u(), u);
+    if (v) c.add(h->v(), v);
+    FS2D_HIP(h, copy_rows_in_order(h->stream, c, h->R, h->P, h->R));
     return FS2D_OK;
 }
 
@@ -961,9 +953,9 @@ static int fs2d_hip_download_pressure_impl(fs2d_handle* h, float* p) {
         std::memset(p, 0, sizeof(float) * static_cast<size_t>(h->R) * h->R);
         return FS2D_OK;
     }
-    int rc = copy_out(h, p, h->f[F_P], hipMemcpyDeviceToHost);
-    if (rc) return rc;
-    FS2D_HIP(h, hipStreamSynchronize(h->stream));
+    RowCopies c;
+    c.add(h->f[F_P], p);
+    FS2D_HIP(h, stage_out(h->stage, h->stream, c, h->R, h->P));
     return FS2D_OK;
 }
 
@@ -975,11 +967,27 @@ static int fs2d_hip_solve_impl(fs2d_handle* h, float* rho, const float* rho_src,
                    const float* u_src, const float* v_src, float visc, float dt) {
     if (!h || !rho || !rho_src || !u || !v || !u_src || !v_src)
         return fail(h, FS2D_ERR_ARGUMENT, "fs2d_hip_solve: NULL argument");
+    // All six arrays in one transfer; the step and the read-back follow on the
+    // stream, and the one wait is stage_out's.
+    RowCopies in, out;
+    in.add(rho, h->rho());
+    in.add(u, h->u());
+    in.add(v, h->v());
+    in.add(rho_src, h->f[F_RS]);
+    in.add(u_src, h->f[F_US]);
+    in.add(v_src, h->f[F_VS]);
+    h->speed_valid = false;
+    FS2D_HIP(h, stage_in(h->stage, h->stream, in, h->R, h->P));
     int rc;
-    if ((rc = fs2d_hip_upload(h, rho, u, v))) return rc;
-    if ((rc = fs2d_hip_set_sources(h, rho_src, u_src, v_src))) return rc;
-    if ((rc = advance(h, diff, visc, dt))) return rc;
-    return fs2d_hip_download(h, rho, u, v);
+    if ((rc = advance(h, diff, visc, dt))) {
+        (void)hipStreamSynchronize(h->stream);  // the staging buffer is the host's again
+        return rc;
+    }
+    out.add(h->rho(), rho);
+    out.add(h->u(), u);
+    out.add(h->v(), v);
+    FS2D_HIP(h, stage_out(h->stage, h->stream, out, h->R, h->P));
+    return FS2D_OK;
 }
 
 int fs2d_hip_solve(fs2d_handle* h, float* rho, const float* rho_src, float diff, float* u, float* v,

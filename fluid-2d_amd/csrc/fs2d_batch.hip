@@ -319,6 +319,7 @@ struct fs2d_batch {
     long long interior = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    HostStage stage;  // host transfers (fs2d_transfer.hip)
     Roles roles{};
     BatchSim* sims = nullptr;     // device copy of host_sims
     int2* cell_work = nullptr;    // single-pass stage blocks, all simulations
@@ -636,22 +637,6 @@ int advance(fs2d_batch* b) {
     return FS2D_OK;
 }
 
-int copy_sim(fs2d_batch* b, int sim, float* dst_arena, const float* host) {
-    const BatchSim& S = b->host_sims[sim];
-    const size_t row = sizeof(float) * S.R;
-    FS2D_BHIP(b, hipMemcpy2DAsync(dst_arena + S.off, sizeof(float) * S.P, host, row, row, S.R,
-                                  hipMemcpyHostToDevice, b->stream));
-    return FS2D_OK;
-}
-
-int copy_sim_out(fs2d_batch* b, int sim, float* host, const float* src_arena) {
-    const BatchSim& S = b->host_sims[sim];
-    const size_t row = sizeof(float) * S.R;
-    FS2D_BHIP(b, hipMemcpy2DAsync(host, row, src_arena + S.off, sizeof(float) * S.P, row, S.R,
-                                  hipMemcpyDeviceToHost, b->stream));
-    return FS2D_OK;
-}
-
 // Exceptions thrown on the host (allocation in plan building, maps and
 // vectors) never cross the C ABI: they become an error code and message.
 template <class F>
@@ -686,6 +671,7 @@ int fs2d_hip_batch_destroy(fs2d_batch* b) {
     if (b->scatter_windows) (void)hipFree(b->scatter_windows);
     if (b->scatter_scratch) (void)hipFree(b->scatter_scratch);
     if (b->scatter_flag) (void)hipFree(b->scatter_flag);
+    stage_free(b->stage);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -841,11 +827,13 @@ int fs2d_hip_batch_create(int count, const fs2d_batch_sim* sims, const fs2d_para
 static int fs2d_hip_batch_upload_impl(fs2d_batch* b, int sim, const float* rho, const float* u, const float* v) {
     if (!b || sim < 0 || sim >= (b ? b->count : 0) || !rho || !u || !v)
         return bfail(b, FS2D_ERR_ARGUMENT, "fs2d_hip_batch_upload: bad argument");
-    int rc;
+    const BatchSim& S = b->host_sims[sim];
+    RowCopies c;
+    c.add(rho, b->roles.a[A_RHO] + S.off);
+    c.add(u, b->roles.a[A_U] + S.off);
+    c.add(v, b->roles.a[A_V] + S.off);
     b->speed_valid = false;
-    if ((rc = copy_sim(b, sim, b->roles.a[A_RHO], rho))) return rc;
-    if ((rc = copy_sim(b, sim, b->roles.a[A_U], u))) return rc;
-    if ((rc = copy_sim(b, sim, b->roles.a[A_V], v))) return rc;
+    FS2D_BHIP(b, stage_in(b->stage, b->stream, c, S.R, S.P));
     FS2D_BHIP(b, hipStreamSynchronize(b->stream));
     return FS2D_OK;
 }
@@ -860,16 +848,17 @@ static int fs2d_hip_batch_set_sources_impl(fs2d_batch* b, int sim, const float* 
     const int dst[3] = {A_RS, A_US, A_VS};
     const BatchSim& S = b->host_sims[sim];
     const size_t n = static_cast<size_t>(S.R) * S.P;
+    RowCopies c;
     for (int i = 0; i < 3; ++i) {
         if (src[i]) {
-            int rc = copy_sim(b, sim, b->roles.a[dst[i]], src[i]);
-            if (rc) return rc;
+            c.add(src[i], b->roles.a[dst[i]] + S.off);
         } else {
             hipLaunchKernelGGL(kb_fill, dim3((unsigned)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 4096))),
                                dim3(256), 0, b->stream, reinterpret_cast<uint32_t*>(b->roles.a[dst[i]] + S.off), n);
             FS2D_BHIP(b, hipGetLastError());
         }
     }
+    FS2D_BHIP(b, stage_in(b->stage, b->stream, c, S.R, S.P));
     FS2D_BHIP(b, hipStreamSynchronize(b->stream));
     return FS2D_OK;
 }
@@ -893,11 +882,12 @@ int fs2d_hip_batch_step_n(fs2d_batch* b, int n) {
 
 static int fs2d_hip_batch_download_impl(fs2d_batch* b, int sim, float* rho, float* u, float* v) {
     if (!b || sim < 0 || sim >= b->count) return bfail(b, FS2D_ERR_ARGUMENT, "fs2d_hip_batch_download: bad argument");
-    int rc;
-    if (rho && (rc = copy_sim_out(b, sim, rho, b->roles.a[A_RHO]))) return rc;
-    if (u && (rc = copy_sim_out(b, sim, u, b->roles.a[A_U]))) return rc;
-    if (v && (rc = copy_sim_out(b, sim, v, b->roles.a[A_V]))) return rc;
-    FS2D_BHIP(b, hipStreamSynchronize(b->stream));
+    const BatchSim& S = b->host_sims[sim];
+    RowCopies c;
+    if (rho) c.add(b->roles.a[A_RHO] + S.off, rho);
+    if (u) c.add(b->roles.a[A_U] + S.off, u);
+    if (v) c.add(b->roles.a[A_V] + S.off, v);
+    FS2D_BHIP(b, stage_out(b->stage, b->stream, c, S.R, S.P));
     return FS2D_OK;
 }
 

@@ -167,6 +167,36 @@ hipError_t launch_set_boundary(hipStream_t s, float* x, int R, int P, Ring ring)
 hipError_t launch_copy4(hipStream_t s, float4* dst, const float4* src, size_t n4);
 hipError_t launch_fill(hipStream_t s, void* p, uint32_t value, size_t n_words);
 
+// Rows of unpadded R x R arrays and of pitched fields (fs2d_transfer.hip):
+// `count` copies of R rows of R floats, source pitch sp, destination pitch dp
+// (floats), in one launch; copy_rows_in_order splits it where destinations
+// overlap.
+struct RowCopies {
+    static constexpr int kMax = 6;
+    const float* src[kMax] = {};
+    float* dst[kMax] = {};
+    int count = 0;
+    void add(const float* s, float* d) {
+        src[count] = s;
+        dst[count++] = d;
+    }
+};
+hipError_t launch_copy_rows(hipStream_t s, const RowCopies& c, int R, int sp, int dp);
+hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int sp, int dp);
+// Host arrays (src, unpadded) into fields (dst, pitch P), and fields (src) out
+// to host arrays (dst).  The buffers are grown on demand and belong to one
+// stream.  stage_in enqueues: the stream is synchronised before the next use of
+// the buffers by the host (stage_out does so itself and returns with the data
+// in place).
+struct HostStage {
+    float* pin = nullptr;  // pinned host memory
+    float* dev = nullptr;  // one unpadded array
+    size_t pin_floats = 0, dev_floats = 0;
+};
+hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P);
+hipError_t stage_out(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P);
+void stage_free(HostStage& h);
+
 // Visual output (fs2d_render.hip): density -> RGBA8 (R * R * 4 bytes), velocity
 // -> line vertices (R * R lines of 40 bytes), both unpitched, row-major.
 hipError_t launch_render_density(hipStream_t s, const float* d, int R, int P, float mr, float mg, float mb,

@@ -1,0 +1,145 @@
+// fs2d_transfer.hip -- fields in and out of the device: rows between a
+// caller's unpadded R x R arrays and the pitched fields.
+//
+// What bounds it: a transfer from or to pageable host memory, by PCIe and by
+// the runtime's own work per call.  A pitched copy of pageable memory
+// (hipMemcpy2DAsync) is issued row by row, about 9 us each: 2.4 ms for one
+// 256 x 256 field in, 1.7 ms out, whatever its bytes.  So rows are never copied one by
+// one here: host arrays move as whole ranges, and a kernel places the rows.
+//   * Up to kPinnedStage bytes per call, the arrays are copied into (or out
+//     of) a pinned buffer by the host, and one kernel moves all of them
+//     between that buffer, read and written over PCIe, and the fields: one
+//     launch and one wait per call.  Measured: a 256 x 256 array in, 18 us
+//     alone with its launch and wait; 1026 x 1026, 55 us of host copy and 86 us of kernel.
+//   * Larger transfers take hipMemcpyAsync on each whole array (31-35 GB/s in
+//     and 18 GB/s out of pageable memory from 1026 x 1026 up: 134 us in) and a
+//     device buffer of one array.  The two ways cost the same at about 4 MB
+//     an array; the line lies below that, at 8 MB a call, which also bounds
+//     what a handle pins.
+#include "fs2d_internal.hpp"
+
+#include <cstring>
+
+namespace fs2d {
+namespace {
+
+constexpr size_t kPinnedStage = size_t(8) << 20;
+
+// Field blockIdx.z, row blockIdx.y.
+__global__ __launch_bounds__(256) void k_copy_rows(RowCopies c, int R, int sp, int dp) {
+    const float* __restrict__ s = c.src[blockIdx.z] + (size_t)blockIdx.y * sp;
+    float* __restrict__ d = c.dst[blockIdx.z] + (size_t)blockIdx.y * dp;
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    if (j < R) d[j] = s[j];
+}
+
+// The stream's device is current while this lives (a handle may be read from a
+// thread whose current device is another).
+struct OnDeviceOf {
+    int saved = -1;
+    explicit OnDeviceOf(hipStream_t s) {
+        hipDevice_t want = 0;
+        int have = 0;
+        if (hipStreamGetDevice(s, &want) != hipSuccess || hipGetDevice(&have) != hipSuccess || have == want) return;
+        if (hipSetDevice(want) == hipSuccess) saved = have;
+    }
+    ~OnDeviceOf() {
+        if (saved >= 0) (void)hipSetDevice(saved);
+    }
+};
+
+hipError_t grow(float** p, size_t* have, size_t floats, hipStream_t s, bool pinned) {
+    if (*have >= floats) return hipSuccess;
+    hipError_t e = hipStreamSynchronize(s);  // the old buffer may be in use
+    if (e != hipSuccess) return e;
+    if (*p) (void)(pinned ? hipHostFree(*p) : hipFree(*p));
+    *p = nullptr;
+    *have = 0;
+    void* q = nullptr;
+    e = pinned ? hipHostMalloc(&q, floats * sizeof(float), hipHostMallocDefault) : hipMalloc(&q, floats * sizeof(float));
+    if (e != hipSuccess) return e;
+    *p = static_cast<float*>(q);
+    *have = floats;
+    return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t launch_copy_rows(hipStream_t s, const RowCopies& c, int R, int sp, int dp) {
+    if (c.count <= 0) return hipSuccess;
+    const OnDeviceOf device(s);
+    const dim3 grid((R + 255) / 256, R, c.count);
+    hipLaunchKernelGGL(k_copy_rows, grid, dim3(256), 0, s, c, R, sp, dp);
+    return hipGetLastError();
+}
+
+// A later array wins where two destinations overlap, as with copies made one
+// after the other: such a set is copied by one launch per array.
+hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int sp, int dp) {
+    const size_t span = (size_t)(R - 1) * dp + R;
+    bool apart = true;
+    for (int a = 0; a < c.count; ++a)
+        for (int b = 0; b < a; ++b) apart = apart && (c.dst[a] + span <= c.dst[b] || c.dst[b] + span <= c.dst[a]);
+    if (apart) return launch_copy_rows(s, c, R, sp, dp);
+    for (int a = 0; a < c.count; ++a) {
+        RowCopies one;
+        one.add(c.src[a], c.dst[a]);
+        const hipError_t e = launch_copy_rows(s, one, R, sp, dp);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P) {
+    const OnDeviceOf device(s);
+    const size_t n = (size_t)R * R, bytes = n * sizeof(float);
+    hipError_t e;
+    if (c.count * bytes <= kPinnedStage) {
+        if ((e = grow(&h.pin, &h.pin_floats, c.count * n, s, true)) != hipSuccess) return e;
+        RowCopies d = c;
+        for (int k = 0; k < c.count; ++k) {
+            std::memcpy(h.pin + k * n, c.src[k], bytes);
+            d.src[k] = h.pin + k * n;
+        }
+        return launch_copy_rows(s, d, R, R, P);
+    }
+    if ((e = grow(&h.dev, &h.dev_floats, n, s, false)) != hipSuccess) return e;
+    for (int k = 0; k < c.count; ++k) {
+        RowCopies one;
+        one.add(h.dev, c.dst[k]);
+        if ((e = hipMemcpyAsync(h.dev, c.src[k], bytes, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+        if ((e = launch_copy_rows(s, one, R, R, P)) != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t stage_out(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P) {
+    const OnDeviceOf device(s);
+    const size_t n = (size_t)R * R, bytes = n * sizeof(float);
+    hipError_t e;
+    if (c.count * bytes <= kPinnedStage) {
+        if ((e = grow(&h.pin, &h.pin_floats, c.count * n, s, true)) != hipSuccess) return e;
+        RowCopies d = c;
+        for (int k = 0; k < c.count; ++k) d.dst[k] = h.pin + k * n;
+        if ((e = launch_copy_rows(s, d, R, P, R)) != hipSuccess) return e;
+        if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+        for (int k = 0; k < c.count; ++k) std::memcpy(c.dst[k], h.pin + k * n, bytes);
+        return hipSuccess;
+    }
+    if ((e = grow(&h.dev, &h.dev_floats, n, s, false)) != hipSuccess) return e;
+    for (int k = 0; k < c.count; ++k) {
+        RowCopies one;
+        one.add(c.src[k], h.dev);
+        if ((e = launch_copy_rows(s, one, R, P, R)) != hipSuccess) return e;
+        if ((e = hipMemcpyAsync(c.dst[k], h.dev, bytes, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+    }
+    return hipStreamSynchronize(s);
+}
+
+void stage_free(HostStage& h) {
+    if (h.pin) (void)hipHostFree(h.pin);
+    if (h.dev) (void)hipFree(h.dev);
+    h = HostStage{};
+}
+
+}  // namespace fs2d
