@@ -66,9 +66,13 @@ struct Layer {
     long count() const { return wn + cout; }
 };
 
-// Activation and gradient buffers of one (N, H, W) shape.
+// Activation and gradient buffers of one (N, H, W) shape, and how many blocks
+// share each layer's weight gradient (partial sums at `part` of the buffer
+// "part", for training).
 struct Acts {
     int N = 0, H = 0, W = 0;
+    int splits[kNumLayers] = {};
+    long part[kNumLayers] = {}, part_floats = 0;
     std::map<std::string, void*> buf;
     bf16* operator()(const char* k) const { return static_cast<bf16*>(buf.at(k)); }
     float* f(const char* k) const { return static_cast<float*>(buf.at(k)); }
@@ -88,6 +92,7 @@ struct fs2d_net {
     float* loss = nullptr;  // device scalar
     double* scal = nullptr;  // device: sums of squares and the scale (prediction on fields)
     std::map<std::tuple<int, int, int>, Acts*> acts;
+    HostStage stage;  // host transfers (fs2d_transfer.hip)
     std::string err;
 };
 
@@ -128,26 +133,37 @@ struct Rng {
 int real_cin(int l) { return l == E1A ? 2 : kLayers[l].cin; }
 int real_cout(int l) { return l == OUT ? 1 : kLayers[l].cout; }
 
+// The bf16 weights, and the data gradient's (flipped and transposed).
 int refresh_bf16(fs2d_net* n) {
-    for (auto& L : n->layer)
+    for (auto& L : n->layer) {
         hipLaunchKernelGGL(k_to_bf16, dim3(blocks_for(L.wn)), dim3(256), 0, n->stream, L.p, L.w16, L.wn);
+        hipLaunchKernelGGL(k_flip_weights, dim3(blocks_for(L.wn)), dim3(256), 0, n->stream, L.w16, L.wt16, L.cin, L.cout);
+    }
     NHIP(n, hipGetLastError());
     return FS2D_OK;
 }
 
 // One 3x3 convolution launch: the LDS-staged kernel where the image tiles into
-// 8 x 16 pixel blocks, the direct one otherwise (the small 1/8-scale levels).
-int launch_conv(fs2d_net* n, const bf16* x, int N, int H, int W, int Cin, const bf16* w, const float* bias, void* y,
-                int Cout, int relu, bool f32_out) {
-    const int tiles = Cout / 16;
+// 8 x 16 pixel blocks, the direct one otherwise (the coarse levels of small or
+// odd fields; the two add the same products in different orders, so which one
+// runs is part of a shape's results).  The LDS kernel's tile is 16 rows (4 a
+// wave) where that leaves 4 blocks a CU or more, else 8.
+int launch_conv(fs2d_net* n, const bf16* x, int N, int H, int W, int Cin, const bf16* w, const ConvOut& o,
+                bool f32_out) {
+    const int tiles = o.Cout / 16;
     const int nt = tiles % 4 == 0 ? 4 : (tiles % 3 == 0 ? 3 : (tiles % 2 == 0 ? 2 : 1));
     const dim3 blk(256);
+    if (f32_out && nt != 1) return nfail(n, FS2D_ERR_ARGUMENT, "conv: fp32 output needs 16 channels");
     if (H % 8 == 0 && W % 16 == 0) {
-        const dim3 grid(static_cast<unsigned>(static_cast<long>(N) * (H / 8) * (W / 16)), tiles / nt);
-#define FS2D_CONV_LDS(NT_, F32_) \
-    hipLaunchKernelGGL((k_conv3x3_lds<NT_, F32_>), grid, blk, 0, n->stream, x, N, H, W, Cin, w, bias, y, Cout, relu)
-        if (f32_out && nt == 1) FS2D_CONV_LDS(1, true);
-        else if (f32_out) return nfail(n, FS2D_ERR_ARGUMENT, "conv: fp32 output needs 16 channels");
+        const long per_row = static_cast<long>(N) * (W / 16) * (tiles / nt);
+        const bool tall = per_row * ((H + 15) / 16) >= 1024;
+        const dim3 grid(static_cast<unsigned>(static_cast<long>(N) * (tall ? (H + 15) / 16 : H / 8) * (W / 16)), tiles / nt);
+#define FS2D_CONV_LDS(NT_, F32_)                                                                                  \
+    do {                                                                                                          \
+        if (tall) hipLaunchKernelGGL((k_conv3x3_lds<NT_, 4, F32_>), grid, blk, 0, n->stream, x, N, H, W, Cin, w, o); \
+        else hipLaunchKernelGGL((k_conv3x3_lds<NT_, 2, F32_>), grid, blk, 0, n->stream, x, N, H, W, Cin, w, o);      \
+    } while (0)
+        if (f32_out) FS2D_CONV_LDS(1, true);
         else if (nt == 4) FS2D_CONV_LDS(4, false);
         else if (nt == 3) FS2D_CONV_LDS(3, false);
         else if (nt == 2) FS2D_CONV_LDS(2, false);
@@ -157,9 +173,8 @@ int launch_conv(fs2d_net* n, const bf16* x, int N, int H, int W, int Cin, const 
         const long npix = static_cast<long>(N) * H * W;
         const dim3 grid(static_cast<unsigned>((npix / 16 + CONV_WAVES - 1) / CONV_WAVES), tiles / nt);
 #define FS2D_CONV(NT_, F32_) \
-    hipLaunchKernelGGL((k_conv3x3<NT_, F32_>), grid, blk, 0, n->stream, x, N, H, W, Cin, w, bias, y, Cout, relu)
-        if (f32_out && nt == 1) FS2D_CONV(1, true);
-        else if (f32_out) return nfail(n, FS2D_ERR_ARGUMENT, "conv: fp32 output needs 16 channels");
+    hipLaunchKernelGGL((k_conv3x3<NT_, F32_>), grid, blk, 0, n->stream, x, N, H, W, Cin, w, o)
+        if (f32_out) FS2D_CONV(1, true);
         else if (nt == 4) FS2D_CONV(4, false);
         else if (nt == 3) FS2D_CONV(3, false);
         else if (nt == 2) FS2D_CONV(2, false);
@@ -172,37 +187,60 @@ int launch_conv(fs2d_net* n, const bf16* x, int N, int H, int W, int Cin, const 
 
 int conv(fs2d_net* n, int l, const bf16* x, void* y, int N, int H, int W, bool f32_out = false) {
     const Layer& L = n->layer[l];
-    return launch_conv(n, x, N, H, W, L.cin, L.w16, L.b(), y, L.cout, L.relu ? 1 : 0, f32_out);
+    const ConvOut o{y, nullptr, nullptr, L.b(), L.cout, L.cout, L.relu ? 1 : 0};
+    return launch_conv(n, x, N, H, W, L.cin, L.w16, o, f32_out);
 }
 
-// Data gradient of layer l: dx = conv(dz, flipped transposed weights).
-int conv_dx(fs2d_net* n, int l, const bf16* dz, bf16* dx, int N, int H, int W) {
+// Data gradient of layer l: conv(dz, flipped transposed weights), channels
+// [0, Ca) into dx and the others into dx2 (a concatenation's two parts), zeroed
+// where mask, the layer's input if it came out of a ReLU, is not positive.
+int conv_dx(fs2d_net* n, int l, const bf16* dz, bf16* dx, int Ca, bf16* dx2, const bf16* mask, int N, int H, int W) {
     const Layer& L = n->layer[l];
-    hipLaunchKernelGGL(k_flip_weights, dim3(blocks_for(L.wn)), dim3(256), 0, n->stream, L.w16, L.wt16, L.cin, L.cout);
-    return launch_conv(n, dz, N, H, W, L.cout, L.wt16, nullptr, dx, L.cin, 0, false);
+    const ConvOut o{dx, dx2, mask, nullptr, L.cin, Ca, 0};
+    return launch_conv(n, dz, N, H, W, L.cout, L.wt16, o, false);
 }
 
-// Weight and bias gradients of layer l (accumulated into its gradient arena).
-int conv_dw(fs2d_net* n, int l, const bf16* x, const bf16* dz, int N, int H, int W) {
+// Channel tiles (of 16) that one block of the weight gradient takes: the wider
+// the block, the more each fragment it reads from LDS is used; 2 x 2 and 1 x 3 are
+// what the accumulators of 9 taps leave room for.
+struct WgTile {
+    int na, nb;
+};
+WgTile wgrad_tile(int l) {
+    const int cin = kLayers[l].cin, cout = kLayers[l].cout;
+    if (cout % 32) return WgTile{1, cin == 48 ? 3 : 1};
+    return WgTile{2, cin % 32 == 0 ? 2 : 1};
+}
+
+// Blocks sharing a layer's pixels: enough for one block a CU (two of the
+// narrow ones, which leave half the registers free), and no more, since each
+// writes its own partial sums.
+int wgrad_splits(int l, int N, int h, int w) {
+    const WgTile t = wgrad_tile(l);
+    const int combos = kLayers[l].cin / (16 * t.nb) * (kLayers[l].cout / (16 * t.na));
+    const long tiles = static_cast<long>(N) * ((h + WG_R - 1) / WG_R) * ((w + WG_C - 1) / WG_C);
+    const int want = std::max(1, (t.na * t.nb == 1 ? 512 : 256) / combos);
+    return static_cast<int>(std::min<long>(want, tiles));
+}
+
+// Weight and bias gradients of layer l, as partial sums.
+int conv_dw(fs2d_net* n, const Acts& a, int l, const bf16* x, const bf16* dz, int N, int H, int W) {
     const Layer& L = n->layer[l];
-    const long npix = static_cast<long>(N) * H * W;
-    const long chunk = std::max<long>(64, std::min<long>(16384, npix / 16 / 16 * 16));  // a multiple of 64
-    const long chunk64 = (chunk + 63) / 64 * 64;
-    const dim3 grid(9 * (L.cout / 16) * (L.cin / 16), static_cast<unsigned>((npix + chunk64 - 1) / chunk64));
-    hipLaunchKernelGGL(k_conv3x3_wgrad, grid, dim3(64 * CONV_WAVES), 0, n->stream, x, dz, N, H, W, L.cin, L.cout, L.g,
-                       chunk64);
-    const long bchunk = 4096;
-    hipLaunchKernelGGL(k_bias_grad, dim3(static_cast<unsigned>((npix + bchunk - 1) / bchunk)), dim3(256), 0, n->stream,
-                       dz, npix, L.cout, L.g + L.wn, bchunk);
+    const WgTile t = wgrad_tile(l);
+    const dim3 grid(a.splits[l], L.cin / (16 * t.nb) * (L.cout / (16 * t.na)));
+    float* part = a.f("part") + a.part[l];
+#define FS2D_WGRAD(NA_, NB_) \
+    hipLaunchKernelGGL((k_conv3x3_wgrad<NA_, NB_>), grid, dim3(WG_THREADS), 0, n->stream, x, dz, N, H, W, L.cin, L.cout, part)
+    if (t.na == 2 && t.nb == 2) FS2D_WGRAD(2, 2);
+    else if (t.na == 2) FS2D_WGRAD(2, 1);
+    else if (t.nb == 3) FS2D_WGRAD(1, 3);
+    else FS2D_WGRAD(1, 1);
+#undef FS2D_WGRAD
     NHIP(n, hipGetLastError());
     return FS2D_OK;
 }
 
-int relu_mask(fs2d_net* n, bf16* dy, const bf16* y, long count) {
-    hipLaunchKernelGGL(k_relu_mask, dim3(blocks_for(count)), dim3(256), 0, n->stream, dy, y, count);
-    NHIP(n, hipGetLastError());
-    return FS2D_OK;
-}
+constexpr int kSumBlocks = 64;  // blocks sharing a sample's sums of squares
 
 int acts_for(fs2d_net* n, int N, int H, int W, Acts** out) {
     const auto key = std::make_tuple(N, H, W);
@@ -221,13 +259,21 @@ int acts_for(fs2d_net* n, int N, int H, int W, Acts** out) {
         long elems;
         int bytes;
     };
+    // halvings of each layer's image: e1*, d1*, out 0; e2*, d2* 1; e3*, d3* 2; e4* 3
+    const int level[kNumLayers] = {0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 1, 1, 0, 0, 0};
+    for (int l = 0; l < kNumLayers; ++l) {
+        a->splits[l] = wgrad_splits(l, N, H >> level[l], W >> level[l]);
+        a->part[l] = a->part_floats;
+        a->part_floats += a->splits[l] * n->layer[l].count();
+    }
     const B list[] = {
         {"x0", p1 * 16, 2},  {"a1", p1 * 16, 2},  {"e1", p1 * 16, 2},  {"p1", p2 * 16, 2},  {"a2", p2 * 32, 2},
         {"e2", p2 * 32, 2},  {"p2", p3 * 32, 2},  {"a3", p3 * 64, 2},  {"e3", p3 * 64, 2},  {"p3", p4 * 64, 2},
         {"a4", p4 * 128, 2}, {"e4", p4 * 128, 2}, {"c3", p3 * 192, 2}, {"b3", p3 * 64, 2},
         {"d3", p3 * 64, 2},  {"c2", p2 * 96, 2},  {"b2", p2 * 32, 2},  {"d2", p2 * 32, 2},
-        {"c1", p1 * 48, 2},  {"b1", p1 * 16, 2},  {"d1", p1 * 16, 2},  {"o", p1 * 16, 4},
-        {"prev", p1, 4},     {"tgt", p1, 4},      {"scale", N, 4},
+        {"c1", p1 * 48, 2},  {"b1", p1 * 16, 2},  {"d1", p1 * 16, 2},  {"o", p1, 4},
+        {"prev", p1, 4},     {"tgt", p1, 4},      {"scale", N, 4},      {"inv", N, 4},
+        {"sums", static_cast<long>(N) * kSumBlocks * 2, 8},             {"part", a->part_floats, 4},
         // gradients
         {"dO", p1 * 16, 2},  {"gA", p1 * 48, 2},  {"gB", p1 * 48, 2},  {"gS1", p1 * 16, 2}, {"gS2", p2 * 32, 2},
         {"gS3", p3 * 64, 2},
@@ -247,12 +293,12 @@ int acts_for(fs2d_net* n, int N, int H, int W, Acts** out) {
     return FS2D_OK;
 }
 
-// Forward pass on a->x0 into a->o (fp32, channel 0 meaningful).
+// Forward pass on a->x0 into a->o (fp32, one value a pixel).
 int forward(fs2d_net* n, Acts& a) {
     const int N = a.N, H = a.H, W = a.W;
     int rc;
     auto pool = [&](const bf16* x, bf16* y, int h, int w, int C) {
-        hipLaunchKernelGGL(k_avgpool2, dim3(blocks_for(static_cast<long>(N) * h * w * C / 4)), dim3(256), 0, n->stream,
+        hipLaunchKernelGGL(k_avgpool2, dim3(blocks_for(static_cast<long>(N) * h * w * C / 32)), dim3(256), 0, n->stream,
                            x, y, N, h, w, C);
     };
     // upsample the coarse level and concatenate the skip in one pass
@@ -285,93 +331,75 @@ int forward(fs2d_net* n, Acts& a) {
     return FS2D_OK;
 }
 
-// Backward pass from a->dO (set by the loss); accumulates every layer's gradients.
+// Backward pass from a->dO (set by the loss): every layer's weight gradients as
+// partial sums.  gA and gB hold the gradient of one layer's output in turn,
+// already through that output's ReLU: whichever kernel writes it applies the mask.
 int backward(fs2d_net* n, Acts& a) {
     const int N = a.N, H = a.H, W = a.W;
-    const long p1 = static_cast<long>(N) * H * W, p2 = p1 / 4, p3 = p1 / 16, p4 = p1 / 64;
     int rc;
     bf16 *gA = a("gA"), *gB = a("gB");
-    auto split = [&](const bf16* dy, bf16* da, bf16* db, long np, int Ca, int Cb) {
-        hipLaunchKernelGGL(k_split, dim3(blocks_for(np * (Ca + Cb))), dim3(256), 0, n->stream, dy, da, db, np, Ca, Cb);
+    auto up_bwd = [&](const bf16* dy, const bf16* mask, bf16* dx, int h, int w, int C) {
+        hipLaunchKernelGGL(k_upsample2_bwd, dim3(blocks_for(static_cast<long>(N) * h * w * (C / 8))), dim3(256), 0,
+                           n->stream, dy, mask, dx, N, h, w, C);
     };
-    auto up_bwd = [&](const bf16* dy, bf16* dx, int h, int w, int C) {
-        hipLaunchKernelGGL(k_upsample2_bwd, dim3(blocks_for(static_cast<long>(N) * h * w * C)), dim3(256), 0,
-                           n->stream, dy, dx, N, h, w, C);
+    auto pool_bwd = [&](const bf16* dy, const bf16* skip, const bf16* mask, bf16* out, int h, int w, int C) {
+        hipLaunchKernelGGL(k_pool_bwd_add, dim3(blocks_for(static_cast<long>(N) * h * w * (C / 8))), dim3(256), 0,
+                           n->stream, dy, skip, mask, out, N, h, w, C);
     };
-    auto pool_bwd = [&](const bf16* dy, const bf16* skip, bf16* out, int h, int w, int C) {
-        hipLaunchKernelGGL(k_pool_bwd_add, dim3(blocks_for(static_cast<long>(N) * h * w * C)), dim3(256), 0,
-                           n->stream, dy, skip, out, N, h, w, C);
-    };
-    // layer step: mask dy by the layer's ReLU output y, weight gradients from
-    // its input x, data gradient into dx (if given)
-    auto layer_bwd = [&](int l, const bf16* x, const bf16* y, bf16* dy, bf16* dx, int h, int w) -> int {
-        const Layer& L = n->layer[l];
-        const long np = static_cast<long>(N) * h * w;
-        int r;
-        if (L.relu && (r = relu_mask(n, dy, y, np * L.cout))) return r;
-        if ((r = conv_dw(n, l, x, dy, N, h, w))) return r;
-        if (dx && (r = conv_dx(n, l, dy, dx, N, h, w))) return r;
-        return FS2D_OK;
+    // layer step: weight gradients from the layer's input x and its output's
+    // gradient dz, then the data gradient into dx (through x's own ReLU where mask
+    // is x), split after Ca channels into dx and dx2
+    auto layer_bwd = [&](int l, const bf16* x, const bf16* dz, bf16* dx, const bf16* mask, int h, int w, int Ca = 0,
+                         bf16* dx2 = nullptr) -> int {
+        const int r = conv_dw(n, a, l, x, dz, N, h, w);
+        return r ? r : conv_dx(n, l, dz, dx, Ca ? Ca : n->layer[l].cin, dx2, mask, N, h, w);
     };
     // level 1 decoder
-    if ((rc = layer_bwd(OUT, a("d1"), nullptr, a("dO"), gA, H, W))) return rc;  // gA: dd1 (16)
-    if ((rc = layer_bwd(D1B, a("b1"), a("d1"), gA, gB, H, W))) return rc;       // gB: db1 (16)
-    if ((rc = layer_bwd(D1A, a("c1"), a("b1"), gB, gA, H, W))) return rc;       // gA: dc1 (48)
-    split(gA, gB, a("gS1"), p1, 32, 16);                                         // gB: du1 (32), gS1: e1 skip
-    up_bwd(gB, gA, H / 2, W / 2, 32);                                            // gA: dd2 (32 @ H/2)
-    if ((rc = layer_bwd(D2B, a("b2"), a("d2"), gA, gB, H / 2, W / 2))) return rc;  // gB: db2 (32)
-    if ((rc = layer_bwd(D2A, a("c2"), a("b2"), gB, gA, H / 2, W / 2))) return rc;  // gA: dc2 (96)
-    split(gA, gB, a("gS2"), p2, 64, 32);                                           // gB: du2 (64), gS2
-    up_bwd(gB, gA, H / 4, W / 4, 64);                                              // gA: dd3 (64 @ H/4)
-    if ((rc = layer_bwd(D3B, a("b3"), a("d3"), gA, gB, H / 4, W / 4))) return rc;  // gB: db3
-    if ((rc = layer_bwd(D3A, a("c3"), a("b3"), gB, gA, H / 4, W / 4))) return rc;  // gA: dc3 (192)
-    split(gA, gB, a("gS3"), p3, 128, 64);                                          // gB: du3 (128), gS3
-    up_bwd(gB, gA, H / 8, W / 8, 128);                                             // gA: de4 (128 @ H/8)
-    if ((rc = layer_bwd(E4B, a("a4"), a("e4"), gA, gB, H / 8, W / 8))) return rc;  // gB: da4
-    if ((rc = layer_bwd(E4A, a("p3"), a("a4"), gB, gA, H / 8, W / 8))) return rc;  // gA: dp3 (64 @ H/8)
-    pool_bwd(gA, a("gS3"), gB, H / 4, W / 4, 64);                                  // gB: de3
-    if ((rc = layer_bwd(E3B, a("a3"), a("e3"), gB, gA, H / 4, W / 4))) return rc;  // gA: da3
-    if ((rc = layer_bwd(E3A, a("p2"), a("a3"), gA, gB, H / 4, W / 4))) return rc;  // gB: dp2 (32 @ H/4)
-    pool_bwd(gB, a("gS2"), gA, H / 2, W / 2, 32);                                  // gA: de2
-    if ((rc = layer_bwd(E2B, a("a2"), a("e2"), gA, gB, H / 2, W / 2))) return rc;  // gB: da2
-    if ((rc = layer_bwd(E2A, a("p1"), a("a2"), gB, gA, H / 2, W / 2))) return rc;  // gA: dp1 (16 @ H/2)
-    pool_bwd(gA, a("gS1"), gB, H, W, 16);                                          // gB: de1
-    if ((rc = layer_bwd(E1B, a("a1"), a("e1"), gB, gA, H, W))) return rc;          // gA: da1
-    if ((rc = layer_bwd(E1A, a("x0"), a("a1"), gA, nullptr, H, W))) return rc;
-    (void)p4;
+    if ((rc = layer_bwd(OUT, a("d1"), a("dO"), gA, a("d1"), H, W))) return rc;         // gA: dd1 (16)
+    if ((rc = layer_bwd(D1B, a("b1"), gA, gB, a("b1"), H, W))) return rc;              // gB: db1 (16)
+    if ((rc = layer_bwd(D1A, a("c1"), gB, gA, nullptr, H, W, 32, a("gS1")))) return rc;  // gA: du1 (32), gS1: e1 skip
+    up_bwd(gA, a("d2"), gB, H / 2, W / 2, 32);                                         // gB: dd2 (32 @ H/2)
+    if ((rc = layer_bwd(D2B, a("b2"), gB, gA, a("b2"), H / 2, W / 2))) return rc;      // gA: db2 (32)
+    if ((rc = layer_bwd(D2A, a("c2"), gA, gB, nullptr, H / 2, W / 2, 64, a("gS2")))) return rc;  // gB: du2 (64), gS2
+    up_bwd(gB, a("d3"), gA, H / 4, W / 4, 64);                                         // gA: dd3 (64 @ H/4)
+    if ((rc = layer_bwd(D3B, a("b3"), gA, gB, a("b3"), H / 4, W / 4))) return rc;      // gB: db3
+    if ((rc = layer_bwd(D3A, a("c3"), gB, gA, nullptr, H / 4, W / 4, 128, a("gS3")))) return rc;  // gA: du3 (128), gS3
+    up_bwd(gA, a("e4"), gB, H / 8, W / 8, 128);                                        // gB: de4 (128 @ H/8)
+    if ((rc = layer_bwd(E4B, a("a4"), gB, gA, a("a4"), H / 8, W / 8))) return rc;      // gA: da4
+    if ((rc = layer_bwd(E4A, a("p3"), gA, gB, nullptr, H / 8, W / 8))) return rc;      // gB: dp3 (64 @ H/8)
+    pool_bwd(gB, a("gS3"), a("e3"), gA, H / 4, W / 4, 64);                             // gA: de3
+    if ((rc = layer_bwd(E3B, a("a3"), gA, gB, a("a3"), H / 4, W / 4))) return rc;      // gB: da3
+    if ((rc = layer_bwd(E3A, a("p2"), gB, gA, nullptr, H / 4, W / 4))) return rc;      // gA: dp2 (32 @ H/4)
+    pool_bwd(gA, a("gS2"), a("e2"), gB, H / 2, W / 2, 32);                             // gB: de2
+    if ((rc = layer_bwd(E2B, a("a2"), gB, gA, a("a2"), H / 2, W / 2))) return rc;      // gA: da2
+    if ((rc = layer_bwd(E2A, a("p1"), gA, gB, nullptr, H / 2, W / 2))) return rc;      // gB: dp1 (16 @ H/2)
+    pool_bwd(gB, a("gS1"), a("e1"), gA, H, W, 16);                                     // gA: de1
+    if ((rc = layer_bwd(E1B, a("a1"), gA, gB, a("a1"), H, W))) return rc;              // gB: da1
+    if ((rc = conv_dw(n, a, E1A, a("x0"), gB, N, H, W))) return rc;
     NHIP(n, hipGetLastError());
     return FS2D_OK;
 }
 
-// Pack host samples: s = RMS of the previous pressure (else of the
-// divergence, else 1); x0 = (d / s, prev / s, 0...) in bf16; prev and target
-// in fp32 divided by s.
-void pack_host(int N, int H, int W, const float* d, const float* prev, const float* target, std::vector<bf16>& x0,
-               std::vector<float>& pv, std::vector<float>& tg, std::vector<float>& scale) {
-    const long hw = static_cast<long>(H) * W;
-    x0.assign(static_cast<size_t>(N) * hw * 16, 0);
-    pv.resize(static_cast<size_t>(N) * hw);
-    tg.resize(target ? static_cast<size_t>(N) * hw : 0);
-    scale.resize(N);
-    for (int b = 0; b < N; ++b) {
-        double sp = 0, sd = 0;
-        for (long q = 0; q < hw; ++q) {
-            sp += static_cast<double>(prev[b * hw + q]) * prev[b * hw + q];
-            sd += static_cast<double>(d[b * hw + q]) * d[b * hw + q];
-        }
-        double s = std::sqrt(sp / hw);
-        if (!(s > 0)) s = std::sqrt(sd / hw);
-        if (!(s > 0)) s = 1.0;
-        const float inv = static_cast<float>(1.0 / s);
-        scale[b] = static_cast<float>(s);
-        for (long q = 0; q < hw; ++q) {
-            const long i = b * hw + q;
-            x0[i * 16 + 0] = f2bf(d[i] * inv);
-            x0[i * 16 + 1] = f2bf(prev[i] * inv);
-            pv[i] = prev[i] * inv;
-            if (target) tg[i] = target[i] * inv;
-        }
-    }
+// Host samples to the network's input: the arrays as they are, then on the
+// device s = RMS of the previous pressure (else of the divergence, else 1),
+// x0 = (d / s, prev / s, 0...) in bf16, and prev and target in fp32 divided by s.
+// The 16-channel input is 4 to 8 times the arrays' bytes, so it is not made on
+// the host (20 ms of packing and transfer at 1024 x 1024; now 0.3 ms).
+int load_samples(fs2d_net* net, Acts& a, const float* d, const float* prev, const float* target) {
+    const long hw = static_cast<long>(a.H) * a.W, npix = a.N * hw;
+    const int G = static_cast<int>(std::min<long>(kSumBlocks, hw / 1024));
+    float* const dd = static_cast<float*>(a.buf.at("gA"));  // free until the backward pass
+    double* const sums = static_cast<double*>(a.buf.at("sums"));
+    const size_t bytes = sizeof(float) * npix;
+    NHIP(net, hipMemcpyAsync(dd, d, bytes, hipMemcpyHostToDevice, net->stream));
+    NHIP(net, hipMemcpyAsync(a.f("prev"), prev, bytes, hipMemcpyHostToDevice, net->stream));
+    hipLaunchKernelGGL(k_sumsq_samples, dim3(G, a.N), dim3(256), 0, net->stream, dd, a.f("prev"), hw, sums);
+    hipLaunchKernelGGL(k_scale_samples, dim3(a.N), dim3(64), 0, net->stream, sums, G, hw, a.f("scale"), a.f("inv"));
+    if (target) NHIP(net, hipMemcpyAsync(a.f("tgt"), target, bytes, hipMemcpyHostToDevice, net->stream));
+    hipLaunchKernelGGL(k_pack_samples, dim3(blocks_for(npix)), dim3(256), 0, net->stream, dd, a.f("prev"),
+                       target ? a.f("tgt") : nullptr, hw, npix, a.f("inv"), a("x0"), a.f("prev"), a.f("tgt"));
+    NHIP(net, hipGetLastError());
+    return FS2D_OK;
 }
 
 int check_shape(fs2d_net* net, int n, int h, int w) {
@@ -444,7 +472,7 @@ __global__ __launch_bounds__(256) void k_unpack_fields(const float* __restrict__
     for (long t = static_cast<long>(blockIdx.x) * 256 + threadIdx.x; t < static_cast<long>(n) * n;
          t += static_cast<long>(gridDim.x) * 256) {
         const int i = static_cast<int>(t / n) + 1, j = static_cast<int>(t % n) + 1;
-        const float v = (o[t * 16] + pv[t]) * s;
+        const float v = (o[t] + pv[t]) * s;
         p[static_cast<long>(i) * P + j] = v;
         if (i == 1) p[j] = v;
         if (i == n) p[static_cast<long>(R - 1) * P + j] = v;
@@ -519,6 +547,7 @@ int fs2d_net_destroy(fs2d_net* net) {
     for (float* p : {net->params, net->grads, net->m1, net->m2, net->loss})
         if (p) (void)hipFree(p);
     if (net->scal) (void)hipFree(net->scal);
+    stage_free(net->stage);
     for (auto& L : net->layer) {
         if (L.w16) (void)hipFree(L.w16);
         if (L.wt16) (void)hipFree(L.wt16);
@@ -644,30 +673,25 @@ static int fs2d_net_train_step_impl(fs2d_net* net, int n, int h, int w, const fl
     if (!d || !prev || !target || !loss) return nfail(net, FS2D_ERR_ARGUMENT, "fs2d_net_train_step: NULL argument");
     Acts* a = nullptr;
     if ((rc = acts_for(net, n, h, w, &a))) return rc;
-    std::vector<bf16> x0;
-    std::vector<float> pv, tg, sc;
-    pack_host(n, h, w, d, prev, target, x0, pv, tg, sc);
     const long npix = static_cast<long>(n) * h * w;
-    NHIP(net, hipMemcpyAsync((*a)("x0"), x0.data(), sizeof(bf16) * x0.size(), hipMemcpyHostToDevice, net->stream));
-    NHIP(net, hipMemcpyAsync(a->f("prev"), pv.data(), sizeof(float) * pv.size(), hipMemcpyHostToDevice, net->stream));
-    NHIP(net, hipMemcpyAsync(a->f("tgt"), tg.data(), sizeof(float) * tg.size(), hipMemcpyHostToDevice, net->stream));
+    if ((rc = load_samples(net, *a, d, prev, target))) return rc;
     if ((rc = forward(net, *a))) return rc;
     hipLaunchKernelGGL(k_zero_f32, dim3(1), dim3(256), 0, net->stream, net->loss, 1L);
     hipLaunchKernelGGL(k_mse, dim3(blocks_for(npix)), dim3(256), 0, net->stream, a->f("o"), a->f("prev"), a->f("tgt"),
                        npix, (*a)("dO"), net->loss);
-    hipLaunchKernelGGL(k_zero_f32, dim3(blocks_for(net->total)), dim3(256), 0, net->stream, net->grads, net->total);
     if ((rc = backward(net, *a))) return rc;
     ++net->adam_t;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.f - std::pow(b1, static_cast<float>(net->adam_t));
     const float c2 = 1.f - std::pow(b2, static_cast<float>(net->adam_t));
-    for (auto& L : net->layer) {
-        hipLaunchKernelGGL(k_adam, dim3(blocks_for(L.wn)), dim3(256), 0, net->stream, L.p, L.g, L.m, L.v, L.w16, L.wn,
-                           lr, b1, b2, 1e-8f, c1, c2);
-        hipLaunchKernelGGL(k_adam, dim3(1), dim3(256), 0, net->stream, L.p + L.wn, L.g + L.wn, L.m + L.wn,
-                           L.v + L.wn, static_cast<bf16*>(nullptr), static_cast<long>(L.cout), lr, b1, b2, 1e-8f, c1,
-                           c2);
+    LayerSpans<kNumLayers> spans;
+    for (int l = 0; l < kNumLayers; ++l) {
+        const Layer& L = net->layer[l];
+        spans.l[l] = LayerSpan{L.p - net->params, L.wn, a->part[l], a->splits[l], L.cin, L.cout, L.w16, L.wt16};
     }
+    hipLaunchKernelGGL(k_reduce_adam<kNumLayers>, dim3(static_cast<unsigned>((net->total + 63) / 64)), dim3(1024), 0,
+                       net->stream, spans, a->f("part"), net->total, net->params, net->grads, net->m1, net->m2, lr, b1,
+                       b2, 1e-8f, c1, c2);
     NHIP(net, hipGetLastError());
     float sum = 0.f;
     NHIP(net, hipMemcpyAsync(&sum, net->loss, sizeof(float), hipMemcpyDeviceToHost, net->stream));
@@ -687,17 +711,21 @@ static int fs2d_net_predict_host_impl(fs2d_net* net, int n, int h, int w, const 
     if (!d || !prev || !out) return nfail(net, FS2D_ERR_ARGUMENT, "fs2d_net_predict_host: NULL argument");
     Acts* a = nullptr;
     if ((rc = acts_for(net, n, h, w, &a))) return rc;
-    std::vector<bf16> x0;
-    std::vector<float> pv, tg, sc;
-    pack_host(n, h, w, d, prev, nullptr, x0, pv, tg, sc);
-    const long npix = static_cast<long>(n) * h * w;
-    NHIP(net, hipMemcpyAsync((*a)("x0"), x0.data(), sizeof(bf16) * x0.size(), hipMemcpyHostToDevice, net->stream));
+    const long hw = static_cast<long>(h) * w, npix = n * hw;
+    const size_t bytes = sizeof(float) * npix;
+    if ((rc = load_samples(net, *a, d, prev, nullptr))) return rc;
     if ((rc = forward(net, *a))) return rc;
-    std::vector<float> o(static_cast<size_t>(npix) * 16);
-    NHIP(net, hipMemcpyAsync(o.data(), a->f("o"), sizeof(float) * o.size(), hipMemcpyDeviceToHost, net->stream));
+    // up to the pinned buffer's size the prediction is written over PCIe by the
+    // kernel that computes it
+    float* pin = nullptr;
+    NHIP(net, stage_pinned(net->stage, net->stream, npix, &pin));
+    float* const dst = pin ? pin : static_cast<float*>(a->buf.at("gA"));
+    hipLaunchKernelGGL(k_unpack_samples, dim3(blocks_for(npix)), dim3(256), 0, net->stream, a->f("o"), a->f("prev"),
+                       a->f("scale"), hw, npix, dst);
+    NHIP(net, hipGetLastError());
+    if (!pin) NHIP(net, hipMemcpyAsync(out, dst, bytes, hipMemcpyDeviceToHost, net->stream));
     NHIP(net, hipStreamSynchronize(net->stream));
-    const long hw = static_cast<long>(h) * w;
-    for (long i = 0; i < npix; ++i) out[i] = (o[i * 16] + pv[i]) * sc[i / hw];
+    if (pin) std::memcpy(out, pin, bytes);
     return FS2D_OK;
 }
 

@@ -195,6 +195,9 @@ struct HostStage {
 };
 hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P);
 hipError_t stage_out(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P);
+// The pinned buffer itself, at least `floats` long, for a kernel to write; null
+// where that is more than a handle pins.
+hipError_t stage_pinned(HostStage& h, hipStream_t s, size_t floats, float** out);
 void stage_free(HostStage& h);
 
 // Visual output (fs2d_render.hip): density -> RGBA8 (R * R * 4 bytes), velocity

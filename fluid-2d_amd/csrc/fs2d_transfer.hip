@@ -136,6 +136,15 @@ hipError_t stage_out(HostStage& h, hipStream_t s, const RowCopies& c, int R, int
     return hipStreamSynchronize(s);
 }
 
+hipError_t stage_pinned(HostStage& h, hipStream_t s, size_t floats, float** out) {
+    *out = nullptr;
+    if (floats * sizeof(float) > kPinnedStage) return hipSuccess;
+    const OnDeviceOf device(s);
+    const hipError_t e = grow(&h.pin, &h.pin_floats, floats, s, true);
+    if (e == hipSuccess) *out = h.pin;
+    return e;
+}
+
 void stage_free(HostStage& h) {
     if (h.pin) (void)hipHostFree(h.pin);
     if (h.dev) (void)hipFree(h.dev);
