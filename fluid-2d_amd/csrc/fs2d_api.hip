@@ -61,7 +61,7 @@ struct fs2d_handle {
     bool pressure_zero = true;  // last projection had K_p == 0 (p is identically 0)
     bool speed_valid = false;   // max_bits holds max |u|, |v| of the current velocity
     long long steps_done = 0;
-    double* res_sums = nullptr;  // 2 doubles: residual sums of the seeded projection
+    double* res_sums = nullptr;  // the residual's partial sums (2 * kResidualBlocks)
     void* sort_buf = nullptr;    // the density scatter's sorted path (scatter_sort_bytes), on the first advect
     void* render_buf = nullptr;  // device staging of the visual output, grown on demand
     size_t render_bytes = 0;
@@ -1314,11 +1314,11 @@ int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches) {
 
 // ---- the seeded projection (include/fs2d_cnn.h) ---------------------------
 static int residual_of(fs2d_handle* h, double* rel) {
-    if (!h->res_sums) FS2D_HIP(h, hipMalloc(&h->res_sums, 2 * sizeof(double)));
-    FS2D_HIP(h, launch_fill(h->stream, h->res_sums, 0u, 4));
-    FS2D_HIP(h, launch_pressure_residual(h->stream, h->f[F_D], h->f[F_P], h->R, h->P, h->res_sums));
-    double sums[2] = {0, 0};
-    FS2D_HIP(h, hipMemcpyAsync(sums, h->res_sums, sizeof sums, hipMemcpyDeviceToHost, h->stream));
+    if (!h->res_sums) FS2D_HIP(h, hipMalloc(&h->res_sums, 2 * kResidualBlocks * sizeof(double)));
+    float* pin = nullptr;  // the two sums, written by the device
+    FS2D_HIP(h, stage_pinned(h->stage, h->stream, 4, &pin));
+    double* const sums = reinterpret_cast<double*>(pin);
+    FS2D_HIP(h, launch_pressure_residual(h->stream, h->f[F_D], h->f[F_P], h->R, h->P, h->res_sums, sums));
     FS2D_HIP(h, hipStreamSynchronize(h->stream));
     *rel = sums[1] > 0 ? std::sqrt(sums[0] / sums[1]) : std::sqrt(sums[0]);
     return FS2D_OK;
@@ -1337,11 +1337,13 @@ int fs2d_hip_pressure_residual(fs2d_handle* h, double* rel) {
 // is <= tol (checked every `check` sweeps) or max_sweeps have run.  A
 // non-finite residual stops it at once: a NaN or infinite iterate stays
 // non-finite under the sweeps, so the budget would be spent for nothing.
-static int jacobi_until(fs2d_handle* h, float tol, int max_sweeps, int check, int* sweeps, double* rel) {
+// rel_known: *rel already is the residual of the field as it stands.
+static int jacobi_until(fs2d_handle* h, float tol, int max_sweeps, int check, int* sweeps, double* rel,
+                        bool rel_known = false) {
     const int depth = jacobi_depth_known(h, SWEEP_PRESSURE, h->prm.pressure_iterations);
     const SweepArgs A = sweep_args(h->f[F_P], h->f[F_D], h->R, h->P, SWEEP_PRESSURE, 0.f, 0.f, BND_CONT, max_sweeps, 0);
     int rc;
-    if ((rc = residual_of(h, rel))) return rc;
+    if (!rel_known && (rc = residual_of(h, rel))) return rc;
     int done = 0, since = 0;
     while (done < max_sweeps && !(*rel <= tol) && std::isfinite(*rel)) {
         const int m = std::min(depth, max_sweeps - done);
@@ -1399,28 +1401,36 @@ static int mg_levels(fs2d_handle* h) {
 }
 
 // One V-cycle on level l (0: the handle's pressure, scratch and divergence
-// fields); the result is left in the level's iterate pointer.
-static int mg_vcycle(fs2d_handle* h, size_t l) {
+// fields), from zero where `zero` (the level's iterate is then not read); the
+// result is left in the level's iterate pointer.
+static int mg_vcycle(fs2d_handle* h, size_t l, bool zero) {
     float** p = l == 0 ? &h->f[F_P] : &h->mg[l - 1].p;
     float** t = l == 0 ? &h->f[F_SCRATCH] : &h->mg[l - 1].t;
     const float* b = l == 0 ? h->f[F_D] : h->mg[l - 1].b;
-    const int R = l == 0 ? h->R : h->mg[l - 1].R, P = l == 0 ? h->P : h->mg[l - 1].P;
-    auto smooth = [&](int count) -> int {
-        for (int k = 0; k < count; ++k) {
+    const int R = l == 0 ? h->R : h->mg[l - 1].R, P = l == 0 ? h->P : h->mg[l - 1].P, n = R - 2;
+    if (n <= kMgTailSide) {
+        const int last = h->mg.empty() ? h->R - 2 : h->mg.back().n;
+        FS2D_HIP(h, launch_mg_tail(h->stream, *p, b, n, P, static_cast<int>(h->mg.size() - l) + 1,
+                                   mg_coarsest_sweeps(last), zero, kMgOmega));
+        return FS2D_OK;
+    }
+    if (l == h->mg.size()) {  // an odd side past the tail's
+        if (zero) FS2D_HIP(h, launch_fill(h->stream, *p, 0u, static_cast<size_t>(R) * P));
+        for (int k = 0; k < mg_coarsest_sweeps(n); ++k) {
             FS2D_HIP(h, launch_mg_smooth(h->stream, *p, *t, b, R, P, kMgOmega));
             std::swap(*p, *t);
         }
         return FS2D_OK;
-    };
-    int rc;
-    if (l == h->mg.size()) return smooth(mg_coarsest_sweeps(R - 2));
-    if ((rc = smooth(kMgPre))) return rc;
+    }
+    static_assert(kMgPre == 2 && kMgPost == 2, "launch_mg_down and launch_mg_up take two sweeps each");
     fs2d_handle::MgLevel& C = h->mg[l];
-    FS2D_HIP(h, launch_mg_restrict(h->stream, *p, b, P, C.b, C.R, C.P));
-    FS2D_HIP(h, launch_fill(h->stream, C.p, 0u, static_cast<size_t>(C.R) * C.P));
-    if ((rc = mg_vcycle(h, l + 1))) return rc;
-    FS2D_HIP(h, launch_mg_prolong(h->stream, C.p, C.P, *p, R, P));
-    return smooth(kMgPost);
+    FS2D_HIP(h, launch_mg_down(h->stream, zero ? nullptr : *p, *t, b, n, P, C.b, C.P, kMgOmega));
+    std::swap(*p, *t);
+    int rc;
+    if ((rc = mg_vcycle(h, l + 1, true))) return rc;
+    FS2D_HIP(h, launch_mg_up(h->stream, *p, *t, b, n, P, C.p, C.P, kMgOmega));
+    std::swap(*p, *t);
+    return FS2D_OK;
 }
 
 static int fs2d_hip_project_seeded_impl(fs2d_handle* h, fs2d_net* net, int seed, float tol, int max_sweeps, int check,
@@ -1451,13 +1461,13 @@ static int fs2d_hip_project_seeded_impl(fs2d_handle* h, fs2d_net* net, int seed,
         for (const auto& L : h->mg)
             if (!L.p || !L.t || !L.b) return fail(h, FS2D_ERR_STATE, "fs2d_hip_project_seeded: multigrid level not allocated");
         for (int c = 0; c < kMgMaxCycles; ++c) {
-            if ((rc = mg_vcycle(h, 0))) return rc;
+            if ((rc = mg_vcycle(h, 0, c == 0))) return rc;
             fine_smooth += h->mg.empty() ? mg_coarsest_sweeps(h->R - 2) : kMgPre + kMgPost;
             if ((rc = residual_of(h, &rel))) return rc;
             if (rel <= tol) break;
         }
     }
-    if ((rc = jacobi_until(h, tol, max_sweeps, check, &sweeps, &rel))) return rc;
+    if ((rc = jacobi_until(h, tol, max_sweeps, check, &sweeps, &rel, seed == 3))) return rc;
     sweeps += fine_smooth;
     int fb = 0;
     if (keep_prev && !(rel <= tol)) {

@@ -150,10 +150,13 @@ hipError_t launch_gather_velocity(hipStream_t s, float* u1, float* v1, const flo
 // p_zero (may be null): also zero this pressure iterate, ring included.
 hipError_t launch_divergence(hipStream_t s, float* d, const float* u, const float* v, int R, int P,
                              float neg_half_h, float* p_zero);
-// sums[0] += sum ||d - L p||^2 and sums[1] += sum d^2 over the interior (FP64),
-// L the compact 5-point operator 4 p - (pN + pS + pW + pE) of the pressure
-// sweeps (src/fluid_solver_cpu.cpp:196-204) with p's stored ring.
-hipError_t launch_pressure_residual(hipStream_t s, const float* d, const float* p, int R, int P, double* sums);
+// out[0] = sum ||d - L p||^2 and out[1] = sum d^2 over the interior (FP64, in a
+// fixed order), L the compact 5-point operator 4 p - (pN + pS + pW + pE) of the
+// pressure sweeps (src/fluid_solver_cpu.cpp:196-204) with p's stored ring.
+// part: 2 * kResidualBlocks doubles of scratch; out may be pinned host memory.
+constexpr int kResidualBlocks = 1024;
+hipError_t launch_pressure_residual(hipStream_t s, const float* d, const float* p, int R, int P, double* part,
+                                    double* out);
 
 // Max-speed reduction slots: kSpeedSlots words, kSlotStride words apart
 // (separate cache lines), zero between uses.
@@ -207,15 +210,21 @@ hipError_t launch_render_density(hipStream_t s, const float* d, int R, int P, fl
 hipError_t launch_render_velocity(hipStream_t s, const float* u, const float* v, int R, int P, float hs, float vs,
                                   void* lines);
 
-// Multigrid pieces for the pressure equation with the continuous ring
-// (fs2d_mg.hip).  smooth: one weighted Jacobi sweep src -> dst.  restrict: the
-// coarse right-hand side of each coarse interior cell = the sum of the
-// residuals b - (4p - sum nbrs) of its 2 x 2 fine cells (fine side = 2 x coarse
-// side).  prolong: pf += bilinear interpolation of pc (pc's ring included).
-// Each writes the ring of what it writes.
+// Multigrid for the pressure equation with the continuous ring (fs2d_mg.hip),
+// interior side n.  smooth: one weighted Jacobi sweep src -> dst.  down: two
+// sweeps from p (null: from zero) into out, and the coarse right-hand side bc of
+// each coarse cell = the sum of the residuals b - (4p - sum nbrs) of its 2 x 2 fine
+// cells.  up: p + bilinear interpolation of pc, then two sweeps, into out (ring
+// included).  tail: a whole V-cycle of the `levels` grids from side n <=
+// kMgTailSide down, in place (ring included), from zero where `zero`.
+constexpr int kMgTailSide = 128;
 hipError_t launch_mg_smooth(hipStream_t s, const float* src, float* dst, const float* b, int R, int P, float omega);
-hipError_t launch_mg_restrict(hipStream_t s, const float* p, const float* b, int Pf, float* bc, int Rc, int Pc);
-hipError_t launch_mg_prolong(hipStream_t s, const float* pc, int Pc, float* pf, int Rf, int Pf);
+hipError_t launch_mg_down(hipStream_t s, const float* p, float* out, const float* b, int n, int P, float* bc, int Pc,
+                          float omega);
+hipError_t launch_mg_up(hipStream_t s, const float* p, float* out, const float* b, int n, int P, const float* pc,
+                        int Pc, float omega);
+hipError_t launch_mg_tail(hipStream_t s, float* p, const float* b, int n, int P, int levels, int coarsest, bool zero,
+                          float omega);
 
 // Gauss-Seidel tile wavefront: one launch per level of the tile hyperplane.
 struct GsPlan {

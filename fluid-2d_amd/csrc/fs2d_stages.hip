@@ -208,31 +208,42 @@ __global__ __launch_bounds__(256) void k_set_boundary(float* __restrict__ x, int
     }
 }
 
+// Block b sums rows b + 1, b + 1 + blocks, ... into part[2 b], part[2 b + 1].
+// (One pair of atomics a block instead made the pass 29 us at 1024 x 1024,
+// almost all of it the 4096 blocks' atomics on two words.)
 __global__ __launch_bounds__(256) void k_pressure_residual(const float* __restrict__ d, const float* __restrict__ p,
-                                                          int R, int P, double* __restrict__ sums) {
+                                                          int R, int P, double* __restrict__ part) {
     const int n = R - 2;
     double rr = 0, dd = 0;
-    for (long t = static_cast<long>(blockIdx.x) * 256 + threadIdx.x; t < static_cast<long>(n) * n;
-         t += static_cast<long>(gridDim.x) * 256) {
-        const size_t o = (size_t)(t / n + 1) * P + t % n + 1;
-        const double r = (double)d[o] - (4.0 * p[o] - (((double)p[o - P] + p[o + P]) + ((double)p[o - 1] + p[o + 1])));
-        rr += r * r;
-        dd += (double)d[o] * d[o];
-    }
+    for (int i = blockIdx.x + 1; i <= n; i += gridDim.x)
+        for (int j = threadIdx.x + 1; j <= n; j += 256) {
+            const size_t o = (size_t)i * P + j;
+            const double r = (double)d[o] - (4.0 * p[o] - (((double)p[o - P] + p[o + P]) + ((double)p[o - 1] + p[o + 1])));
+            rr += r * r;
+            dd += (double)d[o] * d[o];
+        }
     for (int off = 32; off > 0; off >>= 1) {
         rr += __shfl_xor(rr, off);
         dd += __shfl_xor(dd, off);
     }
-    __shared__ double part[2][4];
+    __shared__ double w[2][4];
     if ((threadIdx.x & 63) == 0) {
-        part[0][threadIdx.x >> 6] = rr;
-        part[1][threadIdx.x >> 6] = dd;
+        w[0][threadIdx.x >> 6] = rr;
+        w[1][threadIdx.x >> 6] = dd;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {  // one pair of atomics per block
-        atomicAdd(sums, (part[0][0] + part[0][1]) + (part[0][2] + part[0][3]));
-        atomicAdd(sums + 1, (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]));
-    }
+    if (threadIdx.x < 2)
+        part[2 * blockIdx.x + threadIdx.x] =
+            (w[threadIdx.x][0] + w[threadIdx.x][1]) + (w[threadIdx.x][2] + w[threadIdx.x][3]);
+}
+
+__global__ __launch_bounds__(128) void k_residual_fold(const double* __restrict__ part, int blocks,
+                                                      double* __restrict__ out) {
+    const int which = threadIdx.x >> 6;  // wave 0: residual, wave 1: divergence
+    double s = 0;
+    for (int b = threadIdx.x & 63; b < blocks; b += 64) s += part[2 * b + which];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if ((threadIdx.x & 63) == 0) out[which] = s;
 }
 
 __global__ __launch_bounds__(256) void k_copy4(float4* __restrict__ dst, const float4* __restrict__ src, size_t n) {
@@ -294,10 +305,11 @@ hipError_t launch_set_boundary(hipStream_t s, float* x, int R, int P, Ring ring)
     return hipGetLastError();
 }
 
-hipError_t launch_pressure_residual(hipStream_t s, const float* d, const float* p, int R, int P, double* sums) {
-    const long cells = static_cast<long>(R - 2) * (R - 2);
-    const unsigned blocks = static_cast<unsigned>(std::max<long>(1, std::min<long>((cells + 255) / 256, 1024)));
-    hipLaunchKernelGGL(k_pressure_residual, dim3(blocks), dim3(256), 0, s, d, p, R, P, sums);
+hipError_t launch_pressure_residual(hipStream_t s, const float* d, const float* p, int R, int P, double* part,
+                                    double* out) {
+    const int blocks = std::min(R - 2, kResidualBlocks);
+    hipLaunchKernelGGL(k_pressure_residual, dim3(blocks), dim3(256), 0, s, d, p, R, P, part);
+    hipLaunchKernelGGL(k_residual_fold, dim3(1), dim3(128), 0, s, part, blocks, out);
     return hipGetLastError();
 }
 
