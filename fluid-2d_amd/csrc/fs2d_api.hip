@@ -266,10 +266,12 @@ constexpr int kJacobiDefaultDepth = 4;
 // Sweeps fused per Jacobi launch: the fixed jacobi_block if one was given,
 // otherwise the depth in {1, 2, 4, 8} with the least measured time per solve,
 // chosen on the first solve of each (kind, K): one launch of each depth is
-// timed (best of two, after a warm-up) reading the live iterate and writing
-// only the scratch field.  Results are identical for every depth.  A stream
+// timed (best of two, after a warm-up) reading the live iterates and writing
+// only the scratch fields.  Results are identical for every depth.  A stream
 // under capture cannot be timed; the default depth is used then (not kept).
-int jacobi_depth_for(fs2d_handle* h, const SweepArgs& A, int* out) {
+// scratch[f]: a field to write in place of field f's iterate.
+int jacobi_depth_for(fs2d_handle* h, const SweepSet& set, float* const* scratch, int* out) {
+    const SweepArgs& A = set.a[0];
     if (h->prm.jacobi_block) {
         *out = h->prm.jacobi_block;
         return FS2D_OK;
@@ -286,6 +288,8 @@ int jacobi_depth_for(fs2d_handle* h, const SweepArgs& A, int* out) {
         *out = kJacobiDefaultDepth;
         return FS2D_OK;
     }
+    const float* src[SweepSet::kMax];
+    for (int f = 0; f < set.count; ++f) src[f] = set.a[f].x;
     float best = 0.f;
     int best_m = kJacobiDefaultDepth;
     for (int m : {1, 2, 4, 8}) {
@@ -293,7 +297,7 @@ int jacobi_depth_for(fs2d_handle* h, const SweepArgs& A, int* out) {
         float t = 0.f;
         for (int rep = 0; rep < 3; ++rep) {
             FS2D_HIP(h, hipEventRecord(h->ev0, h->stream));
-            FS2D_HIP(h, launch_jacobi_pass(h->stream, A, A.x, h->f[F_SCRATCH], A.zero_start, m, h->jacobi_kernel));
+            FS2D_HIP(h, launch_jacobi_pass(h->stream, set, src, scratch, A.zero_start, m, h->jacobi_kernel));
             FS2D_HIP(h, hipEventRecord(h->ev1, h->stream));
             FS2D_HIP(h, hipEventSynchronize(h->ev1));
             float ms = 0.f;
@@ -319,6 +323,23 @@ int jacobi_depth_known(const fs2d_handle* h, int kind, int K) {
     return it != h->jacobi_depth.end() ? it->second : kJacobiDefaultDepth;
 }
 
+// The set's Jacobi solves, fields[f] and scratch[f] the pointers that hold field
+// f's iterate and a free field: an odd launch count leaves the result in the
+// scratch field, and the two pointers are swapped.
+int jacobi_solve(fs2d_handle* h, SweepSet set, float** const* fields, float** const* scratch) {
+    float* t[SweepSet::kMax];
+    for (int f = 0; f < set.count; ++f) {
+        t[f] = *scratch[f];
+        known_quotient(set.a[f]);
+    }
+    int depth = kJacobiDefaultDepth, rc;
+    if ((rc = jacobi_depth_for(h, set, t, &depth))) return rc;
+    FS2D_HIP(h, launch_jacobi_solve(h->stream, set, t, depth, h->jacobi_kernel));
+    if (jacobi_launches(set.a[0].K, depth) & 1)
+        for (int f = 0; f < set.count; ++f) std::swap(*fields[f], *scratch[f]);
+    return FS2D_OK;
+}
+
 // K relaxation sweeps of x against b; Jacobi may leave the result in the
 // scratch field, in which case the two pointers are swapped.
 int linear_solve(fs2d_handle* h, float*& x, const float* b, int kind, float a, float denom, int mode, int K,
@@ -335,13 +356,13 @@ int linear_solve(fs2d_handle* h, float*& x, const float* b, int kind, float a, f
             A.zero_start = 0;
         }
         FS2D_HIP(h, launch_gs_solve(h->stream, *plan, A));
-    } else {
-        int depth = kJacobiDefaultDepth, rc;
-        if ((rc = jacobi_depth_for(h, A, &depth))) return rc;
-        FS2D_HIP(h, launch_jacobi_solve(h->stream, A, h->f[F_SCRATCH], depth, h->jacobi_kernel));
-        if (jacobi_launches(K, depth) & 1) std::swap(x, h->f[F_SCRATCH]);
+        return FS2D_OK;
     }
-    return FS2D_OK;
+    SweepSet set{};
+    set.a[0] = A;
+    set.count = 1;
+    float **fx = &x, **ft = &h->f[F_SCRATCH];
+    return jacobi_solve(h, set, &fx, &ft);
 }
 
 int diffuse(fs2d_handle* h, float*& x, int mode, float rate, float dt, int K) {
@@ -524,8 +545,8 @@ int joint_levels(const JointPlans& j) {
     return static_cast<int>(std::unique(lv.begin(), lv.end()) - lv.begin());
 }
 
-// The three diffuses of a step relaxed together (Gauss-Seidel unit plans):
-// density in place, u and v on fresh iterates so that the density scatter can
+// A step whose three diffuses are relaxed together (Gauss-Seidel unit plans, or
+// Jacobi block tiles): density in place, u and v on fresh iterates so that the density scatter can
 // still read the pre-step velocity (src/fluid_solver_cpu.cpp:16-24).  Same
 // results as the sequential order: the three solves share no data.
 int step_shared_diffuse(fs2d_handle* h, float diff, float visc, float dt) {
@@ -568,9 +589,16 @@ int step_shared_diffuse(fs2d_handle* h, float diff, float visc, float dt) {
             // on-load divergence, which only the pipelined first solve needs)
             return project(h, Kp);
         }
-        const GsPlan* plan = nullptr;
-        FS2D_HIP(h, gs_plan_for(h, Kd, SWEEP_DIFFUSE, &plan));
-        FS2D_HIP(h, launch_gs_solve_set(h->stream, *plan, set));
+        if (h->prm.sweep_order == FS2D_ORDER_JACOBI) {
+            // the advections' temporaries are free until the scatter
+            float** const fields[3] = {&h->f[F_RHO], &h->f[F_UN], &h->f[F_VN]};
+            float** const scratch[3] = {&h->f[F_SCRATCH], &h->f[F_T1], &h->f[F_T2]};
+            if ((rc = jacobi_solve(h, set, fields, scratch))) return rc;
+        } else {
+            const GsPlan* plan = nullptr;
+            FS2D_HIP(h, gs_plan_for(h, Kd, SWEEP_DIFFUSE, &plan));
+            FS2D_HIP(h, launch_gs_solve_set(h->stream, *plan, set));
+        }
     }
     if ((rc = advect_density(h, dt))) return rc;  // reads the pre-step u, v
     std::swap(h->u(), h->f[F_UN]);
@@ -581,12 +609,18 @@ int step_shared_diffuse(fs2d_handle* h, float diff, float visc, float dt) {
     return project(h, Kp);
 }
 
+// Whether a step's three diffuses share their launches (not with the one-sweep
+// Gauss-Seidel tiles and the LDS Jacobi blocks).
+bool shares_diffuses(const fs2d_handle* h) {
+    return h->prm.sweep_order == FS2D_ORDER_GS_LEX ? gs_units(h) : h->jacobi_kernel == FS2D_JACOBI_WAVE;
+}
+
 // fluid_solver_cpu::solve, src/fluid_solver_cpu.cpp:6-31.
 int step(fs2d_handle* h, float diff, float visc, float dt) {
     const int Kd = h->prm.diffuse_iterations, Kp = h->prm.pressure_iterations;
     const int R = h->R, P = h->P;
     int rc;
-    if (h->prm.sweep_order == FS2D_ORDER_GS_LEX && gs_units(h)) return step_shared_diffuse(h, diff, visc, dt);
+    if (shares_diffuses(h)) return step_shared_diffuse(h, diff, visc, dt);
     // density: add source, diffuse, scatter-advect (:16-18)
     FS2D_HIP(h, launch_add_sources(h->stream, h->rho(), h->f[F_X0], h->f[F_RS], R, P, dt));
     if ((rc = diffuse(h, h->rho(), BND_CONT, diff, dt, Kd))) return rc;
@@ -1149,14 +1183,24 @@ static int fs2d_hip_time_diffuse_sweeps_impl(fs2d_handle* h, float diff, float v
                                  reinterpret_cast<const float4*>(h->f[pr[1]]), n4));
     const float ad = dt * cells(R) * diff, av = dt * cells(R) * visc;
     const float dd = 1.f + 4.f * ad, dv = 1.f + 4.f * av;
+    // the Jacobi order's third free field, for the timing only
+    const bool spare_needed = h->prm.sweep_order == FS2D_ORDER_JACOBI && shares_diffuses(h);
+    float* spare = nullptr;
+    if (spare_needed) FS2D_HIP(h, hipMalloc(&spare, h->field_bytes));
+    float* const spare_field = spare;
     auto once = [&]() -> int {
         if (Kd <= 0) return FS2D_OK;
-        if (h->prm.sweep_order == FS2D_ORDER_GS_LEX && gs_units(h)) {  // as the step relaxes them
+        if (shares_diffuses(h)) {  // as the step relaxes them
             SweepSet set{};
             set.count = 3;
             set.a[0] = sweep_args(h->f[F_T1], h->f[F_X0], R, P, SWEEP_DIFFUSE, ad, dd, BND_CONT, Kd, 0);
             set.a[1] = sweep_args(h->f[F_UN], h->f[F_X0U], R, P, SWEEP_DIFFUSE, av, dv, BND_OPP_H, Kd, 0);
             set.a[2] = sweep_args(h->f[F_VN], h->f[F_X0V], R, P, SWEEP_DIFFUSE, av, dv, BND_OPP_V, Kd, 0);
+            if (h->prm.sweep_order == FS2D_ORDER_JACOBI) {
+                float** const fields[3] = {&h->f[F_T1], &h->f[F_UN], &h->f[F_VN]};
+                float** const scratch[3] = {&h->f[F_SCRATCH], &h->f[F_T2], &spare};
+                return jacobi_solve(h, set, fields, scratch);
+            }
             const GsPlan* plan = nullptr;
             FS2D_HIP(h, gs_plan_for(h, Kd, SWEEP_DIFFUSE, &plan));
             FS2D_HIP(h, launch_gs_solve_set(h->stream, *plan, set));
@@ -1167,17 +1211,26 @@ static int fs2d_hip_time_diffuse_sweeps_impl(fs2d_handle* h, float diff, float v
         if ((rc = linear_solve(h, h->f[F_UN], h->f[F_X0U], SWEEP_DIFFUSE, av, dv, BND_OPP_H, Kd, 0))) return rc;
         return linear_solve(h, h->f[F_VN], h->f[F_X0V], SWEEP_DIFFUSE, av, dv, BND_OPP_V, Kd, 0);
     };
-    int rc = once();  // warm
-    if (rc) return rc;
-    FS2D_HIP(h, hipEventRecord(h->ev0, h->stream));
-    for (int i = 0; i < reps; ++i)
-        if ((rc = once())) return rc;
-    FS2D_HIP(h, hipEventRecord(h->ev1, h->stream));
-    FS2D_HIP(h, hipEventSynchronize(h->ev1));
-    float total = 0.f;
-    FS2D_HIP(h, hipEventElapsedTime(&total, h->ev0, h->ev1));
-    *ms = total / reps;
-    return FS2D_OK;
+    auto timed = [&]() -> int {
+        int rc = once();  // warm
+        if (rc) return rc;
+        FS2D_HIP(h, hipEventRecord(h->ev0, h->stream));
+        for (int i = 0; i < reps; ++i)
+            if ((rc = once())) return rc;
+        FS2D_HIP(h, hipEventRecord(h->ev1, h->stream));
+        FS2D_HIP(h, hipEventSynchronize(h->ev1));
+        float total = 0.f;
+        FS2D_HIP(h, hipEventElapsedTime(&total, h->ev0, h->ev1));
+        *ms = total / reps;
+        return FS2D_OK;
+    };
+    const int rc = timed();
+    if (spare_needed) {
+        (void)hipStreamSynchronize(h->stream);
+        if (spare != spare_field) std::swap(h->f[F_VN], spare);  // the handle keeps its own field
+        (void)hipFree(spare);
+    }
+    return rc;
 }
 
 int fs2d_hip_time_diffuse_sweeps(fs2d_handle* h, float diff, float visc, float dt, int reps, float* ms) {
@@ -1341,13 +1394,15 @@ int fs2d_hip_pressure_residual(fs2d_handle* h, double* rel) {
 static int jacobi_until(fs2d_handle* h, float tol, int max_sweeps, int check, int* sweeps, double* rel,
                         bool rel_known = false) {
     const int depth = jacobi_depth_known(h, SWEEP_PRESSURE, h->prm.pressure_iterations);
-    const SweepArgs A = sweep_args(h->f[F_P], h->f[F_D], h->R, h->P, SWEEP_PRESSURE, 0.f, 0.f, BND_CONT, max_sweeps, 0);
+    SweepSet set{};
+    set.a[0] = sweep_args(h->f[F_P], h->f[F_D], h->R, h->P, SWEEP_PRESSURE, 0.f, 0.f, BND_CONT, max_sweeps, 0);
+    set.count = 1;
     int rc;
     if (!rel_known && (rc = residual_of(h, rel))) return rc;
     int done = 0, since = 0;
     while (done < max_sweeps && !(*rel <= tol) && std::isfinite(*rel)) {
         const int m = std::min(depth, max_sweeps - done);
-        FS2D_HIP(h, launch_jacobi_pass(h->stream, A, h->f[F_P], h->f[F_SCRATCH], 0, m, h->jacobi_kernel));
+        FS2D_HIP(h, launch_jacobi_pass(h->stream, set, &h->f[F_P], &h->f[F_SCRATCH], 0, m, h->jacobi_kernel));
         std::swap(h->f[F_P], h->f[F_SCRATCH]);
         done += m;
         since += m;

@@ -84,11 +84,17 @@ inline SweepArgs sweep_args(float* x, const float* b, int R, int P, int kind, fl
 // dividend from the division floor up, with y2 the largest float <= 1/d and
 // y2_lo = RN(1/d - y2) > 0; if so, sets A.div_checked, A.inv_hi2 and
 // A.inv_lo2, and raises A.div_lo to where RN(x y2_lo) stays normal.  The tail
-// being positive, +-inf dividends come out +-inf as well.  Decided once per
-// divisor by trying every significand of one binade (the quotients of the
-// other binades are exact power-of-two scalings of those) and cached.  Host
-// only; a diffuse solve's first call with a new divisor costs about 4-18 ms.
+// being positive, +-inf dividends come out +-inf as well.  Decided from the few
+// significands of one binade whose quotients lie next to a midpoint of two floats
+// (the quotients of the other binades are exact power-of-two scalings of those).
+// Host only, about a microsecond.
 void two_product_quotient(SweepArgs& A);
+
+// two_product_quotient, and for a power of two (d = 1 when a = 0) the pair (1 / d,
+// 2^-149): x / d is then x y2 rounded once, and the tail, too small to change a
+// finite quotient, keeps infinite dividends infinite, so the quotient is exact for
+// every dividend and div_lo is 0.  What the kernels' launchers use.
+void known_quotient(SweepArgs& A);
 
 // Up to three independent solves with the same sweep count, relaxed by the
 // same level launches (e.g. the density, u and v diffuses of one step).
@@ -264,15 +270,19 @@ hipError_t launch_gs_pipelined(hipStream_t s, const GsPlan& pd, const SweepSet& 
 // sweeps with tile columns TWd and Md sweeps per unit.
 int gs_pipeline_offset(const GsPlan& pp, int R, int Kd, int TWd, int Md);
 
-// Jacobi sweeps, `block` sweeps fused per launch, ping-ponging x -> scratch ->
-// x -> ...; after an odd number of launches the result is in scratch.
-// kernel: JACOBI_WAVE (register strips, one wave per tile, DPP lane exchange)
+// Jacobi sweeps.  kernel: JACOBI_WAVE (block tiles in registers, fs2d_jacobi.hip)
 // or JACOBI_LDS (256-thread blocks, halo exchange in LDS); identical results.
 enum JacobiKernel : int { JACOBI_WAVE = 1, JACOBI_LDS = 2 };
-hipError_t launch_jacobi_solve(hipStream_t s, const SweepArgs& a, float* scratch, int block, int kernel);
-// One launch of m fused Jacobi sweeps from src into dst (m in 1..8).
-hipError_t launch_jacobi_pass(hipStream_t s, const SweepArgs& a, const float* src, float* dst, int zero_src, int m,
-                              int kernel);
+// `block` sweeps fused per launch, ping-ponging x -> scratch -> x -> ...; after an
+// odd number of launches the result is in scratch.  The set's fields (one to three
+// of a kind, size and sweep count) share each JACOBI_WAVE launch; scratch[f] is
+// field f's.
+hipError_t launch_jacobi_solve(hipStream_t s, const SweepSet& set, float* const* scratch, int block, int kernel);
+// One launch (JACOBI_LDS: one per field) of m fused sweeps, m in 1..8, from src[f] into dst[f].
+hipError_t launch_jacobi_pass(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
+                              int zero_src, int m, int kernel);
+hipError_t launch_jacobi_tiles(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
+                               int zero_src, int m);
 int jacobi_launches(int K, int block);
 
 }  // namespace fs2d

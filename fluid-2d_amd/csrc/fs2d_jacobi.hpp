@@ -210,6 +210,177 @@ __device__ __forceinline__ void jacobi_strip(const SweepArgs& A, const float* __
     }
 }
 
+// ===================== Jacobi, block tiles ===============================
+// A block of NW waves relaxes a region of NW RPW rows x 64 columns m times (m <=
+// kTileMaxSweeps, a run-time count): wave w holds rows RPW w .. of the iterate
+// and of the right-hand side in registers, lane l column l.  West and east come
+// from lanes l -+ 1 by a full-wave DPP shift folded into the additions, north
+// and south from the wave's own rows or, at its first and last row, through
+// LDS: each sweep starts with every wave storing those two rows and one barrier
+// (two buffers, used in turn).
+//
+// Against one wave per tile (48 rows in one wave's registers) no halo lies between
+// waves, and a tile has 8 times the waves, each an eighth of the chain: a launch of
+// 8 sweeps of 258 x 258 cells took 18.6 us and takes 5.5.  The measured shapes
+// and what bounds them are in fs2d_jacobi.hip.
+//
+// Rows live in RPW + 1 register slots: a sweep down the rows writes row r where
+// row r - 1 was, the next sweep, up the rows, writes it back, so no sweep copies
+// registers.  Tiles never start outside the grid: the ring is a region's own
+// first or last row or column there, and needs no halo.  A ring neighbour is the
+// stored ring in a launch's first sweep, and the ring of the sweep before, the
+// sign-adjusted value of the cell itself, after that.
+constexpr int kTileMaxSweeps = 8, kTileCols = 64;
+
+struct TileJob {
+    const float *src, *b;
+    float* dst;
+    int R, P, m;
+    bool zero;  // the iterate starts as zero (src is not read)
+    float a;
+    Divisor dv;
+    Ring rg;
+    int gi0, gj0;            // grid cell of the region's first cell
+    int ilo, ihi, jlo, jhi;  // cells written
+};
+
+// Tiles of regions `extent` cells long that cover R cells, m of each end of a
+// region lost to the sweeps except where the grid ends.
+__host__ __device__ inline int tile_count(int R, int extent, int m) {
+    return R <= extent ? 1 : (R - 2 * m + extent - 2 * m - 1) / (extent - 2 * m);
+}
+// The region and output range of tile (ty, tx) of tiles_y x tiles_x (tile_count)
+// with H x kTileCols regions; the last tile is moved back to end with the grid.
+__device__ __forceinline__ void tile_place(TileJob& t, int H, int ty, int tx, int tiles_y, int tiles_x) {
+    const int sy = H - 2 * t.m, sx = kTileCols - 2 * t.m;
+    t.gi0 = t.R <= H ? 0 : min(ty * sy, t.R - H);
+    t.gj0 = t.R <= kTileCols ? 0 : min(tx * sx, t.R - kTileCols);
+    t.ilo = ty == 0 ? 1 : ty * sy + t.m;
+    t.ihi = ty == tiles_y - 1 ? t.R - 2 : ty * sy + H - 1 - t.m;
+    t.jlo = tx == 0 ? 1 : tx * sx + t.m;
+    t.jhi = tx == tiles_x - 1 ? t.R - 2 : tx * sx + kTileCols - 1 - t.m;
+}
+
+enum TileKind : int { TILE_DIFFUSE = 0, TILE_PRESSURE = 1, TILE_DIFFUSE_CHECKED = 2 };
+
+// The update of one cell.  A checked divisor's quotient is taken at once; where
+// some lane's dividend lies below its range, the IEEE division replaces it.
+// Zeros lie below it too, but their quotient is exact.
+template <int KIND>
+__device__ __forceinline__ float relax_tile(float b, float n, float s, float w, float e, float a, const Divisor& dv) {
+    if constexpr (KIND == TILE_PRESSURE) return ((((b + e) + w) + s) + n) / 4.0f;
+    const float x = b + a * (((n + s) + w) + e);
+    if constexpr (KIND == TILE_DIFFUSE) return div_rn(x, dv);
+    float q = __builtin_fmaf(x, dv.y2, x * dv.y2_lo);
+    const bool low = !(fabsf(x) >= dv.lo);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(low) != 0, 0)) {
+        const bool bad = low && x != 0.f;
+        if (__builtin_amdgcn_ballot_w64(bad) != 0) q = bad ? x / dv.d : q;
+    }
+    return q;
+}
+
+// ROWS / COLS: the region holds ring rows / columns.  ex: 4 NW kTileCols floats of LDS.
+template <int RPW, int NW, int KIND, bool ROWS, bool COLS>
+__device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict__ ex) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int R = t.R, P = t.P, n = R - 2, i0 = t.gi0 + wave * RPW, gj = t.gj0 + lane;
+    const int cj = min(gj, R - 1);  // a grid narrower than the region
+    float X[RPW + 1], B[RPW];
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) X[r + 1] = t.zero ? 0.f : t.src[(size_t)min(i0 + r, R - 1) * P + cj];
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) B[r] = t.b[(size_t)min(i0 + r, R - 1) * P + cj];
+
+    const float a = t.a;
+    const Divisor dv = t.dv;
+    const Ring rg = t.rg;
+    // row r of sweep s, from its own value c and its neighbours above and below
+    auto row = [&](int s, int r, float c, float north, float south) {
+        float west = lane_west(c), east = lane_east(c);
+        if (ROWS && s > 0) {
+            const int gi = i0 + r;  // the same in all lanes
+            const float m = sgn(rg.neg_tb, c);
+            north = gi == 1 ? m : north;
+            south = gi == n ? m : south;
+        }
+        if (COLS && s > 0) {
+            const float m = sgn(rg.neg_lr, c);
+            west = gj == 1 ? m : west;
+            east = gj == n ? m : east;
+        }
+        return relax_tile<KIND>(B[r], north, south, west, east, a, dv);
+    };
+    auto exchange = [&](int s, float first, float last, float& above, float& below) {
+        float* const e = ex + (s & 1) * NW * 2 * kTileCols + lane;
+        e[(2 * wave) * kTileCols] = first;
+        e[(2 * wave + 1) * kTileCols] = last;
+        __syncthreads();
+        above = e[(2 * max(wave - 1, 0) + 1) * kTileCols];
+        below = e[(2 * min(wave + 1, NW - 1)) * kTileCols];
+    };
+    // rows in slots 1 .. RPW -> slots 0 .. RPW - 1, and back
+    auto down = [&](int s) {
+        float above, below;
+        exchange(s, X[1], X[RPW], above, below);
+#pragma unroll
+        for (int r = 0; r < RPW; ++r)
+            X[r] = row(s, r, X[r + 1], r > 0 ? X[r] : above, r + 1 < RPW ? X[r + 2 <= RPW ? r + 2 : RPW] : below);
+    };
+    auto up = [&](int s) {
+        float above, below;
+        exchange(s, X[0], X[RPW - 1], above, below);
+#pragma unroll
+        for (int r = RPW - 1; r >= 0; --r)
+            X[r + 1] = row(s, r, X[r], r > 0 ? X[r > 0 ? r - 1 : 0] : above, r + 1 < RPW ? X[r + 1] : below);
+    };
+    int s = 0;
+    for (; s + 1 < t.m; s += 2) {
+        down(s);
+        up(s + 1);
+    }
+    if (s < t.m) {
+        down(s);
+#pragma unroll
+        for (int r = RPW - 1; r >= 0; --r) X[r + 1] = X[r];
+    }
+
+    if (gj < t.jlo || gj > t.jhi) return;
+    float* __restrict__ dst = t.dst;
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) {
+        const int gi = i0 + r;
+        if (gi < t.ilo || gi > t.ihi) continue;  // the same in all lanes
+        const float v = X[r + 1];
+        const size_t g = (size_t)gi * P + gj;
+        dst[g] = v;
+        if (!ROWS && !COLS) continue;
+        // the ring beside the cell
+        const float tb = sgn(rg.neg_tb, v), lr = sgn(rg.neg_lr, v);
+        const float cn = 0.5f * (tb + lr);
+        if (gi == 1) dst[g - P] = tb;
+        if (gi == n) dst[g + P] = tb;
+        if (gj == 1) dst[g - 1] = lr;
+        if (gj == n) dst[g + 1] = lr;
+        if (gi == 1 && gj == 1) dst[g - P - 1] = cn;
+        if (gi == 1 && gj == n) dst[g - P + 1] = cn;
+        if (gi == n && gj == 1) dst[g + P - 1] = cn;
+        if (gi == n && gj == n) dst[g + P + 1] = cn;
+    }
+}
+
+template <int RPW, int NW, int KIND>
+__device__ __forceinline__ void jacobi_tile_any(const TileJob& t, float* __restrict__ ex) {
+    const bool rows = t.gi0 == 0 || t.gi0 + NW * RPW >= t.R, cols = t.gj0 == 0 || t.gj0 + kTileCols >= t.R;
+    if (rows) {
+        if (cols) jacobi_tile<RPW, NW, KIND, true, true>(t, ex);
+        else jacobi_tile<RPW, NW, KIND, true, false>(t, ex);
+    } else {
+        if (cols) jacobi_tile<RPW, NW, KIND, false, true>(t, ex);
+        else jacobi_tile<RPW, NW, KIND, false, false>(t, ex);
+    }
+}
+
 // Blocks are dealt round-robin to the 8 XCDs; the first 8 * floor(nb / 8)
 // are renumbered so that each XCD walks a contiguous run of tiles (rows of
 // tiles in order), whose shared halo rows and columns then meet in its L2.

@@ -121,7 +121,10 @@ extern "C" int fs2d_hip_project_noalloc(int rows, const fs2d_params* params, flo
         if (gs) {
             if ((rc = hip(launch_gs_solve_implicit(s, R, K, tw, gsb, lag, A), "Gauss-Seidel sweeps"))) return rc;
         } else {
-            if ((rc = hip(launch_jacobi_solve(s, A, t, depth, jk), "Jacobi sweeps"))) return rc;
+            SweepSet set{};
+            set.a[0] = A;
+            set.count = 1;
+            if ((rc = hip(launch_jacobi_solve(s, set, &t, depth, jk), "Jacobi sweeps"))) return rc;
             if (jacobi_launches(K, depth) & 1) pf = t;
         }
     }

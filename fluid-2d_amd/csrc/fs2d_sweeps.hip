@@ -37,8 +37,6 @@
 
 #include <algorithm>
 #include <cstring>
-#include <mutex>
-#include <unordered_map>
 #include <vector>
 
 namespace fs2d {
@@ -828,57 +826,6 @@ __global__ __launch_bounds__(JT) void k_jacobi_block(SweepArgs A, const float* _
     }
 }
 
-template <int M, int TY, int KIND>
-__global__ __launch_bounds__(64 * JW_WAVES) void k_jacobi_wave(SweepArgs A, const float* __restrict__ src,
-                                                              float* __restrict__ dst, int zero_src, int tiles_x,
-                                                              int tiles) {
-    const int t = xcd_block(blockIdx.x, gridDim.x) * JW_WAVES + threadIdx.x / 64;
-    if (t >= tiles) return;  // whole wave
-    const int ty = t / tiles_x, tx = t - ty * tiles_x;
-    constexpr int OX = 64 - 2 * M;
-    const int gi0 = 1 + TY * ty - M, gj0 = 1 + OX * tx - M;
-    const int R = A.R;
-    const bool plain = gi0 >= 1 && gi0 + TY + 2 * M - 1 <= R - 2 && gj0 >= 1 && gj0 + 63 <= R - 2;
-    const int lane = threadIdx.x & 63;
-    if (plain)
-        jacobi_strip<M, TY, KIND, false>(A, src, dst, zero_src != 0, gi0, gj0, lane);
-    else
-        jacobi_strip<M, TY, KIND, true>(A, src, dst, zero_src != 0, gi0, gj0, lane);
-}
-
-constexpr int JW_TY = 32;  // rows per tile
-
-template <int M>
-hipError_t launch_jw(hipStream_t s, const SweepArgs& a, const float* src, float* dst, int zero_src) {
-    constexpr int OX = 64 - 2 * M;
-    const int n = a.R - 2;
-    const int tiles_x = (n + OX - 1) / OX, tiles_y = (n + JW_TY - 1) / JW_TY;
-    const int tiles = tiles_x * tiles_y;
-    const dim3 grid((tiles + JW_WAVES - 1) / JW_WAVES);
-    if (a.kind == SWEEP_DIFFUSE)
-        hipLaunchKernelGGL((k_jacobi_wave<M, JW_TY, SWEEP_DIFFUSE>), grid, dim3(64 * JW_WAVES), 0, s, a, src, dst,
-                           zero_src, tiles_x, tiles);
-    else
-        hipLaunchKernelGGL((k_jacobi_wave<M, JW_TY, SWEEP_PRESSURE>), grid, dim3(64 * JW_WAVES), 0, s, a, src, dst,
-                           zero_src, tiles_x, tiles);
-    return hipGetLastError();
-}
-
-hipError_t launch_jacobi_wave(hipStream_t s, const SweepArgs& a, const float* src, float* dst, int zero_src,
-                              int m) {
-    switch (m) {
-        case 1: return launch_jw<1>(s, a, src, dst, zero_src);
-        case 2: return launch_jw<2>(s, a, src, dst, zero_src);
-        case 3: return launch_jw<3>(s, a, src, dst, zero_src);
-        case 4: return launch_jw<4>(s, a, src, dst, zero_src);
-        case 5: return launch_jw<5>(s, a, src, dst, zero_src);
-        case 6: return launch_jw<6>(s, a, src, dst, zero_src);
-        case 7: return launch_jw<7>(s, a, src, dst, zero_src);
-        case 8: return launch_jw<8>(s, a, src, dst, zero_src);
-        default: return hipErrorInvalidValue;
-    }
-}
-
 template <int M>
 hipError_t launch_jb(hipStream_t s, const SweepArgs& a, const float* src, float* dst, int zero_src) {
     const dim3 grid((a.R - 2 + JX - 1) / JX, (a.R - 2 + JY - 1) / JY);
@@ -1048,33 +995,42 @@ void gs_plan_destroy(GsPlan* plan) {
 
 // ---- the two-product quotient check ----------------------------------------
 namespace {
-// The significands m of [1, 2) for which x = 2^E m gives
-// RN(x y + RN(x y_lo)) != RN(x / d) (every operation a float one).  Two
-// copies of one loop: with the FMA instruction, and through the C library.
-__attribute__((target("fma"))) long two_product_misses_hw(float d, float y, float yl, int E) {
-    const float scale = std::ldexp(1.0f, E);
-    long misses = 0;
-    for (uint32_t m = 0; m < (1u << 23); ++m) {
-        const uint32_t bits = 0x3f800000u | m;
-        float x;
-        std::memcpy(&x, &bits, 4);
-        x *= scale;
-        if (__builtin_fmaf(x, y, x * yl) != x / d) ++misses;
+// Whether RN(x y + RN(x y_lo)) == RN(x / d) for every x of the binade
+// [2^E, 2^(E + 1)) (every operation a float one).  The value rounded last lies
+// within 2^-46 of x / d (the pair within 2^-47 of 1 / d, the product's rounding as
+// much again), so only an x whose quotient is that close to a midpoint of two
+// neighbouring floats can miss, and those are found instead of tried for: with X
+// and D the 24-bit significands of x and d, and 2^(s - 24) X / D the quotient in
+// [1, 2) (s = 24 for X >= D, else 25), a midpoint is u / 2^24 with u odd in
+// (2^24, 2^25), and
+//     2^s X - u D = r,   |r| <= 2^-22 X 2^(s - 24) < 8.
+// r has the power of two of D (u is odd, and D's is below 2^s), which fixes u
+// modulo 2^s / that power: at most a few X for each r.  (Trying all 2^23
+// significands took 4 to 18 ms a divisor; this takes a microsecond, so nothing is
+// kept from one call to the next.)
+bool two_product_exact(float d, float y, float yl, int E) {
+    int e = 0;
+    const uint64_t D = static_cast<uint64_t>(std::frexp(d, &e) * 0x1p24f);
+    const int t = __builtin_ctzll(D);
+    const uint64_t Do = D >> t;
+    uint64_t inv = Do;  // Do^-1 modulo 2^64: each step doubles the bits that are right (3 at first)
+    for (int k = 0; k < 5; ++k) inv *= 2 - Do * inv;
+    constexpr int kMost = 16;  // twice the bound
+    for (int r = -kMost; r <= kMost; ++r) {
+        if (r == 0 || __builtin_ctz(static_cast<unsigned>(r < 0 ? -r : r)) != t) continue;
+        const uint64_t ro = static_cast<uint64_t>(static_cast<int64_t>(r) / (int64_t(1) << t));
+        for (int s = 24; s <= 25; ++s) {
+            const uint64_t mod = uint64_t(1) << (s - t), u0 = (0 - ro * inv) & (mod - 1);
+            for (uint64_t u = u0 + ((uint64_t(1) << 24) - u0 + mod - 1) / mod * mod * (u0 < (uint64_t(1) << 24));
+                 u < (uint64_t(1) << 25); u += mod) {
+                const uint64_t X = (u * D + static_cast<uint64_t>(static_cast<int64_t>(r))) >> s;
+                if (X < (uint64_t(1) << 23) || X >= (uint64_t(1) << 24) || (X >= D) != (s == 24)) continue;
+                const float x = std::ldexp(static_cast<float>(X), E - 23);
+                if (std::fma(x, y, x * yl) != x / d) return false;
+            }
+        }
     }
-    return misses;
-}
-
-long two_product_misses_soft(float d, float y, float yl, int E) {
-    const float scale = std::ldexp(1.0f, E);
-    long misses = 0;
-    for (uint32_t m = 0; m < (1u << 23); ++m) {
-        const uint32_t bits = 0x3f800000u | m;
-        float x;
-        std::memcpy(&x, &bits, 4);
-        x *= scale;
-        if (std::fma(x, y, x * yl) != x / d) ++misses;
-    }
-    return misses;
+    return true;
 }
 }  // namespace
 
@@ -1101,31 +1057,23 @@ void two_product_quotient(SweepArgs& A) {
     if (static_cast<double>(tf) < t) tf = std::nextafter(tf, 0x1p127f);
     const float lo = std::max(A.div_lo, tf);
     const int E = std::max(0, std::ilogb(tf) + 1);
-    static std::mutex mu;
-    static std::unordered_map<uint64_t, bool> exact;
-    uint32_t db, lb;
-    std::memcpy(&db, &d, 4);
-    std::memcpy(&lb, &yl, 4);
-    const uint64_t key = (static_cast<uint64_t>(db) << 32) | lb;
-    bool ok;
-    {
-        std::lock_guard<std::mutex> g(mu);
-        auto it = exact.find(key);
-        if (it != exact.end()) {
-            ok = it->second;
-        } else {
-            const long misses = __builtin_cpu_supports("fma") ? two_product_misses_hw(d, y, yl, E)
-                                                              : two_product_misses_soft(d, y, yl, E);
-            ok = misses == 0;
-            exact.emplace(key, ok);
-        }
-    }
-    if (ok) {
+    if (two_product_exact(d, y, yl, E)) {
         A.div_checked = 1;
         A.div_lo = lo;
         A.inv_hi2 = y;
         A.inv_lo2 = yl;
     }
+}
+
+void known_quotient(SweepArgs& A) {
+    two_product_quotient(A);
+    if (A.div_checked || A.kind != SWEEP_DIFFUSE) return;
+    int e = 0;
+    if (!(A.denom >= 1.f && A.denom <= 0x1p100f) || std::frexp(A.denom, &e) != 0.5f) return;
+    A.div_checked = 1;
+    A.div_lo = 0.f;
+    A.inv_hi2 = 1.0f / A.denom;
+    A.inv_lo2 = 0x1p-149f;
 }
 
 // Whether fields [0, count) of a set all take the checked two-product quotient.
@@ -1139,7 +1087,7 @@ static bool all_checked(const SweepSet& set, int count) {
 static SweepSet with_checked_divisions(const SweepSet& set) {
     SweepSet out = set;
     for (int f = 0; f < std::min(out.count, SweepSet::kMax); ++f)
-        if (out.a[f].kind == SWEEP_DIFFUSE) two_product_quotient(out.a[f]);
+        if (out.a[f].kind == SWEEP_DIFFUSE) known_quotient(out.a[f]);
     return out;
 }
 
@@ -1397,27 +1345,37 @@ hipError_t launch_gs_solve(hipStream_t s, const GsPlan& plan, const SweepArgs& a
 // ---- Jacobi ------------------------------------------------------------------
 int jacobi_launches(int K, int block) { return (K + block - 1) / block; }
 
-hipError_t launch_jacobi_pass(hipStream_t s, const SweepArgs& a, const float* src, float* dst, int zero_src, int m,
-                              int kernel) {
-    return kernel == JACOBI_LDS ? launch_jacobi_block(s, a, src, dst, zero_src, m)
-                                : launch_jacobi_wave(s, a, src, dst, zero_src, m);
+hipError_t launch_jacobi_pass(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
+                              int zero_src, int m, int kernel) {
+    if (kernel != JACOBI_LDS) return launch_jacobi_tiles(s, set, src, dst, zero_src, m);
+    for (int f = 0; f < set.count; ++f) {
+        const hipError_t e = launch_jacobi_block(s, set.a[f], src[f], dst[f], zero_src, m);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
-hipError_t launch_jacobi_solve(hipStream_t s, const SweepArgs& a, float* scratch, int block, int kernel) {
+hipError_t launch_jacobi_solve(hipStream_t s, const SweepSet& set, float* const* scratch, int block, int kernel) {
     // Sweep order: x -> scratch -> x -> ...; an odd launch count ends in
     // scratch, and the caller swaps the two buffers.
-    const float* src = a.x;
-    float* dst = scratch;
+    const float* src[SweepSet::kMax];
+    float* dst[SweepSet::kMax];
+    for (int f = 0; f < set.count; ++f) {
+        src[f] = set.a[f].x;
+        dst[f] = scratch[f];
+    }
     int done = 0;
-    bool zero = a.zero_start != 0;
-    while (done < a.K) {
-        const int m = std::min(block, a.K - done);
-        hipError_t e = launch_jacobi_pass(s, a, src, dst, zero ? 1 : 0, m, kernel);
+    bool zero = set.a[0].zero_start != 0;
+    while (done < set.a[0].K) {
+        const int m = std::min(block, set.a[0].K - done);
+        hipError_t e = launch_jacobi_pass(s, set, src, dst, zero ? 1 : 0, m, kernel);
         if (e != hipSuccess) return e;
         zero = false;
         done += m;
-        src = dst;
-        dst = (dst == scratch) ? a.x : scratch;
+        for (int f = 0; f < set.count; ++f) {
+            src[f] = dst[f];
+            dst[f] = (dst[f] == scratch[f]) ? set.a[f].x : scratch[f];
+        }
     }
     return hipSuccess;
 }

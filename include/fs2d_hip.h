@@ -189,15 +189,16 @@ int fs2d_gs_pipeline_offset(int rows, int diffuse_iterations, int pressure_itera
  * infinite dividend comes out infinite too), else 0.  lo = the smallest
  * nonzero |dividend| the FMA-based quotients take (smaller ones, zero and NaN,
  * and for the corrected quotient those above 2^100 and inf, take the IEEE
- * division).  The first call for a divisor tries 2^23 dividends (about 4-18
- * ms); the answer is cached. */
+ * division). */
 int fs2d_division_plan(float denom, float* inv, float* inv_lo, float* two_hi, float* two_lo, float* lo,
                        int* checked);
 /* On-device copy bandwidth: a float4 copy kernel over `bytes` (read + write
  * counted), timed with HIP events over `reps` copies; the achievable HBM
  * figure beside the 8 TB/s peak. */
 int fs2d_hip_copy_bandwidth(long long bytes, int reps, float* gb_per_s);
-/* Number of kernel launches one step enqueues (for per-launch averages). */
+/* Number of kernel launches one step enqueues (for per-launch averages).  In
+ * the Jacobi order a launch that serves density, u and v together counts as
+ * three: the figure is that of one field per launch. */
 int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches);
 
 /* ---- projection without allocation -------------------------------------
