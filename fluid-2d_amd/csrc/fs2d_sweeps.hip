@@ -299,6 +299,11 @@ __global__ __launch_bounds__(64 * M) void k_gs_unit_mixed(SweepSet S, const int2
     }
 }
 
+// The value of the lane before (lane r receives lane r - 1); lane 0 keeps own.
+__device__ __forceinline__ float lane_above(float own, float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(own), __float_as_int(x), 0x138, 0xf, 0xf, false));
+}
+
 // One cell update in the plain units' interval loop: exact (relax_k, the IEEE
 // division where the fast quotient does not cover the dividend) or fast
 // (relax_fast, recording such lanes in bad).
@@ -452,13 +457,12 @@ __device__ __forceinline__ void gs_unit_run(const SweepArgs& A, const int2 wk, f
     const int ofs = M - w;  // X column of skewed column 0 is 1 + (M - 1 - w)
     const float a = A.a;
     const Divisor dv = divisor_of(A);
-    float xprev = 0.f;
     // A unit whose cells all lie in rows and columns 2..n-1 never meets the
     // ring: its sweep needs no clamping (the LDS arrays carry guard space for
     // the reads of inactive lanes, whose results are discarded).  The unit
     // kernel expects a zero-start iterate to be zero-filled by the caller.
-    const bool plain = GS_ROWS * I + 1 - k_hi >= 2 && GS_ROWS * I + GS_ROWS - k_lo <= n - 1 &&
-                       TW * J + 1 - k_hi >= 2 && TW * J + TW - k_lo <= n - 1;
+    const bool rows_edge = GS_ROWS * I + 1 - k_hi <= 1 || GS_ROWS * I + GS_ROWS - k_lo >= n;
+    const bool cols_edge = TW * J + 1 - k_hi <= 1 || TW * J + TW - k_lo >= n;
     // Lagged waves: wave w runs its local step s at tick s + L w, and a barrier
     // opens every interval of L ticks.  An operand of step s from the previous
     // sweep was written by wave w - 1 at its step s - 1, i.e. at tick
@@ -466,217 +470,206 @@ __device__ __forceinline__ void gs_unit_run(const SweepArgs& A, const int2 wk, f
     // a cell this wave reads within the interval; so each wave reads all
     // operands of its L steps right after the barrier and then relaxes them
     // with only the DPP / register chain between steps.
+    //
+    // A level is as long as its slowest unit, and an interval is latency: a
+    // lone wave spends 600 of the 2400 clocks of a microsecond on 4 steps, with
+    // 10 instructions a step at 5 clocks each (8 if dependent), an LDS round
+    // trip, the drain of its stores, a barrier, and 20 clocks a taken branch.  So
+    // a wave goes through its intervals in loops with one branch, by the
+    // edges that wave meets; the lanes of a step are masks in scalar registers;
+    // and the LDS operands lie at constant offsets from a few addresses.  Pressure
+    // solve before and after, us: 130^2 and 20 sweeps 139 and 111, 1026^2 and 40
+    // sweeps 741 and 586, 4098^2 and 80 sweeps 3300 and 2700; diffuse and pressure
+    // together 272 and 217, 1054 and 881, 7420 and 6400.  Slower: reading the
+    // right-hand side or all operands an interval ahead (the LDS serves 8 waves at
+    // once, and waves 2 intervals apart take 18 % more of them), E by a lane shift of S.
     constexpr int STEPS = GS_ROWS + TW - 1;
-    constexpr int NINT = (STEPS + L * (M - 1) + L - 1) / L;
-    // The operand reads of an interval are pinned ahead of its relaxations
-    // (sched_barrier), so they are never sunk into per-tick branches.
-    const int me0 = (1 + r + (M - 1 - w)) * XP + ofs - r;  // X index of this lane's cell at step s: me0 + s
+    constexpr int INTERVALS = (STEPS + L - 1) / L;  // of one wave
+    static_assert(GS_ROWS == 64 && TW % 64 == 0 && 64 % L == 0, "the step phases assume 64-row tiles");
+    const int me0 = (1 + r + (M - 1 - w)) * XP + ofs - r;   // X index of this lane's cell at step s: me0 + s
     const int bme0 = (r + (M - 1 - w)) * BP + ofs - 1 - r;  // Bs index of its right-hand side: bme0 + s
-    if (plain) {
-        // Step phases (lane r relaxes column c = s - r): while s < 64, lane
-        // r's first cell (c = 0, whose west neighbour is the tile halo) is at
-        // step r and lanes r <= s are active; while 64 <= s < TW every lane
-        // is inside the tile (c in [1, TW - 1]); from s = TW on lanes
-        // r >= s - (TW - 1) are active.  Intervals start at multiples of L,
-        // so an interval lies in one phase.  The north halo matters only to
-        // lane 0, which is active while s < TW; it enters as the DPP shift's
-        // old value (lane 0 has no source lane).
-        static_assert(GS_ROWS == 64 && TW % 64 == 0 && 64 % L == 0, "the step phases assume 64-row tiles");
-        // The west neighbour of a lane's first cell (step r) lies in the tile's
-        // west halo column.  Waves w' <= w never write that cell (they would
-        // reach it at a negative tile column); waves w' > w write it at tick
-        // r - 1 + (2 + L) w' - 2 w, after this wave's step r (tick r + L w).
-        // So its value at the unit's start is the one step r reads: read it
-        // once, into xprev, which a lane keeps until its first step (r), so
-        // that step takes it as W like every later step takes the lane's
-        // previous cell.
-        __syncthreads();
-        xprev = X[me0 + r - 1];
-        const int guard_r = XH * XP + r;  // lane r's word in the guard space after X
-        for (int it = 0; it < NINT; ++it) {
+    using Lds = __attribute__((address_space(3))) float*;
+    auto lds = [](float* p) {
+        Lds q = (Lds)p;
+        asm("" : "+v"(q));  // an address of its own, not an offset from the array's
+        return q;
+    };
+    auto idle = [&](int intervals) {
+        for (int t = 0; t < intervals; ++t) __syncthreads();
+    };
+    auto flip = [](float v, unsigned sign) { return __uint_as_float(__float_as_uint(v) ^ sign); };
+    // mask ? a : b, in the encoding that names its mask register: with an
+    // implicit vcc one such select took 30 clocks, not 5, with 8 waves on a
+    // compute unit (solves 5 % longer)
+    auto pick = [](unsigned long long mask, auto a, auto b) {
+        decltype(a) d;
+        asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(d) : "v"(b), "v"(a), "s"(mask));
+        return d;
+    };
+    enum { GROW, FULL, SHRINK, ANY };
+    __syncthreads();
+    const int c_left = 1 - jbase, c_right = n - jbase;  // skewed columns of j = 1 and j = n
+    auto sweep = [&](auto rows_t, auto left_t, auto right_t) {
+        constexpr bool RE = decltype(rows_t)::value, LE = decltype(left_t)::value, TE = decltype(right_t)::value;
+        constexpr bool CE = LE || TE;
+        // A neighbour on the ring is, for sweep k > 0, the sign-adjusted
+        // previous-sweep value of the cell itself (overwritten only by its own
+        // relaxation), and for sweep 0 the stored ring, which the unit loaded.
+        // Write-back stores the ring of every edge cell, so the next unit finds
+        // the ring of the latest sweep there.  The ring enters through operands
+        // that exist already:
+        //  * row n takes its own cell for S (another offset, a sign);
+        //  * the lane above row 1 is idle and has row 1 to its south: it hands
+        //    down that value, with its sign, where a relaxing lane hands down
+        //    its result (row 1 in lane 0 takes its own cell for the tile halo);
+        //  * a cell is its west neighbour's E a step earlier: that value, with
+        //    its sign, is the W of column 1 (taken by the lane, still idle, as
+        //    its previous result) and the E of column n.
+        // Which edges a wave meets is known at compile time (RE: rows 1 or n, LE:
+        // column 1 and its virtual ring, TE: column n); what a case leaves out
+        // cannot occur in its waves.
+        const bool kpos = (k > 0);
+        const unsigned tb_sign = rg.neg_tb ? 0x80000000u : 0u, lr_sign = rg.neg_lr ? 0x80000000u : 0u;
+        const unsigned long long rows_in = __ballot(i >= 1 && i <= n), above = __ballot(kpos && i == 0);
+        const unsigned s_sign = kpos && (i == n || i == 0) ? tb_sign : 0u;
+        const bool n_own = RE && kpos && GS_ROWS * I == k;  // row 1 in lane 0
+        const int c_lo = LE ? min(c_left, TW) : 0, c_hi = TE ? c_right : TW - 1;
+        const unsigned long long e_virtual = __ballot(kpos);
+        Lds pn = lds(X + me0 - (n_own ? 0 : XP)), po = RE ? lds(X + me0) : pn + XP;
+        Lds ps = lds(X + me0 + (RE && kpos && i == n ? 0 : XP)), pb = lds(Bs + bme0);
+        // An idle lane's store goes to words of the guard space after X that no
+        // one uses (lane r: r + q for step q of an interval), so no exec mask
+        // changes.
+        const Lds guard = lds(X + XH * XP + r - (RE ? 0 : XP));
+        // West of the lane's first cell (c_lo, at step c_lo + r): the tile's west
+        // halo column (or the ring, which no sweep writes).  Waves w' <= w never
+        // write that cell (they would reach it at a negative tile column); waves
+        // w' > w write it after this wave's step r.  So its value at the unit's
+        // start is the one that step reads: it is read once, into xprev, which a
+        // lane keeps until its first step, so that step takes it as W like every
+        // later step takes the lane's previous cell.
+        float xprev = X[me0 + c_lo + r - 1];
+        float ring = 0.f;  // the step's own cell with the side rings' sign
+        if constexpr (CE) {
+            // lane 0's cell at step 0: no earlier sweep of this unit writes it
+            ring = flip(X[me0], lr_sign);
+            if (LE && c_lo == 0) xprev = r == 0 ? ring : xprev;
+        }
+        // bit c of cols: column c is in [c_lo, c_hi]; bits move down as columns pass
+        unsigned long long cols[2] = {0, 0};
+        if constexpr (CE)
+            for (int h = 0; h < TW / 64; ++h) {
+                const int lo = min(max(c_lo - 64 * h, 0), 64), hi = min(max(c_hi + 1 - 64 * h, 0), 64);
+                cols[h] = hi > lo ? (~0ull >> (64 - (hi - lo))) << lo : 0ull;
+            }
+        // One interval from the lanes whose column is in range at its first step
+        // (GROW: a lane more a step from below, SHRINK: a lane fewer, FULL: all);
+        // returns those at the next one's.  The steps take the fast quotient; if
+        // a lane's dividend needed the IEEE division, they are redone exactly
+        // from the interval's start (no other wave reads this interval's stores
+        // before the next barrier, so the first pass's stores are simply
+        // overwritten; nh keeps its lane 0 through the shift, where the second
+        // pass finds it).  One branch per interval instead of one per step.
+        auto interval = [&](auto phase_t, unsigned long long lanes) {
+            constexpr int PH = decltype(phase_t)::value;
+            constexpr bool MASKED = RE || PH != FULL;
             __syncthreads();
-            const int s0 = it * L - L * w;
-            // a wave with no step of this interval in [0, STEPS) only joins the barrier
-            if (!wave_ok || s0 + L <= 0 || s0 >= STEPS) continue;
-            const int x0 = me0 + s0, b0 = bme0 + s0;
-            float so[L], e[L], bb[L];
-            // An interval's steps take the fast quotient; if any lane's dividend
-            // needed the IEEE division, they are redone exactly from the
-            // interval's start (no other wave reads this interval's stores
-            // before the next barrier, so the first pass's stores are simply
-            // overwritten).  One branch per interval instead of one per step.
-            unsigned long long bad = 0;
-            auto run_interval = [&](auto steps) {
-                const float xp0 = xprev;
-                steps(std::false_type{});
-                if constexpr (KIND == SWEEP_DIFFUSE) {
-                    if (__builtin_expect(bad != 0, 0)) {
-                        xprev = xp0;
-                        steps(std::true_type{});
+            float so[L], e[L], bb[L], nh[L];
+#pragma unroll
+            for (int q = 0; q < L; ++q) {
+                so[q] = ps[q];
+                e[q] = po[q + 1];
+                bb[q] = pb[q];
+                if (PH != SHRINK) nh[q] = pn[q];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (RE && PH != SHRINK && __builtin_expect(n_own, 0)) {
+#pragma unroll
+                for (int q = 0; q < L; ++q) nh[q] = flip(nh[q], tb_sign);
+            }
+            unsigned long long bad = 0, cin;
+            float own;
+            auto steps = [&](auto exact_t) {
+                cin = lanes;
+                own = ring;
+#pragma unroll
+                for (int q = 0; q < L; ++q) {
+                    unsigned long long next = cin;
+                    if constexpr (PH == GROW) next = cin << 1 | 1;
+                    if constexpr (PH == SHRINK) next = cin << 1;
+                    if constexpr (PH == ANY) next = cin << 1 | (cols[0] >> (q + 1) & 1);
+                    const unsigned long long act = RE ? cin & rows_in : cin;
+                    const float sv = RE ? flip(so[q], s_sign) : so[q];
+                    float ev = e[q];
+                    if constexpr (CE) {
+                        if constexpr (TE) ev = pick(cin & ~next & e_virtual, own, ev);
+                        own = flip(e[q], lr_sign);
                     }
+                    if constexpr (PH == SHRINK)
+                        nh[q] = __int_as_float(
+                            __builtin_amdgcn_mov_dpp(__float_as_int(xprev), 0x138, 0xf, 0xf, false));
+                    else
+                        nh[q] = lane_above(nh[q], xprev);
+                    unsigned long long odd = 0;
+                    const float v = relax_step<KIND, CHECKED>(exact_t, bb[q], nh[q], sv, xprev, ev, a, dv, odd);
+                    bad |= RE || CE ? odd & act : odd;
+                    if constexpr (MASKED) {
+                        const Lds at = pick(act, RE ? po : pn, guard);
+                        at[q + (RE ? 0 : XP)] = v;
+                    } else {
+                        po[q] = v;
+                    }
+                    // (once all lanes have started, what an idle one holds does not matter)
+                    if constexpr (LE) xprev = pick(cin, v, own);
+                    else if constexpr (PH == GROW || PH == ANY) xprev = pick(cin, v, xprev);
+                    else xprev = v;
+                    if constexpr (RE) xprev = pick(above, sv, xprev);
+                    cin = next;
                 }
             };
-            if (s0 < 64) {
-                float nh[L];
-#pragma unroll
-                for (int q = 0; q < L; ++q) {
-                    so[q] = X[x0 + q + XP];
-                    e[q] = X[x0 + q + 1];
-                    bb[q] = Bs[b0 + q];
-                    nh[q] = X[x0 + q - XP];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                auto steps = [&](auto exact_t) {
-#pragma unroll
-                    for (int q = 0; q < L; ++q) {
-                        const int s = s0 + q;
-                        const float nv = __int_as_float(__builtin_amdgcn_update_dpp(
-                            __float_as_int(nh[q]), __float_as_int(xprev), 0x138, 0xf, 0xf, false));
-                        const float v = relax_step<KIND, CHECKED>(exact_t, bb[q], nv, so[q], xprev, e[q], a, dv, bad);
-                        const bool act = (r <= s);
-                        // an idle lane stores to its own guard word (no exec mask change)
-                        X[(act ? x0 : guard_r - q) + q] = v;
-                        xprev = act ? v : xprev;
-                    }
-                };
-                run_interval(steps);
-            } else if (s0 < TW) {
-                float nh[L];
-#pragma unroll
-                for (int q = 0; q < L; ++q) {
-                    so[q] = X[x0 + q + XP];
-                    e[q] = X[x0 + q + 1];
-                    bb[q] = Bs[b0 + q];
-                    nh[q] = X[x0 + q - XP];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                auto steps = [&](auto exact_t) {
-#pragma unroll
-                    for (int q = 0; q < L; ++q) {
-                        const float nv = __int_as_float(__builtin_amdgcn_update_dpp(
-                            __float_as_int(nh[q]), __float_as_int(xprev), 0x138, 0xf, 0xf, false));
-                        const float v = relax_step<KIND, CHECKED>(exact_t, bb[q], nv, so[q], xprev, e[q], a, dv, bad);
-                        X[x0 + q] = v;
-                        xprev = v;
-                    }
-                };
-                run_interval(steps);
-            } else {
-#pragma unroll
-                for (int q = 0; q < L; ++q) {
-                    so[q] = X[x0 + q + XP];
-                    e[q] = X[x0 + q + 1];
-                    bb[q] = Bs[b0 + q];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                auto steps = [&](auto exact_t) {
-#pragma unroll
-                    for (int q = 0; q < L; ++q) {
-                        const int s = s0 + q;
-                        const float nv =
-                            __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(xprev), 0x138, 0xf, 0xf, false));
-                        const float v = relax_step<KIND, CHECKED>(exact_t, bb[q], nv, so[q], xprev, e[q], a, dv, bad);
-                        X[(r >= s - (TW - 1) ? x0 : guard_r - q) + q] = v;
-                        xprev = v;
-                    }
-                };
-                run_interval(steps);
-            }
-        }
-    } else {
-        // Units that meet the ring: a neighbour on the ring is, for sweep
-        // k > 0, the sign-adjusted previous-sweep value of the cell itself
-        // (read with the other operands; the cell is overwritten only after
-        // its own relaxation), and for sweep 0 the stored ring, which the
-        // unit loaded.  Write-back stores the ring of every edge cell, so the
-        // next unit finds the ring of the latest sweep there.  The loop is
-        // specialised by the edges the unit meets (top/bottom rows, left/right
-        // columns); the tests it leaves out cannot hold in such a unit.
-        const bool row_ok = wave_ok && i >= 1 && i <= n;
-        const bool kpos = (k > 0);
-        const bool top = row_ok && i == 1, bot = row_ok && i == n;
-        const int c_left = 1 - jbase, c_right = n - jbase;  // skewed columns of j = 1 and j = n
-        const int c_lo = row_ok ? max(0, c_left) : TW, c_hi = min(TW - 1, c_right);
-        const unsigned tb_sign = rg.neg_tb ? 0x80000000u : 0u, lr_sign = rg.neg_lr ? 0x80000000u : 0u;
-        const bool n_virtual = top && kpos, s_virtual = bot && kpos;
-        // W at the lane's first column: the tile halo, or on the left edge
-        // the ring (virtual for k > 0); wave-uniform
-        const bool w_virtual = kpos && c_left >= 0;
-        const bool rows_edge = GS_ROWS * I + 1 - k_hi <= 1 || GS_ROWS * I + GS_ROWS - k_lo >= n;
-        const bool cols_edge = TW * J + 1 - k_hi <= 1 || TW * J + TW - k_lo >= n;
-        // West of the lane's first cell (c_lo, at step c_lo + r): the tile's west
-        // halo, written only by later waves after that step, or the ring, which
-        // no sweep writes -- read once (as in the plain units).
-        __syncthreads();
-        const float w_first = X[me0 + c_lo + r - 1];
-        const int guard_r = XH * XP + r;  // lane r's word in the guard space after X
-        auto sweeps = [&](auto rows_t, auto cols_t) {
-            constexpr bool RE = decltype(rows_t)::value, CE = decltype(cols_t)::value;
-            for (int it = 0; it < NINT; ++it) {
-                __syncthreads();
-                const int s0 = it * L - L * w;
-                if (!wave_ok || s0 + L <= 0 || s0 >= STEPS) continue;
-                const int x0 = me0 + s0, b0 = bme0 + s0;
-                float so[L], e[L], bb[L], nh[L], self[L];
-#pragma unroll
-                for (int q = 0; q < L; ++q) {
-                    so[q] = X[x0 + q + XP];
-                    e[q] = X[x0 + q + 1];
-                    bb[q] = Bs[b0 + q];
-                    nh[q] = X[x0 + q - XP];
-                    self[q] = X[x0 + q];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                // fast quotient for the interval, redone exactly if needed (as in the plain units)
-                unsigned long long bad = 0;
-                auto steps = [&](auto exact_t) {
-#pragma unroll
-                    for (int q = 0; q < L; ++q) {
-                        const int c = s0 + q - r;
-                        // lane 0 receives the tile halo as the shift's old value
-                        const float up = __int_as_float(__builtin_amdgcn_update_dpp(
-                            __float_as_int(nh[q]), __float_as_int(xprev), 0x138, 0xf, 0xf, false));
-                        float nv = up, sv = so[q], ev = e[q], wv;
-                        if constexpr (RE) {
-                            const float tbv = __uint_as_float(__float_as_uint(self[q]) ^ tb_sign);
-                            nv = n_virtual ? tbv : (top ? nh[q] : up);
-                            sv = s_virtual ? tbv : so[q];
-                        }
-                        if constexpr (CE) {
-                            const float lrv = __uint_as_float(__float_as_uint(self[q]) ^ lr_sign);
-                            wv = (c == c_lo) ? (w_virtual ? lrv : w_first) : xprev;
-                            ev = (kpos && c == c_right) ? lrv : e[q];
-                        } else {
-                            wv = (c == c_lo) ? w_first : xprev;
-                        }
-                        const float v = relax_step<KIND, CHECKED>(exact_t, bb[q], nv, sv, wv, ev, a, dv, bad);
-                        if constexpr (KIND == SWEEP_PRESSURE) {
-                            X[(c >= c_lo && c <= c_hi ? x0 : guard_r - q) + q] = v;
-                        } else {
-                            if (c >= c_lo && c <= c_hi) X[x0 + q] = v;
-                        }
-                        xprev = v;
-                    }
-                };
-                const float xp0 = xprev;
-                steps(std::false_type{});
-                if constexpr (KIND == SWEEP_DIFFUSE) {
-                    if (__builtin_expect(bad != 0, 0)) {
-                        xprev = xp0;
-                        steps(std::true_type{});
-                    }
+            const float xp0 = xprev;
+            steps(std::false_type{});
+            if constexpr (KIND == SWEEP_DIFFUSE) {
+                if (__builtin_expect(bad != 0, 0)) {
+                    xprev = xp0;
+                    steps(std::true_type{});
                 }
             }
+            ring = own;
+            pn += L;
+            ps += L;
+            pb += L;
+            po = RE ? po + L : pn + XP;
+            if constexpr (PH == ANY) cols[0] = cols[0] >> L | (TW > 64 ? cols[1] << (64 - L) : 0);
+            if constexpr (PH == ANY && TW > 64) cols[1] >>= L;
+            return cin;
         };
-        using yes = std::integral_constant<bool, true>;
-        using no = std::integral_constant<bool, false>;
-        if (rows_edge && cols_edge)
-            sweeps(yes{}, yes{});
-        else if (rows_edge)
-            sweeps(yes{}, no{});
-        else
-            sweeps(no{}, yes{});
-    }
+        idle(w);
+        if constexpr (CE) {
+            unsigned long long lanes = cols[0] & 1;
+            for (int t = 0; t < INTERVALS; ++t) lanes = interval(std::integral_constant<int, ANY>{}, lanes);
+        } else {
+            unsigned long long lanes = 1;
+            for (int t = 0; t < 64 / L; ++t) lanes = interval(std::integral_constant<int, GROW>{}, lanes);
+            for (int t = 0; t < TW / L - 64 / L; ++t) interval(std::integral_constant<int, FULL>{}, ~0ull);
+            lanes = ~0ull << 1;
+            for (int t = 0; t < INTERVALS - TW / L; ++t)
+                lanes = interval(std::integral_constant<int, SHRINK>{}, lanes);
+        }
+        idle(M - 1 - w);
+    };
+    // Every wave passes the same INTERVALS + M - 1 barriers: the intervals before
+    // its first step, its own, and those of the waves behind it.
+    using yes = std::true_type;
+    using no = std::false_type;
+    const bool left = k > 0 && c_left >= 0, right = c_right < TW;
+    auto by_cols = [&](auto rows_t) {
+        if (left) right ? sweep(rows_t, yes{}, yes{}) : sweep(rows_t, yes{}, no{});
+        else right ? sweep(rows_t, no{}, yes{}) : sweep(rows_t, no{}, no{});
+    };
+    if (!wave_ok) idle(INTERVALS + M - 1);
+    else if (GS_ROWS * I + 1 - k <= 1 || GS_ROWS * I + GS_ROWS - k >= n) by_cols(yes{});
+    else by_cols(no{});
     __syncthreads();
 
     // ---- write back every cell this unit relaxed (its latest sweep).  A unit
@@ -708,7 +701,7 @@ __device__ __forceinline__ void gs_unit_run(const SweepArgs& A, const int2 wk, f
             }
         }
     }
-    if (!plain) {
+    if (rows_edge || cols_edge) {
         // rows 1 and n, then columns 1 and n, of this unit's region
         for (int e = tid; e < 2 * XW + 2 * XH; e += NT) {
             const bool row = e < 2 * XW;
