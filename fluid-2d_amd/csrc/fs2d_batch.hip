@@ -11,12 +11,12 @@
 //
 // Each stage is one launch over a work list: the single-pass stages over
 // (simulation, 64 x 4 cell block) entries, the Jacobi sweeps over
-// (simulation, field, tile) entries with the register-strip tile of the
-// one-grid solver.  Simulation s runs its K_s sweeps as K_s / M launches of M
-// fused sweeps; launch j covers the simulations with more than j launches
-// (the work list is ordered by launch count, so that is a prefix of it), and
-// ping-pongs home -> S1 -> S2 -> S1 ... -> home, so that every solve ends in
-// its home field whatever its launch count (K_s / M >= 2).
+// (simulation, field, tile) entries with the block tile of the one-grid solver.
+// Simulation s runs its K_s sweeps in L_s launches of at most 8 fused sweeps,
+// as evenly as they go; launch j covers the simulations with more than j
+// launches (the work list is ordered by launch count, so that is a prefix of
+// it), and ping-pongs home -> S1 -> S2 -> S1 ... -> home, so that every solve
+// ends in its home field whatever its launch count (L_s >= 2).
 //
 // The step follows fluid_solver_cpu::solve (src/fluid_solver_cpu.cpp:6-31)
 // in the Jacobi order, exactly as fs2d_handle's step does: each simulation's
@@ -57,11 +57,13 @@ struct Roles {
 struct BatchSim {
     size_t off;  // floats, 256-byte aligned
     int R, P;
-    int launches;     // K / M Jacobi launches per solve (diffuse and pressure)
-    int cell_blocks;  // 64 x 4 blocks over the interior
+    int launches;     // Jacobi launches per solve (diffuse and pressure)
+    int sweeps;       // fewest sweeps of a launch; the first `longer` launches have one more
+    int longer;
     float dt, dt0, h, neg_half_h;
-    float a_rho, denom_rho, inv_rho, lo_rho, inv_lo_rho;
-    float a_vel, denom_vel, inv_vel, lo_vel, inv_lo_vel;
+    float a_rho, a_vel;
+    jac::Divisor dv_rho, dv_vel;
+    int checked_rho, checked_vel;  // the divisor has a known quotient (known_quotient)
 };
 
 constexpr int CBX = 64, CBY = 4;      // single-pass stage blocks
@@ -178,76 +180,74 @@ __global__ __launch_bounds__(CBX* CBY) void kb_gradient(const BatchSim* __restri
     }
 }
 
-// Jacobi launch j of M fused sweeps over (simulation, field, tile) entries:
-// x = simulation | field << 24, y = tile (row-major over tiles_y x tiles_x).
-// Persistent: wave g of the grid walks entries g, g + waves, ... (waves = all
-// of the grid's), each entry one tile of one simulation's field; no
-// block-wide barrier, so a wave leaves when its entries are done.
-template <int M, int TY, int KIND>
-__device__ __forceinline__ void kb_jacobi_entry(const BatchSim* __restrict__ sims, const int2 w, Roles r, int j);
+// Jacobi launch j over (simulation, field, tile) entries: x = simulation |
+// field << 24, y = tile (row-major over tiles_y x tiles_x).  Persistent: block g
+// of G takes entries g, g + G, ... (through xcd_block), each one block tile
+// (fs2d_jacobi.hpp) of RPW JB_WAVES rows x 64 columns.
+//
+// What bounds it: VALU issue (a tile's halo of 8 rows and columns is 0.8 of a grid's
+// cells at side 512, more on smaller ones) and memory, both at about half of a
+// launch's time.  256 simulations of sides 64 to 512 (19.3 M cells, 20 or 40 sweeps),
+// one step's diffuse solves / one pressure solve: one wave per 16-row tile, 4 sweeps
+// a launch 1.50 / 0.45 ms; block tiles of 48 rows, at most 8 sweeps a launch 1.41 /
+// 0.40 ms; of 96 rows 1.21 / 0.38 ms.
+constexpr int JB_WAVES = 8;
 
-template <int M, int TY, int KIND>
-__global__ __launch_bounds__(64 * jac::JW_WAVES) void kb_jacobi(const BatchSim* __restrict__ sims,
-                                                               const int2* __restrict__ work, int n_work, Roles r,
-                                                               int j) {
-    const int waves = (int)gridDim.x * jac::JW_WAVES;
-    for (int t = xcd_block(blockIdx.x, gridDim.x) * jac::JW_WAVES + threadIdx.x / 64; t < n_work; t += waves)
-        kb_jacobi_entry<M, TY, KIND>(sims, work[t], r, j);
-}
-
-template <int M, int TY, int KIND>
-__device__ __forceinline__ void kb_jacobi_entry(const BatchSim* __restrict__ sims, const int2 w, Roles r, int j) {
-    const int s = w.x & 0xffffff, f = w.x >> 24;
-    const BatchSim& S = sims[s];
-    constexpr int OX = 64 - 2 * M;
-    const int n = S.R - 2;
-    const int tiles_x = (n + OX - 1) / OX;
-    const int ty = w.y / tiles_x, tx = w.y - ty * tiles_x;
-    const size_t o = S.off;
-    SweepArgs A{};
-    A.R = S.R;
-    A.P = S.P;
-    A.kind = KIND;
-    float *home, *s1, *s2;
-    if (KIND == SWEEP_PRESSURE) {
-        home = r.a[A_P] + o;
-        A.b = r.a[A_D] + o;
-        s1 = r.a[A_S1A] + o;
-        s2 = r.a[A_S2A] + o;
-        A.ring = ring_of(BND_CONT);
-    } else {
-        const bool rho = f == 0;
-        home = r.a[f == 0 ? A_RHO : (f == 1 ? A_UN : A_VN)] + o;
-        A.b = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
-        s1 = r.a[f == 0 ? A_S1A : (f == 1 ? A_S1B : A_S1C)] + o;
-        s2 = r.a[f == 0 ? A_S2A : (f == 1 ? A_S2B : A_S2C)] + o;
-        A.a = rho ? S.a_rho : S.a_vel;
-        A.denom = rho ? S.denom_rho : S.denom_vel;
-        A.inv_denom = rho ? S.inv_rho : S.inv_vel;
-        A.inv_denom_lo = rho ? S.inv_lo_rho : S.inv_lo_vel;
-        A.div_lo = rho ? S.lo_rho : S.lo_vel;
-        A.ring = ring_of(f == 0 ? BND_CONT : (f == 1 ? BND_OPP_H : BND_OPP_V));
+template <int RPW, int KIND>
+__global__ __launch_bounds__(64 * JB_WAVES) void kb_jacobi(const BatchSim* __restrict__ sims,
+                                                           const int2* __restrict__ work, int n_work, Roles r,
+                                                           int j) {
+    __shared__ float ex[4 * JB_WAVES * jac::kTileCols];
+    for (int e = xcd_block(blockIdx.x, gridDim.x); e < n_work; e += gridDim.x) {
+        const int2 w = work[e];
+        const int s = w.x & 0xffffff, f = w.x >> 24;
+        const BatchSim& S = sims[s];
+        const size_t o = S.off;
+        jac::TileJob t;
+        t.R = S.R;
+        t.P = S.P;
+        bool checked = false;
+        float *home, *s1, *s2;
+        if (KIND == SWEEP_PRESSURE) {
+            home = r.a[A_P] + o;
+            t.b = r.a[A_D] + o;
+            s1 = r.a[A_S1A] + o;
+            s2 = r.a[A_S2A] + o;
+            t.rg = ring_of(BND_CONT);
+            t.a = 0.f;
+            t.dv = jac::Divisor{};
+        } else {
+            home = r.a[f == 0 ? A_RHO : (f == 1 ? A_UN : A_VN)] + o;
+            t.b = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
+            s1 = r.a[f == 0 ? A_S1A : (f == 1 ? A_S1B : A_S1C)] + o;
+            s2 = r.a[f == 0 ? A_S2A : (f == 1 ? A_S2B : A_S2C)] + o;
+            t.rg = ring_of(f == 0 ? BND_CONT : (f == 1 ? BND_OPP_H : BND_OPP_V));
+            t.a = f == 0 ? S.a_rho : S.a_vel;
+            t.dv = f == 0 ? S.dv_rho : S.dv_vel;
+            checked = (f == 0 ? S.checked_rho : S.checked_vel) != 0;
+        }
+        t.src = (j == 0) ? home : (((j - 1) & 1) ? s2 : s1);
+        t.dst = (j == S.launches - 1) ? home : ((j & 1) ? s2 : s1);
+        t.zero = KIND == SWEEP_PRESSURE && j == 0;
+        // tiles are placed for the longest launch
+        t.m = S.sweeps + (S.longer > 0);
+        const int tiles_y = jac::tile_count(t.R, RPW * JB_WAVES, t.m), tiles_x = jac::tile_count(t.R, jac::kTileCols, t.m);
+        const int ty = w.y / tiles_x;
+        jac::tile_place(t, RPW * JB_WAVES, ty, w.y - ty * tiles_x, tiles_y, tiles_x);
+        t.m = S.sweeps + (j < S.longer);
+        if constexpr (KIND == SWEEP_PRESSURE)
+            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_PRESSURE>(t, ex);
+        else if (checked)
+            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_DIFFUSE_CHECKED>(t, ex);
+        else
+            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_DIFFUSE>(t, ex);
+        __syncthreads();  // the next tile's first exchange may take the buffer of this one's last
     }
-    const float* src = (j == 0) ? home : (((j - 1) & 1) ? s2 : s1);
-    float* dst = (j == S.launches - 1) ? home : ((j & 1) ? s2 : s1);
-    const bool zero_src = KIND == SWEEP_PRESSURE && j == 0;
-    const int gi0 = 1 + TY * ty - M, gj0 = 1 + OX * tx - M;
-    const int R = S.R;
-    const bool plain = gi0 >= 1 && gi0 + TY + 2 * M - 1 <= R - 2 && gj0 >= 1 && gj0 + 63 <= R - 2;
-    const int lane = threadIdx.x & 63;
-    if (plain)
-        jac::jacobi_strip<M, TY, KIND, false>(A, src, dst, zero_src, gi0, gj0, lane);
-    else
-        jac::jacobi_strip<M, TY, KIND, true>(A, src, dst, zero_src, gi0, gj0, lane);
 }
 
 __global__ __launch_bounds__(256) void kb_fill(uint32_t* __restrict__ p, size_t n) {
     for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (size_t)gridDim.x * 256) p[t] = 0u;
 }
-
-// Candidate (depth, tile rows) pairs; the tuner keeps the fastest.
-constexpr int kDepths[] = {1, 2, 4, 8};
-constexpr int kTileRows[] = {16, 32};
 
 // Blocks of a persistent launch over `n` entries of `per_block` each, at most
 // `limit` (a multiple of 8 when it binds, so that every block's entries fall
@@ -258,46 +258,34 @@ unsigned persistent_grid(int n, int per_block, int limit) {
     return static_cast<unsigned>(std::max(8, limit - limit % 8));
 }
 
-template <int M, int TY>
-void launch_kb_jacobi_mt(hipStream_t st, int kind, const BatchSim* sims, const int2* w, int n, Roles r, int j,
-                         int limit) {
-    const dim3 grid(persistent_grid(n, jac::JW_WAVES, limit));
-    if (kind == SWEEP_DIFFUSE)
-        hipLaunchKernelGGL((kb_jacobi<M, TY, SWEEP_DIFFUSE>), grid, dim3(64 * jac::JW_WAVES), 0, st, sims, w, n, r, j);
-    else
-        hipLaunchKernelGGL((kb_jacobi<M, TY, SWEEP_PRESSURE>), grid, dim3(64 * jac::JW_WAVES), 0, st, sims, w, n, r,
-                           j);
+template <int RPW>
+void launch_kb_jacobi_rows(hipStream_t st, int kind, const BatchSim* sims, const int2* w, int n, Roles r, int j,
+                           int limit) {
+    const dim3 grid(persistent_grid(n, 1, limit)), block(64 * JB_WAVES);
+    if (kind == SWEEP_DIFFUSE) hipLaunchKernelGGL((kb_jacobi<RPW, SWEEP_DIFFUSE>), grid, block, 0, st, sims, w, n, r, j);
+    else hipLaunchKernelGGL((kb_jacobi<RPW, SWEEP_PRESSURE>), grid, block, 0, st, sims, w, n, r, j);
 }
 
-template <int TY>
-bool launch_kb_jacobi_t(hipStream_t st, int M, int kind, const BatchSim* sims, const int2* w, int n, Roles r, int j,
-                        int limit) {
-    switch (M) {
-        case 1: launch_kb_jacobi_mt<1, TY>(st, kind, sims, w, n, r, j, limit); return true;
-        case 2: launch_kb_jacobi_mt<2, TY>(st, kind, sims, w, n, r, j, limit); return true;
-        case 4: launch_kb_jacobi_mt<4, TY>(st, kind, sims, w, n, r, j, limit); return true;
-        case 8: launch_kb_jacobi_mt<8, TY>(st, kind, sims, w, n, r, j, limit); return true;
-        default: return false;
-    }
-}
-
-hipError_t launch_kb_jacobi(hipStream_t st, int M, int TY, int kind, const BatchSim* sims, const int2* w, int n,
-                            Roles r, int j, int limit) {
+hipError_t launch_kb_jacobi(hipStream_t st, int rows, int kind, const BatchSim* sims, const int2* w, int n, Roles r,
+                            int j, int limit) {
     if (n <= 0) return hipSuccess;
-    const bool ok = TY == 16 ? launch_kb_jacobi_t<16>(st, M, kind, sims, w, n, r, j, limit)
-                             : (TY == 32 ? launch_kb_jacobi_t<32>(st, M, kind, sims, w, n, r, j, limit) : false);
-    return ok ? hipGetLastError() : hipErrorInvalidValue;
+    switch (rows) {
+        case 32: launch_kb_jacobi_rows<4>(st, kind, sims, w, n, r, j, limit); break;
+        case 48: launch_kb_jacobi_rows<6>(st, kind, sims, w, n, r, j, limit); break;
+        case 96: launch_kb_jacobi_rows<12>(st, kind, sims, w, n, r, j, limit); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 }  // namespace
 
-// A Jacobi configuration: depth M, tile rows TY, and the work lists of the
-// diffuse (3 fields) and pressure (1 field) solves with, for each launch j,
-// the number of leading entries whose simulation runs launch j.
-struct JacobiConfig {
-    int M = 0, TY = 0;
-    int2* diffuse_work = nullptr;
-    int2* pressure_work = nullptr;
+// The work lists of the diffuse (3 fields) and pressure (1 field) solves with,
+// for each launch j, the number of leading entries whose simulation runs launch j.
+struct JacobiWork {
+    int rows = 0;  // of a tile's region
+    int2* diffuse = nullptr;
+    int2* pressure = nullptr;
     std::vector<int> diffuse_count, pressure_count;  // per launch j
 };
 
@@ -313,7 +301,7 @@ struct fs2d_batch {
     int count = 0;
     fs2d_params prm{};
     std::vector<fs2d_batch_sim> spec;
-    std::vector<BatchSim> host_sims;  // launches filled in for the chosen depth
+    std::vector<BatchSim> host_sims;
     std::vector<int> order;           // simulations by Jacobi launch count, descending
     size_t arena_floats = 0;
     long long interior = 0;
@@ -332,11 +320,9 @@ struct fs2d_batch {
     int* scatter_flag = nullptr;         // its sorted-path gate
     BatchScatter scatter{};
     int cus = 256;                // compute units of the device
-    int jac_per_cu = 0;           // persistent Jacobi blocks per CU (0 until tuned: one block per 4 entries)
-    int cell_per_cu = 0;          // persistent single-pass blocks per CU (0 until tuned: one per entry)
-    bool occupancy_fixed = false; // set by fs2d_hip_batch_set_occupancy: the tuner keeps them
-    JacobiConfig cfg;
-    bool tuned = false;
+    int jac_per_cu = 0;           // persistent Jacobi blocks per CU (0: one per entry)
+    int cell_per_cu = 8;          // persistent single-pass blocks per CU (0: one per entry)
+    JacobiWork jacobi;
     bool speed_valid = false;
     long long steps_done = 0;
     std::vector<BatchGraph*> graphs;
@@ -363,69 +349,42 @@ float cells_of(int R) { return static_cast<float>(static_cast<size_t>(R) * stati
 int jac_limit(const fs2d_batch* b) { return b->jac_per_cu > 0 ? b->cus * b->jac_per_cu : 0; }
 dim3 cell_grid(const fs2d_batch* b) { return dim3(persistent_grid(b->cell_blocks, 1, b->cell_per_cu > 0 ? b->cus * b->cell_per_cu : 0)); }
 
-void free_config(JacobiConfig& c) {
-    if (c.diffuse_work) (void)hipFree(c.diffuse_work);
-    if (c.pressure_work) (void)hipFree(c.pressure_work);
-    c = JacobiConfig{};
-}
-
-// Work lists of depth M and tile rows TY.  Entries are ordered by the
-// simulation's launch count (descending), so launch j takes a prefix.
-int build_config(fs2d_batch* b, int M, int TY, JacobiConfig* out) {
-    JacobiConfig c;
-    c.M = M;
-    c.TY = TY;
-    const int OX = 64 - 2 * M;
+// Work lists of the Jacobi launches.  Entries are ordered by the simulation's
+// launch count (descending), so launch j takes a prefix.  Rows of a tile's region:
+// as for one grid (fs2d_jacobi.hip), by the cells of a diffuse launch.
+hipError_t build_jacobi_work(fs2d_batch* b) {
+    JacobiWork& c = b->jacobi;
+    c.rows = 3 * b->interior < 500000 ? 32 : (3 * b->interior < 8000000 ? 48 : 96);
     std::vector<int2> dw, pw;
-    std::vector<int> launches(b->count);
-    int max_l = 0;
-    for (int s = 0; s < b->count; ++s) {
-        launches[s] = b->spec[s].iterations / M;
-        max_l = std::max(max_l, launches[s]);
-    }
-    c.diffuse_count.assign(max_l, 0);
-    c.pressure_count.assign(max_l, 0);
     for (int s : b->order) {
-        const int n = b->spec[s].rows - 2;
-        const int tiles = ((n + OX - 1) / OX) * ((n + TY - 1) / TY);
+        const BatchSim& S = b->host_sims[s];
+        const int m = S.sweeps + (S.longer > 0);
+        const int tiles = jac::tile_count(S.R, c.rows, m) * jac::tile_count(S.R, jac::kTileCols, m);
         for (int f = 0; f < 3; ++f)
             for (int t = 0; t < tiles; ++t) dw.push_back(make_int2(s | (f << 24), t));
         for (int t = 0; t < tiles; ++t) pw.push_back(make_int2(s, t));
-        for (int j = 0; j < launches[s]; ++j) {
+        if (c.diffuse_count.empty()) {  // the first has the most launches
+            c.diffuse_count.assign(S.launches, 0);
+            c.pressure_count.assign(S.launches, 0);
+        }
+        for (int j = 0; j < S.launches; ++j) {
             c.diffuse_count[j] += 3 * tiles;
             c.pressure_count[j] += tiles;
         }
     }
-    FS2D_BHIP(b, hipMalloc(&c.diffuse_work, sizeof(int2) * dw.size()));
-    FS2D_BHIP(b, hipMalloc(&c.pressure_work, sizeof(int2) * pw.size()));
-    FS2D_BHIP(b, hipMemcpy(c.diffuse_work, dw.data(), sizeof(int2) * dw.size(), hipMemcpyHostToDevice));
-    FS2D_BHIP(b, hipMemcpy(c.pressure_work, pw.data(), sizeof(int2) * pw.size(), hipMemcpyHostToDevice));
-    *out = c;
-    return FS2D_OK;
-}
-
-// Upload the per-simulation constants with launch counts for depth M.
-int upload_sims(fs2d_batch* b, int M) {
-    for (int s = 0; s < b->count; ++s) b->host_sims[s].launches = b->spec[s].iterations / M;
-    // on the batch's stream: kernels already queued there still read the descriptors
-    FS2D_BHIP(b, hipMemcpyAsync(b->sims, b->host_sims.data(), sizeof(BatchSim) * b->count, hipMemcpyHostToDevice,
-                                b->stream));
-    FS2D_BHIP(b, hipStreamSynchronize(b->stream));
-    return FS2D_OK;
-}
-
-bool depth_fits(const fs2d_batch* b, int M) {
-    for (const auto& s : b->spec)
-        if (s.iterations % M != 0 || s.iterations / M < 2) return false;
-    return true;
+    hipError_t e;
+    if ((e = hipMalloc(&c.diffuse, sizeof(int2) * dw.size())) != hipSuccess) return e;
+    if ((e = hipMalloc(&c.pressure, sizeof(int2) * pw.size())) != hipSuccess) return e;
+    if ((e = hipMemcpy(c.diffuse, dw.data(), sizeof(int2) * dw.size(), hipMemcpyHostToDevice)) != hipSuccess) return e;
+    return hipMemcpy(c.pressure, pw.data(), sizeof(int2) * pw.size(), hipMemcpyHostToDevice);
 }
 
 int solve(fs2d_batch* b, int kind) {
-    const JacobiConfig& c = b->cfg;
+    const JacobiWork& c = b->jacobi;
     const auto& counts = kind == SWEEP_DIFFUSE ? c.diffuse_count : c.pressure_count;
-    const int2* w = kind == SWEEP_DIFFUSE ? c.diffuse_work : c.pressure_work;
+    const int2* w = kind == SWEEP_DIFFUSE ? c.diffuse : c.pressure;
     for (int j = 0; j < static_cast<int>(counts.size()); ++j)
-        FS2D_BHIP(b, launch_kb_jacobi(b->stream, c.M, c.TY, kind, b->sims, w, counts[j], b->roles, j, jac_limit(b)));
+        FS2D_BHIP(b, launch_kb_jacobi(b->stream, c.rows, kind, b->sims, w, counts[j], b->roles, j, jac_limit(b)));
     return FS2D_OK;
 }
 
@@ -441,112 +400,6 @@ int project(fs2d_batch* b) {
                        b->slots);
     hipLaunchKernelGGL(kb_fold_speed, dim3(b->count), dim3(64), 0, b->stream, b->max_bits, b->slots);
     FS2D_BHIP(b, cell_launch_check());
-    return FS2D_OK;
-}
-
-// Time one launch (j = 0, writing only scratch) of each stage solve for a
-// candidate configuration; returns the estimated time of both kinds of
-// solves of one step (3 diffuses counted once, their launches being shared,
-// and 2 pressure solves).
-int time_config(fs2d_batch* b, float* est_ms) {
-    const JacobiConfig& c = b->cfg;
-    float t[2] = {0.f, 0.f};
-    for (int k = 0; k < 2; ++k) {
-        const int kind = k == 0 ? SWEEP_DIFFUSE : SWEEP_PRESSURE;
-        const int2* w = kind == SWEEP_DIFFUSE ? c.diffuse_work : c.pressure_work;
-        const int n0 = kind == SWEEP_DIFFUSE ? c.diffuse_count[0] : c.pressure_count[0];
-        float best = 0.f;
-        for (int rep = 0; rep < 3; ++rep) {
-            FS2D_BHIP(b, hipEventRecord(b->ev0, b->stream));
-            FS2D_BHIP(b, launch_kb_jacobi(b->stream, c.M, c.TY, kind, b->sims, w, n0, b->roles, 0, jac_limit(b)));
-            FS2D_BHIP(b, hipEventRecord(b->ev1, b->stream));
-            FS2D_BHIP(b, hipEventSynchronize(b->ev1));
-            float ms = 0.f;
-            FS2D_BHIP(b, hipEventElapsedTime(&ms, b->ev0, b->ev1));
-            if (rep == 1 || (rep > 1 && ms < best)) best = ms;
-        }
-        // later launches cover fewer entries: scale by the entry counts
-        const auto& counts = kind == SWEEP_DIFFUSE ? c.diffuse_count : c.pressure_count;
-        double total = 0;
-        for (int cnt : counts) total += static_cast<double>(cnt) / n0;
-        t[k] = static_cast<float>(best * total);
-    }
-    *est_ms = t[0] + 2.f * t[1];
-    return FS2D_OK;
-}
-
-// Choose depth and tile rows: the fixed jacobi_block (tile rows tuned), or
-// every depth that divides all iteration counts at least twice.
-int tune(fs2d_batch* b) {
-    std::vector<int> depths;
-    if (b->prm.jacobi_block)
-        depths.push_back(b->prm.jacobi_block);
-    else
-        for (int m : kDepths)
-            if (depth_fits(b, m)) depths.push_back(m);
-    float best = 0.f;
-    JacobiConfig chosen;
-    for (int m : depths)
-        for (int ty : kTileRows) {
-            free_config(b->cfg);
-            int rc = build_config(b, m, ty, &b->cfg);
-            if (rc) return rc;
-            if ((rc = upload_sims(b, m))) return rc;
-            float est = 0.f;
-            if ((rc = time_config(b, &est))) return rc;
-            if (chosen.M == 0 || est < best) {
-                best = est;
-                chosen.M = m;
-                chosen.TY = ty;
-            }
-        }
-    free_config(b->cfg);
-    int rc = build_config(b, chosen.M, chosen.TY, &b->cfg);
-    if (rc) return rc;
-    if ((rc = upload_sims(b, chosen.M))) return rc;
-    if (b->occupancy_fixed) {
-        b->tuned = true;
-        return FS2D_OK;
-    }
-    // waves per CU of the persistent launches: Jacobi blocks (4 waves) per CU
-    // timed on the same launches as above, single-pass blocks (4 waves) per
-    // CU on the divergence (it only writes the divergence arena, which every
-    // projection recomputes first); 0 is one block per work entry
-    float best_j = 0.f;
-    int pick_j = 0;
-    for (int f : {0, 1, 2, 4, 8}) {
-        b->jac_per_cu = f;
-        float est = 0.f;
-        if ((rc = time_config(b, &est))) return rc;
-        if (f == 0 || est < best_j) {
-            best_j = est;
-            pick_j = f;
-        }
-    }
-    b->jac_per_cu = pick_j;
-    float best_c = 0.f;
-    int pick_c = 0;
-    for (int f : {0, 2, 4, 8}) {
-        b->cell_per_cu = f;
-        float t = 0.f;
-        for (int rep = 0; rep < 3; ++rep) {
-            FS2D_BHIP(b, hipEventRecord(b->ev0, b->stream));
-            hipLaunchKernelGGL(kb_divergence, cell_grid(b), dim3(CBX, CBY), 0, b->stream, b->sims, b->cell_work,
-                               b->cell_blocks, b->roles);
-            FS2D_BHIP(b, hipGetLastError());
-            FS2D_BHIP(b, hipEventRecord(b->ev1, b->stream));
-            FS2D_BHIP(b, hipEventSynchronize(b->ev1));
-            float ms = 0.f;
-            FS2D_BHIP(b, hipEventElapsedTime(&ms, b->ev0, b->ev1));
-            if (rep == 1 || (rep > 1 && ms < t)) t = ms;
-        }
-        if (f == 0 || t < best_c) {
-            best_c = t;
-            pick_c = f;
-        }
-    }
-    b->cell_per_cu = pick_c;
-    b->tuned = true;
     return FS2D_OK;
 }
 
@@ -566,7 +419,6 @@ int step(fs2d_batch* b) {
     hipLaunchKernelGGL(kb_add_sources, cell_grid(b), blk, 0, b->stream, b->sims, b->cell_work, b->cell_blocks,
                        b->roles);
     FS2D_BHIP(b, cell_launch_check());
-    if (!b->tuned && (rc = tune(b))) return rc;
     if ((rc = solve(b, SWEEP_DIFFUSE))) return rc;
     FS2D_BHIP(b, launch_batch_scatter(b->stream, b->scatter, b->roles.a[A_T1], b->roles.a[A_RHO], b->roles.a[A_U],
                                       b->roles.a[A_V], b->max_bits));
@@ -593,8 +445,7 @@ void drop_graphs(fs2d_batch* b) {
     b->graphs.clear();
 }
 
-// As fs2d_handle's step graphs: the first step runs eagerly (it tunes), then
-// each pre-step state (arena permutation, speed flag) is captured once and
+// As fs2d_handle's step graphs: the first step runs eagerly, then each pre-step state (arena permutation, speed flag) is captured once and
 // replayed.
 int advance(fs2d_batch* b) {
     if (b->prm.launch_mode == FS2D_LAUNCH_EAGER || b->steps_done == 0) {
@@ -660,7 +511,8 @@ int fs2d_hip_batch_destroy(fs2d_batch* b) {
     if (!b) return FS2D_OK;
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     drop_graphs(b);
-    free_config(b->cfg);
+    if (b->jacobi.diffuse) (void)hipFree(b->jacobi.diffuse);
+    if (b->jacobi.pressure) (void)hipFree(b->jacobi.pressure);
     for (float* p : b->roles.a)
         if (p) (void)hipFree(p);
     if (b->sims) (void)hipFree(b->sims);
@@ -731,20 +583,21 @@ static int fs2d_hip_batch_create_impl(int count, const fs2d_batch_sim* sims, con
         S.h = 1.0f / std::sqrt(cells_of(S.R));
         S.neg_half_h = -0.5f * S.h;
         S.a_rho = q.dt * cells_of(S.R) * q.diffusion_rate;
-        S.denom_rho = 1.f + 4.f * S.a_rho;
         S.a_vel = q.dt * cells_of(S.R) * q.viscosity;
-        S.denom_vel = 1.f + 4.f * S.a_vel;
-        const SweepArgs dr = sweep_args(nullptr, nullptr, S.R, S.P, SWEEP_DIFFUSE, S.a_rho, S.denom_rho, BND_CONT, 2, 0);
-        const SweepArgs dv = sweep_args(nullptr, nullptr, S.R, S.P, SWEEP_DIFFUSE, S.a_vel, S.denom_vel, BND_CONT, 2, 0);
-        S.inv_rho = dr.inv_denom;
-        S.lo_rho = dr.div_lo;
-        S.inv_lo_rho = dr.inv_denom_lo;
-        S.inv_vel = dv.inv_denom;
-        S.lo_vel = dv.div_lo;
-        S.inv_lo_vel = dv.inv_denom_lo;
+        SweepArgs dr = sweep_args(nullptr, nullptr, S.R, S.P, SWEEP_DIFFUSE, S.a_rho, 1.f + 4.f * S.a_rho, BND_CONT, 2, 0);
+        SweepArgs dv = sweep_args(nullptr, nullptr, S.R, S.P, SWEEP_DIFFUSE, S.a_vel, 1.f + 4.f * S.a_vel, BND_CONT, 2, 0);
+        known_quotient(dr);
+        known_quotient(dv);
+        S.dv_rho = jac::divisor_of(dr);
+        S.dv_vel = jac::divisor_of(dv);
+        S.checked_rho = dr.div_checked;
+        S.checked_vel = dv.div_checked;
+        const int most = prm.jacobi_block ? prm.jacobi_block : jac::kTileMaxSweeps;
+        S.launches = std::max(2, (q.iterations + most - 1) / most);
+        S.sweeps = q.iterations / S.launches;
+        S.longer = q.iterations % S.launches;
         const int n = S.R - 2;
         const int gx = (n + CBX - 1) / CBX, gy = (n + CBY - 1) / CBY;
-        S.cell_blocks = gx * gy;
         for (int by = 0; by < gy; ++by)
             for (int bx = 0; bx < gx; ++bx) cw.push_back(make_int2(s, (by << 16) | bx));
         ss[s] = ScatterSim{S.off, S.R, S.P, S.dt0, static_cast<unsigned>(scatter_cells),
@@ -758,7 +611,7 @@ static int fs2d_hip_batch_create_impl(int count, const fs2d_batch_sim* sims, con
         b->order.push_back(s);
     }
     std::stable_sort(b->order.begin(), b->order.end(),
-                     [&](int x, int y) { return sims[x].iterations > sims[y].iterations; });
+                     [&](int x, int y) { return b->host_sims[x].launches > b->host_sims[y].launches; });
     b->arena_floats = off;
     b->cell_blocks = static_cast<int>(cw.size());
     auto bail = [&](hipError_t e, const char* what) {
@@ -791,6 +644,7 @@ static int fs2d_hip_batch_create_impl(int count, const fs2d_batch_sim* sims, con
     if ((e = hipMalloc(&b->slots, sizeof(unsigned) * slot_words)) != hipSuccess) return bail(e, "hipMalloc(slots)");
     hipLaunchKernelGGL(kb_fill, dim3((unsigned)std::min<size_t>((slot_words + 255) / 256, 4096)), dim3(256), 0,
                        b->stream, b->slots, slot_words);
+    if ((e = build_jacobi_work(b)) != hipSuccess) return bail(e, "Jacobi work lists");
     // the density scatter: descriptors, window work list, sorted-path buffers
     if (scatter_cells >= (1ll << 31) || scatter_targets >= (1ll << 32) - 1)
         return bail(hipErrorInvalidValue, "too many cells for the batched density scatter");
@@ -908,13 +762,14 @@ int fs2d_hip_batch_sync(fs2d_batch* b) {
 static int fs2d_hip_batch_info_impl(fs2d_batch* b, int* depth, int* tile_rows, int* launches, int* graphs,
                         long long* interior_cells) {
     if (!b) return bfail(b, FS2D_ERR_ARGUMENT, "fs2d_hip_batch_info: NULL batch");
-    if (depth) *depth = b->cfg.M;
-    if (tile_rows) *tile_rows = b->cfg.TY;
+    if (depth) *depth = b->prm.jacobi_block ? b->prm.jacobi_block : 1;
+    if (tile_rows) *tile_rows = b->jacobi.rows - 2 * jac::kTileMaxSweeps;
     if (launches) {
         // max speed (first step only) aside: add, diffuse launches, the scatter's
         // kernels, 2 x (divergence, pressure launches, gradient, fold), gather
-        const int d = static_cast<int>(b->cfg.diffuse_count.size()), p = static_cast<int>(b->cfg.pressure_count.size());
-        *launches = b->tuned ? 1 + d + batch_scatter_launches(b->scatter.targets) + 2 * (3 + p) + 1 : 0;
+        const int d = static_cast<int>(b->jacobi.diffuse_count.size());
+        const int p = static_cast<int>(b->jacobi.pressure_count.size());
+        *launches = b->steps_done > 0 ? 1 + d + batch_scatter_launches(b->scatter.targets) + 2 * (3 + p) + 1 : 0;
     }
     if (graphs) *graphs = static_cast<int>(b->graphs.size());
     if (interior_cells) *interior_cells = b->interior;
@@ -929,7 +784,6 @@ int fs2d_hip_batch_set_occupancy(fs2d_batch* b, int jacobi_blocks_per_cu, int st
         return bfail(b, FS2D_ERR_STATE, "fs2d_hip_batch_set_occupancy: only before the first step");
     b->jac_per_cu = jacobi_blocks_per_cu;
     b->cell_per_cu = stage_blocks_per_cu;
-    b->occupancy_fixed = true;
     return FS2D_OK;
 }
 

@@ -247,8 +247,8 @@ typedef struct fs2d_batch_sim {
 typedef struct fs2d_batch fs2d_batch;
 
 /* params may be NULL; only sweep_order (must be FS2D_ORDER_JACOBI),
- * jacobi_block (0 = autotuned; otherwise it must divide every simulation's
- * iterations at least twice) and launch_mode are read.  Fields start at zero. */
+ * jacobi_block (0 = launches of at most 8 sweeps; otherwise it must divide every
+ * simulation's iterations at least twice) and launch_mode are read.  Fields start at zero. */
 int fs2d_hip_batch_create(int count, const fs2d_batch_sim* sims, const fs2d_params* params, fs2d_batch** out);
 int fs2d_hip_batch_destroy(fs2d_batch* b);
 /* Host arrays of rows*rows floats for simulation `sim`. */
@@ -261,16 +261,18 @@ int fs2d_hip_batch_step_n(fs2d_batch* b, int n);
 /* Wait for the batch's stream, then copy one simulation out (any pointer may be NULL). */
 int fs2d_hip_batch_download(fs2d_batch* b, int sim, float* density, float* u, float* v);
 int fs2d_hip_batch_sync(fs2d_batch* b);
-/* The configuration in use: Jacobi sweeps per launch, rows per Jacobi tile,
+/* The configuration in use: jacobi_depth, the sweeps every Jacobi launch takes a
+ * multiple of (a fixed jacobi_block, else 1: a simulation's sweeps are spread evenly
+ * over its launches), tile_rows, the rows an inner Jacobi tile writes after 8 sweeps,
  * kernel launches per step, captured step graphs, total interior cells. */
 int fs2d_hip_batch_info(fs2d_batch* b, int* jacobi_depth, int* tile_rows, int* launches_per_step, int* graphs,
                         long long* interior_cells);
-/* The persistent launches' grid, as the autotuner chose it on the first step:
- * blocks (of 4 waves) per compute unit for the Jacobi launches and for the
- * single-pass stages (0: one block per work entry), and the compute units. */
+/* The persistent launches' grid: blocks per compute unit for the Jacobi launches (8
+ * waves each) and for the single-pass stages (4 waves each; 0: one block per work
+ * entry), and the compute units. */
 int fs2d_hip_batch_occupancy(fs2d_batch* b, int* jacobi_blocks_per_cu, int* stage_blocks_per_cu,
                              int* compute_units);
-/* Fix those two figures instead of tuning them (before the first step only;
+/* Fix those two figures (0 and 8 otherwise; before the first step only;
  * 0..64, 0 = one block per work entry).  Results do not depend on them. */
 int fs2d_hip_batch_set_occupancy(fs2d_batch* b, int jacobi_blocks_per_cu, int stage_blocks_per_cu);
 const char* fs2d_hip_batch_last_error(const fs2d_batch* b);
