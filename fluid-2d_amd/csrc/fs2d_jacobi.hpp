@@ -174,8 +174,14 @@ __device__ __forceinline__ float relax_tile(float b, float n, float s, float w, 
     return q;
 }
 
-// ROWS / COLS: the region holds ring rows / columns.  ex: 4 NW kTileCols floats of LDS.
-template <int RPW, int NW, int KIND, bool ROWS, bool COLS>
+// Where a region holds the ring.  A region of a grid no smaller than it has the ring
+// as its own first or last row (ROWS 1) and its first (COLS 1) or last column (COLS 2),
+// so the cells beside the ring are known rows and lanes: two rows of a tile's eighth
+// and one neighbour a row are selected, and the other neighbour stays folded into its
+// addition.  2 / 3: anywhere (a grid smaller than the region, or one with both columns
+// in it), tested by index in every row.
+// ex: 4 NW kTileCols floats of LDS.
+template <int RPW, int NW, int KIND, int ROWS, int COLS>
 __device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict__ ex) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int R = t.R, P = t.P, n = R - 2, i0 = t.gi0 + wave * RPW, gj = t.gj0 + lane;
@@ -189,16 +195,23 @@ __device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict_
     const float a = t.a;
     const Divisor dv = t.dv;
     const Ring rg = t.rg;
+    const bool top = t.gi0 == 0 && wave == 0, bottom = t.gi0 + NW * RPW == R && wave == NW - 1;  // ROWS 1
     // row r of sweep s, from its own value c and its neighbours above and below
     auto row = [&](int s, int r, float c, float north, float south) {
         float west = lane_west(c), east = lane_east(c);
-        if (ROWS && s > 0) {
+        if (ROWS == 1 && s > 0) {
+            if (r == 1) north = top ? sgn(rg.neg_tb, c) : north;
+            if (r == RPW - 2) south = bottom ? sgn(rg.neg_tb, c) : south;
+        }
+        if (COLS == 1 && s > 0) west = lane == 1 ? sgn(rg.neg_lr, c) : west;
+        if (COLS == 2 && s > 0) east = lane == kTileCols - 2 ? sgn(rg.neg_lr, c) : east;
+        if (ROWS == 2 && s > 0) {
             const int gi = i0 + r;  // the same in all lanes
             const float m = sgn(rg.neg_tb, c);
             north = gi == 1 ? m : north;
             south = gi == n ? m : south;
         }
-        if (COLS && s > 0) {
+        if (COLS == 3 && s > 0) {
             const float m = sgn(rg.neg_lr, c);
             west = gj == 1 ? m : west;
             east = gj == n ? m : east;
@@ -265,13 +278,17 @@ __device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict_
 
 template <int RPW, int NW, int KIND>
 __device__ __forceinline__ void jacobi_tile_any(const TileJob& t, float* __restrict__ ex) {
-    const bool rows = t.gi0 == 0 || t.gi0 + NW * RPW >= t.R, cols = t.gj0 == 0 || t.gj0 + kTileCols >= t.R;
-    if (rows) {
-        if (cols) jacobi_tile<RPW, NW, KIND, true, true>(t, ex);
-        else jacobi_tile<RPW, NW, KIND, true, false>(t, ex);
+    const bool left = t.gj0 == 0, right = t.gj0 + kTileCols >= t.R;
+    if (t.R < NW * RPW || (left && right)) {
+        jacobi_tile<RPW, NW, KIND, 2, 3>(t, ex);
+    } else if (t.gi0 == 0 || t.gi0 + NW * RPW == t.R) {
+        if (left) jacobi_tile<RPW, NW, KIND, 1, 1>(t, ex);
+        else if (right) jacobi_tile<RPW, NW, KIND, 1, 2>(t, ex);
+        else jacobi_tile<RPW, NW, KIND, 1, 0>(t, ex);
     } else {
-        if (cols) jacobi_tile<RPW, NW, KIND, false, true>(t, ex);
-        else jacobi_tile<RPW, NW, KIND, false, false>(t, ex);
+        if (left) jacobi_tile<RPW, NW, KIND, 0, 1>(t, ex);
+        else if (right) jacobi_tile<RPW, NW, KIND, 0, 2>(t, ex);
+        else jacobi_tile<RPW, NW, KIND, 0, 0>(t, ex);
     }
 }
 
