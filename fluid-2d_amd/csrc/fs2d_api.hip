@@ -269,8 +269,9 @@ constexpr int kJacobiDefaultDepth = 4;
 // timed (best of two, after a warm-up) reading the live iterates and writing
 // only the scratch fields.  Results are identical for every depth.  A stream
 // under capture cannot be timed; the default depth is used then (not kept).
-// scratch[f]: a field to write in place of field f's iterate.
-int jacobi_depth_for(fs2d_handle* h, const SweepSet& set, float* const* scratch, int* out) {
+// scratch[f]: a field to write in place of field f's iterate.  first: the solve's
+// right-hand sides are not there yet; one such launch forms them.
+int jacobi_depth_for(fs2d_handle* h, const SweepSet& set, float* const* scratch, const JacobiFirst* first, int* out) {
     const SweepArgs& A = set.a[0];
     if (h->prm.jacobi_block) {
         *out = h->prm.jacobi_block;
@@ -289,7 +290,9 @@ int jacobi_depth_for(fs2d_handle* h, const SweepSet& set, float* const* scratch,
         return FS2D_OK;
     }
     const float* src[SweepSet::kMax];
-    for (int f = 0; f < set.count; ++f) src[f] = set.a[f].x;
+    for (int f = 0; f < set.count; ++f) src[f] = first && first->src[f] ? first->src[f] : set.a[f].x;
+    if (first)
+        FS2D_HIP(h, launch_jacobi_pass(h->stream, set, src, scratch, A.zero_start, 1, h->jacobi_kernel, first));
     float best = 0.f;
     int best_m = kJacobiDefaultDepth;
     for (int m : {1, 2, 4, 8}) {
@@ -326,15 +329,16 @@ int jacobi_depth_known(const fs2d_handle* h, int kind, int K) {
 // The set's Jacobi solves, fields[f] and scratch[f] the pointers that hold field
 // f's iterate and a free field: an odd launch count leaves the result in the
 // scratch field, and the two pointers are swapped.
-int jacobi_solve(fs2d_handle* h, SweepSet set, float** const* fields, float** const* scratch) {
+int jacobi_solve(fs2d_handle* h, SweepSet set, float** const* fields, float** const* scratch,
+                 const JacobiFirst* first = nullptr) {
     float* t[SweepSet::kMax];
     for (int f = 0; f < set.count; ++f) {
         t[f] = *scratch[f];
         known_quotient(set.a[f]);
     }
     int depth = kJacobiDefaultDepth, rc;
-    if ((rc = jacobi_depth_for(h, set, t, &depth))) return rc;
-    FS2D_HIP(h, launch_jacobi_solve(h->stream, set, t, depth, h->jacobi_kernel));
+    if ((rc = jacobi_depth_for(h, set, t, first, &depth))) return rc;
+    FS2D_HIP(h, launch_jacobi_solve(h->stream, set, t, depth, h->jacobi_kernel, first));
     if (jacobi_launches(set.a[0].K, depth) & 1)
         for (int f = 0; f < set.count; ++f) std::swap(*fields[f], *scratch[f]);
     return FS2D_OK;
@@ -343,7 +347,7 @@ int jacobi_solve(fs2d_handle* h, SweepSet set, float** const* fields, float** co
 // K relaxation sweeps of x against b; Jacobi may leave the result in the
 // scratch field, in which case the two pointers are swapped.
 int linear_solve(fs2d_handle* h, float*& x, const float* b, int kind, float a, float denom, int mode, int K,
-                 int zero_start) {
+                 int zero_start, const JacobiFirst* first = nullptr) {
     if (K <= 0) return FS2D_OK;
     SweepArgs A = sweep_args(x, b, h->R, h->P, kind, a, denom, mode, K, zero_start);
     if (h->prm.sweep_order == FS2D_ORDER_GS_LEX) {
@@ -362,7 +366,7 @@ int linear_solve(fs2d_handle* h, float*& x, const float* b, int kind, float a, f
     set.a[0] = A;
     set.count = 1;
     float **fx = &x, **ft = &h->f[F_SCRATCH];
-    return jacobi_solve(h, set, &fx, &ft);
+    return jacobi_solve(h, set, &fx, &ft, first);
 }
 
 int diffuse(fs2d_handle* h, float*& x, int mode, float rate, float dt, int K) {
@@ -379,12 +383,31 @@ bool pressure_needs_fill(fs2d_handle* h) {
     return !(h->prm.sweep_order == FS2D_ORDER_GS_LEX && !gs_units(h));
 }
 
+// Whether a solve's first launch forms its right-hand side: Jacobi block tiles, which
+// load whole regions (a Gauss-Seidel step's first projection has its own way).  Saves
+// three launches a step, the sources' pass (48 bytes a cell, of which the first launch
+// writes 12) and two divergences: a step at 201 x 201 94 -> 87 us, 1024 x 1024 272 ->
+// 250 us, 4096 x 4096 3.31 -> 3.18 ms.
+bool forms_rhs(const fs2d_handle* h) {
+    return h->prm.sweep_order == FS2D_ORDER_JACOBI && h->jacobi_kernel == FS2D_JACOBI_WAVE;
+}
+
 int project(fs2d_handle* h, int K) {
     const Scalars s = scalars(h->R, 1.0f);
     const bool fill = K > 0 && pressure_needs_fill(h);
-    FS2D_HIP(h, launch_divergence(h->stream, h->f[F_D], h->u(), h->v(), h->R, h->P, s.neg_half_h,
-                                  fill ? h->f[F_P] : nullptr));
-    int rc = linear_solve(h, h->f[F_P], h->f[F_D], SWEEP_PRESSURE, 0.f, 0.f, BND_CONT, K, fill ? 2 : 1);
+    JacobiFirst first;
+    if (K > 0 && forms_rhs(h)) {
+        first.any = true;
+        first.s0[0] = h->u();
+        first.s1 = h->v();
+        first.scale = s.neg_half_h;
+        first.b[0] = h->f[F_D];
+    } else {
+        FS2D_HIP(h, launch_divergence(h->stream, h->f[F_D], h->u(), h->v(), h->R, h->P, s.neg_half_h,
+                                      fill ? h->f[F_P] : nullptr));
+    }
+    int rc = linear_solve(h, h->f[F_P], h->f[F_D], SWEEP_PRESSURE, 0.f, 0.f, BND_CONT, K, fill ? 2 : 1,
+                          first.any ? &first : nullptr);
     if (rc) return rc;
     h->pressure_zero = (K <= 0);
     FS2D_HIP(h, launch_gradient(h->stream, h->u(), h->v(), h->f[F_P], h->R, h->P, s.h, h->pressure_zero ? 1 : 0,
@@ -553,8 +576,9 @@ int step_shared_diffuse(fs2d_handle* h, float diff, float visc, float dt) {
     const int Kd = h->prm.diffuse_iterations, Kp = h->prm.pressure_iterations;
     const int R = h->R, P = h->P;
     int rc;
-    FS2D_HIP(h, launch_add_sources3(h->stream, h->rho(), h->f[F_X0], h->f[F_RS], h->f[F_UN], h->f[F_X0U], h->u(),
-                                    h->f[F_US], h->f[F_VN], h->f[F_X0V], h->v(), h->f[F_VS], R, P, dt));
+    if (Kd <= 0 || !forms_rhs(h))
+        FS2D_HIP(h, launch_add_sources3(h->stream, h->rho(), h->f[F_X0], h->f[F_RS], h->f[F_UN], h->f[F_X0U], h->u(),
+                                        h->f[F_US], h->f[F_VN], h->f[F_X0V], h->v(), h->f[F_VS], R, P, dt));
     if (Kd > 0) {
         const float ad = dt * cells(R) * diff, av = dt * cells(R) * visc;
         const float dd = 1.f + 4.f * ad, dv = 1.f + 4.f * av;
@@ -593,7 +617,13 @@ int step_shared_diffuse(fs2d_handle* h, float diff, float visc, float dt) {
             // the advections' temporaries are free until the scatter
             float** const fields[3] = {&h->f[F_RHO], &h->f[F_UN], &h->f[F_VN]};
             float** const scratch[3] = {&h->f[F_SCRATCH], &h->f[F_T1], &h->f[F_T2]};
-            if ((rc = jacobi_solve(h, set, fields, scratch))) return rc;
+            const JacobiFirst first{true,
+                                    {h->rho(), h->u(), h->v()},
+                                    {h->f[F_RS], h->f[F_US], h->f[F_VS]},
+                                    nullptr,
+                                    dt,
+                                    {h->f[F_X0], h->f[F_X0U], h->f[F_X0V]}};
+            if ((rc = jacobi_solve(h, set, fields, scratch, &first))) return rc;
         } else {
             const GsPlan* plan = nullptr;
             FS2D_HIP(h, gs_plan_for(h, Kd, SWEEP_DIFFUSE, &plan));
@@ -1355,7 +1385,8 @@ static int fs2d_hip_launches_per_step_impl(fs2d_handle* h, int* launches) {
         *launches = 1 + 1 + joint_levels(joint) + scatter_launches(h->R) + 2 + 1 + 1 + p + 2;
         return FS2D_OK;
     }
-    // adds (one launch shared, x3 otherwise), diffuse (x3, or x1 shared), scatter,
+    // passes, one by one where Jacobi fields share a launch or a solve's first launch
+    // forms its right-hand side: adds (one shared, x3 otherwise), diffuse (x3, or x1 shared), scatter,
     // project x2 (div + solve + grad), gather
     *launches = (shared ? 1 : 3) + (shared ? d : 3 * d) + scatter_launches(h->R) + 2 * (2 + p) + 1;
     return FS2D_OK;

@@ -88,19 +88,6 @@ __device__ __forceinline__ bool cell_of(const BatchSim* __restrict__ sims, const
     return i <= R - 2 && j <= R - 2;
 }
 
-__global__ __launch_bounds__(CBX* CBY) void kb_add_sources(const BatchSim* __restrict__ sims,
-                                                           const int2* __restrict__ work, int nwork, Roles r) {
-    for (int e = blockIdx.x; e < nwork; e += gridDim.x) {
-        int s, i, j, blk;
-        if (!cell_of(sims, work, e, nwork, s, i, j, blk)) continue;
-        const BatchSim& S = sims[s];
-        const size_t o = S.off;
-        cells::add_sources(r.a[A_RHO] + o, r.a[A_X0] + o, r.a[A_RS] + o, S.P, S.dt, i, j);
-        cells::add_sources_split(r.a[A_UN] + o, r.a[A_X0U] + o, r.a[A_U] + o, r.a[A_US] + o, S.R, S.P, S.dt, i, j);
-        cells::add_sources_split(r.a[A_VN] + o, r.a[A_X0V] + o, r.a[A_V] + o, r.a[A_VS] + o, S.R, S.P, S.dt, i, j);
-    }
-}
-
 // Block maximum of the largest finite |u|, |v| into one of the simulation's
 // slots (k_fold folds them).  Ends with a barrier, so a persistent block may
 // reduce its next entry at once.
@@ -152,18 +139,6 @@ __global__ __launch_bounds__(CBX* CBY) void kb_gather_velocity(const BatchSim* _
     }
 }
 
-__global__ __launch_bounds__(CBX* CBY) void kb_divergence(const BatchSim* __restrict__ sims,
-                                                          const int2* __restrict__ work, int nwork, Roles r) {
-    for (int e = blockIdx.x; e < nwork; e += gridDim.x) {
-        int s, i, j, blk;
-        if (!cell_of(sims, work, e, nwork, s, i, j, blk)) continue;
-        const BatchSim& S = sims[s];
-        const size_t o = S.off;
-        // the pressure iterate needs no zero fill: its first Jacobi launch reads zeros itself
-        cells::divergence(r.a[A_D] + o, r.a[A_U] + o, r.a[A_V] + o, S.R, S.P, S.neg_half_h, nullptr, i, j);
-    }
-}
-
 __global__ __launch_bounds__(CBX* CBY) void kb_gradient(const BatchSim* __restrict__ sims,
                                                         const int2* __restrict__ work, int nwork, Roles r,
                                                         unsigned* __restrict__ slots) {
@@ -193,7 +168,9 @@ __global__ __launch_bounds__(CBX* CBY) void kb_gradient(const BatchSim* __restri
 // 0.40 ms; of 96 rows 1.21 / 0.38 ms.
 constexpr int JB_WAVES = 8;
 
-template <int RPW, int KIND>
+// A solve's first launch (FIRST, j = 0) forms its right-hand sides: the sources' terms
+// of density, u and v, or the divergence.
+template <int RPW, int KIND, bool FIRST>
 __global__ __launch_bounds__(64 * JB_WAVES) void kb_jacobi(const BatchSim* __restrict__ sims,
                                                            const int2* __restrict__ work, int n_work, Roles r,
                                                            int j) {
@@ -216,6 +193,10 @@ __global__ __launch_bounds__(64 * JB_WAVES) void kb_jacobi(const BatchSim* __res
             t.rg = ring_of(BND_CONT);
             t.a = 0.f;
             t.dv = jac::Divisor{};
+            t.s0 = r.a[A_U] + o;
+            t.s1 = r.a[A_V] + o;
+            t.scale = S.neg_half_h;
+            t.b_out = r.a[A_D] + o;
         } else {
             home = r.a[f == 0 ? A_RHO : (f == 1 ? A_UN : A_VN)] + o;
             t.b = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
@@ -225,10 +206,16 @@ __global__ __launch_bounds__(64 * JB_WAVES) void kb_jacobi(const BatchSim* __res
             t.a = f == 0 ? S.a_rho : S.a_vel;
             t.dv = f == 0 ? S.dv_rho : S.dv_vel;
             checked = (f == 0 ? S.checked_rho : S.checked_vel) != 0;
+            // u and v go to fresh iterates: the density scatter reads the pre-step
+            // velocity (:16-24)
+            t.src = r.a[f == 0 ? A_RHO : (f == 1 ? A_U : A_V)] + o;
+            t.s0 = r.a[f == 0 ? A_RS : (f == 1 ? A_US : A_VS)] + o;
+            t.scale = S.dt;
+            t.b_out = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
         }
-        t.src = (j == 0) ? home : (((j - 1) & 1) ? s2 : s1);
+        if (!FIRST) t.src = ((j - 1) & 1) ? s2 : s1;
         t.dst = (j == S.launches - 1) ? home : ((j & 1) ? s2 : s1);
-        t.zero = KIND == SWEEP_PRESSURE && j == 0;
+        t.zero = false;
         // tiles are placed for the longest launch
         t.m = S.sweeps + (S.longer > 0);
         const int tiles_y = jac::tile_count(t.R, RPW * JB_WAVES, t.m), tiles_x = jac::tile_count(t.R, jac::kTileCols, t.m);
@@ -236,11 +223,11 @@ __global__ __launch_bounds__(64 * JB_WAVES) void kb_jacobi(const BatchSim* __res
         jac::tile_place(t, RPW * JB_WAVES, ty, w.y - ty * tiles_x, tiles_y, tiles_x);
         t.m = S.sweeps + (j < S.longer);
         if constexpr (KIND == SWEEP_PRESSURE)
-            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_PRESSURE>(t, ex);
+            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_PRESSURE, FIRST ? jac::TILE_DIVERGENCE : jac::TILE_STORED>(t, ex);
         else if (checked)
-            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_DIFFUSE_CHECKED>(t, ex);
+            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_DIFFUSE_CHECKED, FIRST ? jac::TILE_SOURCES : jac::TILE_STORED>(t, ex);
         else
-            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_DIFFUSE>(t, ex);
+            jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_DIFFUSE, FIRST ? jac::TILE_SOURCES : jac::TILE_STORED>(t, ex);
         __syncthreads();  // the next tile's first exchange may take the buffer of this one's last
     }
 }
@@ -258,12 +245,18 @@ unsigned persistent_grid(int n, int per_block, int limit) {
     return static_cast<unsigned>(std::max(8, limit - limit % 8));
 }
 
+template <int RPW, int KIND>
+void launch_kb_jacobi_kind(hipStream_t st, const BatchSim* sims, const int2* w, int n, Roles r, int j, int limit) {
+    const dim3 grid(persistent_grid(n, 1, limit)), block(64 * JB_WAVES);
+    if (j == 0) hipLaunchKernelGGL((kb_jacobi<RPW, KIND, true>), grid, block, 0, st, sims, w, n, r, j);
+    else hipLaunchKernelGGL((kb_jacobi<RPW, KIND, false>), grid, block, 0, st, sims, w, n, r, j);
+}
+
 template <int RPW>
 void launch_kb_jacobi_rows(hipStream_t st, int kind, const BatchSim* sims, const int2* w, int n, Roles r, int j,
                            int limit) {
-    const dim3 grid(persistent_grid(n, 1, limit)), block(64 * JB_WAVES);
-    if (kind == SWEEP_DIFFUSE) hipLaunchKernelGGL((kb_jacobi<RPW, SWEEP_DIFFUSE>), grid, block, 0, st, sims, w, n, r, j);
-    else hipLaunchKernelGGL((kb_jacobi<RPW, SWEEP_PRESSURE>), grid, block, 0, st, sims, w, n, r, j);
+    if (kind == SWEEP_DIFFUSE) launch_kb_jacobi_kind<RPW, SWEEP_DIFFUSE>(st, sims, w, n, r, j, limit);
+    else launch_kb_jacobi_kind<RPW, SWEEP_PRESSURE>(st, sims, w, n, r, j, limit);
 }
 
 hipError_t launch_kb_jacobi(hipStream_t st, int rows, int kind, const BatchSim* sims, const int2* w, int n, Roles r,
@@ -392,8 +385,6 @@ hipError_t cell_launch_check() { return hipGetLastError(); }
 
 int project(fs2d_batch* b) {
     const dim3 grid = cell_grid(b), blk(CBX, CBY);
-    hipLaunchKernelGGL(kb_divergence, grid, blk, 0, b->stream, b->sims, b->cell_work, b->cell_blocks, b->roles);
-    FS2D_BHIP(b, cell_launch_check());
     int rc = solve(b, SWEEP_PRESSURE);
     if (rc) return rc;
     hipLaunchKernelGGL(kb_gradient, grid, blk, 0, b->stream, b->sims, b->cell_work, b->cell_blocks, b->roles,
@@ -414,11 +405,6 @@ int step(fs2d_batch* b) {
         FS2D_BHIP(b, cell_launch_check());
         b->speed_valid = true;
     }
-    // sources of all three fields; u and v go to fresh iterates so that the
-    // density scatter still reads the pre-step velocity (:16-24)
-    hipLaunchKernelGGL(kb_add_sources, cell_grid(b), blk, 0, b->stream, b->sims, b->cell_work, b->cell_blocks,
-                       b->roles);
-    FS2D_BHIP(b, cell_launch_check());
     if ((rc = solve(b, SWEEP_DIFFUSE))) return rc;
     FS2D_BHIP(b, launch_batch_scatter(b->stream, b->scatter, b->roles.a[A_T1], b->roles.a[A_RHO], b->roles.a[A_U],
                                       b->roles.a[A_V], b->max_bits));
@@ -765,8 +751,8 @@ static int fs2d_hip_batch_info_impl(fs2d_batch* b, int* depth, int* tile_rows, i
     if (depth) *depth = b->prm.jacobi_block ? b->prm.jacobi_block : 1;
     if (tile_rows) *tile_rows = b->jacobi.rows - 2 * jac::kTileMaxSweeps;
     if (launches) {
-        // max speed (first step only) aside: add, diffuse launches, the scatter's
-        // kernels, 2 x (divergence, pressure launches, gradient, fold), gather
+        // max speed (first step only) aside, the passes of a step: add, diffuse launches, the scatter's
+        // kernels, 2 x (divergence, pressure launches, gradient, fold), gather; adds and divergences made by first launches
         const int d = static_cast<int>(b->jacobi.diffuse_count.size());
         const int p = static_cast<int>(b->jacobi.pressure_count.size());
         *launches = b->steps_done > 0 ? 1 + d + batch_scatter_launches(b->scatter.targets) + 2 * (3 + p) + 1 : 0;

@@ -277,12 +277,26 @@ enum JacobiKernel : int { JACOBI_WAVE = 1, JACOBI_LDS = 2 };
 // odd number of launches the result is in scratch.  The set's fields (one to three
 // of a kind, size and sweep count) share each JACOBI_WAVE launch; scratch[f] is
 // field f's.
-hipError_t launch_jacobi_solve(hipStream_t s, const SweepSet& set, float* const* scratch, int block, int kernel);
+//
+// A solve's first launch can form the right-hand sides itself (JACOBI_WAVE only) and
+// store them in b[f], the set's own: with any set, a set of diffuses starts from
+// src[f] + scale s0[f] (src[f] in place of the iterate, left as it is), a pressure
+// solve from the divergence of (s0[0], s1) times scale.
+struct JacobiFirst {
+    bool any = false;
+    const float* src[3] = {};
+    const float* s0[3] = {};
+    const float* s1 = nullptr;
+    float scale = 0.f;
+    float* b[3] = {};
+};
+hipError_t launch_jacobi_solve(hipStream_t s, const SweepSet& set, float* const* scratch, int block, int kernel,
+                               const JacobiFirst* first = nullptr);
 // One launch (JACOBI_LDS: one per field) of m fused sweeps, m in 1..8, from src[f] into dst[f].
 hipError_t launch_jacobi_pass(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
-                              int zero_src, int m, int kernel);
+                              int zero_src, int m, int kernel, const JacobiFirst* first = nullptr);
 hipError_t launch_jacobi_tiles(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
-                               int zero_src, int m);
+                               int zero_src, int m, const JacobiFirst* first);
 int jacobi_launches(int K, int block);
 
 }  // namespace fs2d

@@ -11,11 +11,12 @@ struct TileSet {
     SweepArgs a[3];
     const float* src[3];
     float* dst[3];
+    JacobiFirst first;
     int m, zero, tiles_x, tiles_y;
 };
 
 // Block: tile blockIdx.x of field blockIdx.y.
-template <int RPW, int NW, int KIND>
+template <int RPW, int NW, int KIND, int LOAD>
 __global__ __launch_bounds__(64 * NW) void k_jacobi_tile(TileSet S) {
     __shared__ float ex[4 * NW * kTileCols];
     const int f = blockIdx.y, b = xcd_block(blockIdx.x, gridDim.x);
@@ -31,8 +32,18 @@ __global__ __launch_bounds__(64 * NW) void k_jacobi_tile(TileSet S) {
     t.a = A.a;
     t.dv = divisor_of(A);
     t.rg = A.ring;
+    t.s0 = S.first.s0[f];
+    t.s1 = S.first.s1;
+    t.scale = S.first.scale;
+    t.b_out = S.first.b[f];
     tile_place(t, NW * RPW, b / S.tiles_x, b % S.tiles_x, S.tiles_y, S.tiles_x);
-    jacobi_tile_any<RPW, NW, KIND>(t, ex);
+    jacobi_tile_any<RPW, NW, KIND, LOAD>(t, ex);
+}
+
+template <int RPW, int NW, int KIND, int FIRST>
+void launch_kind(hipStream_t s, const TileSet& S, dim3 grid, dim3 block) {
+    if (S.first.any) hipLaunchKernelGGL((k_jacobi_tile<RPW, NW, KIND, FIRST>), grid, block, 0, s, S);
+    else hipLaunchKernelGGL((k_jacobi_tile<RPW, NW, KIND, TILE_STORED>), grid, block, 0, s, S);
 }
 
 template <int RPW, int NW>
@@ -41,10 +52,9 @@ hipError_t launch(hipStream_t s, TileSet& S, int fields, int kind) {
     S.tiles_y = tile_count(R, NW * RPW, S.m);
     S.tiles_x = tile_count(R, kTileCols, S.m);
     const dim3 grid(S.tiles_x * S.tiles_y, fields), block(64 * NW);
-    if (kind == TILE_PRESSURE) hipLaunchKernelGGL((k_jacobi_tile<RPW, NW, TILE_PRESSURE>), grid, block, 0, s, S);
-    else if (kind == TILE_DIFFUSE_CHECKED)
-        hipLaunchKernelGGL((k_jacobi_tile<RPW, NW, TILE_DIFFUSE_CHECKED>), grid, block, 0, s, S);
-    else hipLaunchKernelGGL((k_jacobi_tile<RPW, NW, TILE_DIFFUSE>), grid, block, 0, s, S);
+    if (kind == TILE_PRESSURE) launch_kind<RPW, NW, TILE_PRESSURE, TILE_DIVERGENCE>(s, S, grid, block);
+    else if (kind == TILE_DIFFUSE_CHECKED) launch_kind<RPW, NW, TILE_DIFFUSE_CHECKED, TILE_SOURCES>(s, S, grid, block);
+    else launch_kind<RPW, NW, TILE_DIFFUSE, TILE_SOURCES>(s, S, grid, block);
     return hipGetLastError();
 }
 
@@ -68,7 +78,7 @@ hipError_t launch(hipStream_t s, TileSet& S, int fields, int kind) {
 static int tile_rows(long cells) { return cells < 500000 ? 32 : (cells < 8000000 ? 48 : 96); }
 
 hipError_t launch_jacobi_tiles(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
-                               int zero_src, int m) {
+                               int zero_src, int m, const JacobiFirst* first) {
     if (m < 1 || m > kTileMaxSweeps || set.count < 1 || set.count > 3) return hipErrorInvalidValue;
     TileSet S{};
     bool checked = true;
@@ -78,6 +88,7 @@ hipError_t launch_jacobi_tiles(hipStream_t s, const SweepSet& set, const float* 
         S.src[f] = src[f];
         S.dst[f] = dst[f];
     }
+    if (first) S.first = *first;
     S.m = m;
     S.zero = zero_src;
     const int kind = set.a[0].kind == SWEEP_PRESSURE ? TILE_PRESSURE : (checked ? TILE_DIFFUSE_CHECKED : TILE_DIFFUSE);

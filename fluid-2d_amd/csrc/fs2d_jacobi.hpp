@@ -126,9 +126,22 @@ __device__ __forceinline__ float lane_east(float x) {  // lane l receives lane l
 // sign-adjusted value of the cell itself, after that.
 constexpr int kTileMaxSweeps = 8, kTileCols = 64;
 
+// What a tile loads.  TILE_STORED: the iterate and the right-hand side b.  The first
+// launch of a solve can form b from what b's own pass would read, and store it for the
+// launches after it, so that pass's launch and its reads and writes fall away:
+//   TILE_SOURCES     b and the iterate are src + scale s0 (src_x + dt s, a step's source
+//                    term); ring cells of the iterate are src's
+//   TILE_DIVERGENCE  b is the divergence scale (((s0E - s0W) + s1S) - s1N) of a velocity
+//                    s0, s1; the iterate starts as zero
+// A cell of the halo is formed by every tile that holds it, the same each time.
+enum TileLoad : int { TILE_STORED = 0, TILE_SOURCES = 1, TILE_DIVERGENCE = 2 };
+
 struct TileJob {
     const float *src, *b;
     float* dst;
+    const float *s0, *s1;  // TILE_SOURCES, TILE_DIVERGENCE
+    float scale;
+    float* b_out;
     int R, P, m;
     bool zero;  // the iterate starts as zero (src is not read)
     float a;
@@ -181,16 +194,49 @@ __device__ __forceinline__ float relax_tile(float b, float n, float s, float w, 
 // addition.  2 / 3: anywhere (a grid smaller than the region, or one with both columns
 // in it), tested by index in every row.
 // ex: 4 NW kTileCols floats of LDS.
-template <int RPW, int NW, int KIND, int ROWS, int COLS>
+template <int RPW, int NW, int KIND, int LOAD, int ROWS, int COLS>
 __device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict__ ex) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int R = t.R, P = t.P, n = R - 2, i0 = t.gi0 + wave * RPW, gj = t.gj0 + lane;
     const int cj = min(gj, R - 1);  // a grid narrower than the region
     float X[RPW + 1], B[RPW];
+    if constexpr (LOAD == TILE_STORED) {
 #pragma unroll
-    for (int r = 0; r < RPW; ++r) X[r + 1] = t.zero ? 0.f : t.src[(size_t)min(i0 + r, R - 1) * P + cj];
+        for (int r = 0; r < RPW; ++r) X[r + 1] = t.zero ? 0.f : t.src[(size_t)min(i0 + r, R - 1) * P + cj];
 #pragma unroll
-    for (int r = 0; r < RPW; ++r) B[r] = t.b[(size_t)min(i0 + r, R - 1) * P + cj];
+        for (int r = 0; r < RPW; ++r) B[r] = t.b[(size_t)min(i0 + r, R - 1) * P + cj];
+    } else {
+        if constexpr (LOAD == TILE_SOURCES) {
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) X[r + 1] = t.src[(size_t)min(i0 + r, R - 1) * P + cj];
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) B[r] = t.s0[(size_t)min(i0 + r, R - 1) * P + cj];
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) {
+                B[r] = X[r + 1] + t.scale * B[r];
+                const bool ring = (ROWS && (i0 + r < 1 || i0 + r > n)) || (COLS && (gj < 1 || gj > n));
+                X[r + 1] = ring ? X[r + 1] : B[r];
+            }
+        } else {
+            // the region's first and last rows and lanes lack a neighbour; they are
+            // ring or lost to the first sweep
+            float V[RPW + 2];
+#pragma unroll
+            for (int r = 0; r < RPW + 2; ++r) V[r] = t.s1[(size_t)max(min(i0 + r - 1, R - 1), 0) * P + cj];
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) B[r] = t.s0[(size_t)min(i0 + r, R - 1) * P + cj];
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) {
+                B[r] = t.scale * (((lane_east(B[r]) - lane_west(B[r])) + V[r + 2]) - V[r]);
+                X[r + 1] = 0.f;
+            }
+        }
+        if (gj >= t.jlo && gj <= t.jhi) {
+#pragma unroll
+            for (int r = 0; r < RPW; ++r)
+                if (i0 + r >= t.ilo && i0 + r <= t.ihi) t.b_out[(size_t)(i0 + r) * P + gj] = B[r];
+        }
+    }
 
     const float a = t.a;
     const Divisor dv = t.dv;
@@ -276,19 +322,19 @@ __device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict_
     }
 }
 
-template <int RPW, int NW, int KIND>
+template <int RPW, int NW, int KIND, int LOAD>
 __device__ __forceinline__ void jacobi_tile_any(const TileJob& t, float* __restrict__ ex) {
     const bool left = t.gj0 == 0, right = t.gj0 + kTileCols >= t.R;
     if (t.R < NW * RPW || (left && right)) {
-        jacobi_tile<RPW, NW, KIND, 2, 3>(t, ex);
+        jacobi_tile<RPW, NW, KIND, LOAD, 2, 3>(t, ex);
     } else if (t.gi0 == 0 || t.gi0 + NW * RPW == t.R) {
-        if (left) jacobi_tile<RPW, NW, KIND, 1, 1>(t, ex);
-        else if (right) jacobi_tile<RPW, NW, KIND, 1, 2>(t, ex);
-        else jacobi_tile<RPW, NW, KIND, 1, 0>(t, ex);
+        if (left) jacobi_tile<RPW, NW, KIND, LOAD, 1, 1>(t, ex);
+        else if (right) jacobi_tile<RPW, NW, KIND, LOAD, 1, 2>(t, ex);
+        else jacobi_tile<RPW, NW, KIND, LOAD, 1, 0>(t, ex);
     } else {
-        if (left) jacobi_tile<RPW, NW, KIND, 0, 1>(t, ex);
-        else if (right) jacobi_tile<RPW, NW, KIND, 0, 2>(t, ex);
-        else jacobi_tile<RPW, NW, KIND, 0, 0>(t, ex);
+        if (left) jacobi_tile<RPW, NW, KIND, LOAD, 0, 1>(t, ex);
+        else if (right) jacobi_tile<RPW, NW, KIND, LOAD, 0, 2>(t, ex);
+        else jacobi_tile<RPW, NW, KIND, LOAD, 0, 0>(t, ex);
     }
 }
 

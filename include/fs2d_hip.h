@@ -48,7 +48,7 @@ enum fs2d_sweep_order {
 
 /* Kernel that runs the Jacobi sweeps (identical results). */
 enum fs2d_jacobi_kernel {
-    FS2D_JACOBI_WAVE = 1, /* one wave per tile, rows in registers, lanes exchange by DPP (default) */
+    FS2D_JACOBI_WAVE = 1, /* 8 waves per tile, rows in registers, lanes exchange by DPP (default)   */
     FS2D_JACOBI_LDS = 2   /* 256-thread blocks, halo exchange through LDS                         */
 };
 
@@ -198,7 +198,8 @@ int fs2d_division_plan(float denom, float* inv, float* inv_lo, float* two_hi, fl
 int fs2d_hip_copy_bandwidth(long long bytes, int reps, float* gb_per_s);
 /* Number of kernel launches one step enqueues (for per-launch averages).  In
  * the Jacobi order a launch that serves density, u and v together counts as
- * three: the figure is that of one field per launch. */
+ * three, and the sources' and divergence's passes count although a solve's first
+ * launch makes them: the figure is that of one field and one stage per launch. */
 int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches);
 
 /* ---- projection without allocation -------------------------------------
@@ -264,7 +265,8 @@ int fs2d_hip_batch_sync(fs2d_batch* b);
 /* The configuration in use: jacobi_depth, the sweeps every Jacobi launch takes a
  * multiple of (a fixed jacobi_block, else 1: a simulation's sweeps are spread evenly
  * over its launches), tile_rows, the rows an inner Jacobi tile writes after 8 sweeps,
- * kernel launches per step, captured step graphs, total interior cells. */
+ * passes per step (launches, counting the sources' and the divergences' passes that
+ * a solve's first launch makes), captured step graphs, total interior cells. */
 int fs2d_hip_batch_info(fs2d_batch* b, int* jacobi_depth, int* tile_rows, int* launches_per_step, int* graphs,
                         long long* interior_cells);
 /* The persistent launches' grid: blocks per compute unit for the Jacobi launches (8
