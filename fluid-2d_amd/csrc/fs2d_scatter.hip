@@ -113,7 +113,11 @@ __device__ __forceinline__ Shares shift_shares(const Shares& x) {
 
 // Layout of one launch for radius W: strips of 64 - 2W destination columns,
 // bands of `band` rows, one wave per (band, strip); `band` is the smallest
-// (at least 16) that keeps every wave resident at once (`slots` waves).
+// (at least kMinBand) that keeps every wave resident at once (`slots` waves).
+// A wave is a chain of band + 2W rows, so a grid that leaves the chip idle takes
+// short bands although neighbours then read more rows twice: at 200 x 200, 12.3 us with
+// bands of 16 rows and 6.0 with 4; from about 2500 x 2500 up the bands are as before.
+constexpr int kMinBand = 4;
 struct WindowLayout {
     int strips, band, waves;
 };
@@ -122,7 +126,7 @@ __host__ __device__ inline WindowLayout window_layout(int R, int W, int slots) {
     const int strips = (n + sw - 1) / sw;
     const int maxb = slots / strips > 1 ? slots / strips : 1;
     int band = (n + maxb - 1) / maxb;
-    band = band < 16 ? 16 : band;
+    band = band < kMinBand ? kMinBand : band;
     band = band > n ? n : band;
     return WindowLayout{strips, band, strips * ((n + band - 1) / band)};
 }
@@ -314,9 +318,21 @@ struct FlagGate {
 // Items are 64-bit: target cell i0 * (R - 1) + j0 in the high word (or
 // (R - 1)^2 for a skipped source, sorted last), the source's interior
 // row-major index in the low word.  The sort takes 9-bit digits over chunks of
-// CH items; every kernel walks its work with a grid of at most kSortBlocks
+// NT ipt items; every kernel walks its work with a grid of at most kSortBlocks
 // blocks, so that while the window path is active each returns at once.
-constexpr int IPT = 16, CH = NT * IPT;
+//
+// A chunk is a serial chain of ipt rounds, and the scan one block's walk over the
+// chunks' counts: up to 32 chunks cost the scan little, so grids up to 362 x 362 take
+// fewer rounds.  At 128 x 128 (4 chunks of 16 rounds before, 32 of 2 now), us: keys
+// 13.0 -> 4.7, each scatter 15.3 -> 4.6.
+constexpr int kMaxRounds = 16;
+inline int sort_rounds(long long N) {
+    return static_cast<int>(std::min<long long>(std::max<long long>((N + NT * 32 - 1) / (NT * 32), 1), kMaxRounds));
+}
+inline int sort_chunks(long long N) {
+    const long long chunk = (long long)NT * sort_rounds(N);
+    return static_cast<int>(std::max<long long>((N + chunk - 1) / chunk, 1));
+}
 constexpr int DB = 9, ND = 1 << DB;  // digit bits, digits
 constexpr int kSortBlocks = 512;
 
@@ -324,7 +340,7 @@ constexpr int kSortBlocks = 512;
 // ranges cleared.
 __global__ __launch_bounds__(NT) void k_sort_keys(unsigned long long* __restrict__ items, unsigned* __restrict__ hist,
                                                   int2* __restrict__ bounds, const float* __restrict__ u,
-                                                  const float* __restrict__ v, int R, int P, float dt0, int chunks,
+                                                  const float* __restrict__ v, int R, int P, float dt0, int chunks, int ipt,
                                                   const unsigned* __restrict__ max_bits) {
     if (scatter_radius(max_bits, dt0, R) <= kWindow) return;
     __shared__ unsigned cnt[ND];
@@ -336,8 +352,8 @@ __global__ __launch_bounds__(NT) void k_sort_keys(unsigned long long* __restrict
     for (int c = blockIdx.x; c < chunks; c += gridDim.x) {
         for (int d = threadIdx.x; d < ND; d += NT) cnt[d] = 0u;
         __syncthreads();
-        for (int q = 0; q < IPT; ++q) {
-            const long long s = (long long)c * CH + q * NT + threadIdx.x;
+        for (int q = 0; q < ipt; ++q) {
+            const long long s = ((long long)c * ipt + q) * NT + threadIdx.x;
             if (s >= N) break;
             const int si = 1 + (int)(s / n), sj = 1 + (int)(s % n);
             const size_t o = (size_t)si * P + sj;
@@ -357,14 +373,14 @@ __global__ __launch_bounds__(NT) void k_sort_keys(unsigned long long* __restrict
 // Chunk counts of digit (key >> shift) & (ND - 1): hist[digit * chunks + chunk].
 template <class G>
 __global__ __launch_bounds__(NT) void k_sort_hist(const unsigned long long* __restrict__ items, long long N, int shift,
-                                                  unsigned* __restrict__ hist, int chunks, G gate) {
+                                                  unsigned* __restrict__ hist, int chunks, int ipt, G gate) {
     if (!gate.sorted()) return;
     __shared__ unsigned cnt[ND];
     for (int c = blockIdx.x; c < chunks; c += gridDim.x) {
         for (int d = threadIdx.x; d < ND; d += NT) cnt[d] = 0u;
         __syncthreads();
-        for (int q = 0; q < IPT; ++q) {
-            const long long i = (long long)c * CH + q * NT + threadIdx.x;
+        for (int q = 0; q < ipt; ++q) {
+            const long long i = ((long long)c * ipt + q) * NT + threadIdx.x;
             if (i < N) atomicAdd(&cnt[(unsigned)(items[i] >> (32 + shift)) & (ND - 1)], 1u);
         }
         __syncthreads();
@@ -373,29 +389,59 @@ __global__ __launch_bounds__(NT) void k_sort_hist(const unsigned long long* __re
     }
 }
 
-// Exclusive scan of hist (digit-major) in place, one block.
+// Exclusive scan of hist (digit-major, 16-byte aligned, total a multiple of 4) in
+// place, one block, in tiles of 16 counts a thread: a wave holds 1024 counts, 16
+// bytes a lane and load, all of a tile's loads in flight at once.  Walking each
+// thread's share count by count cost a memory latency each.  A whole density advection whose
+// sources move 10 cells, before and after: 128 x 128 73 -> 38 us, 1024 x 1024 877 ->
+// 214 us, 4096 x 4096 14.3 -> 2.85 ms (the heads that merge_shares holds included).
 template <class G>
 __global__ __launch_bounds__(1024) void k_sort_scan(unsigned* __restrict__ hist, int total, G gate) {
     if (!gate.sorted()) return;
-    __shared__ unsigned part[1024];
-    const int t = threadIdx.x;
-    const int per = (total + 1023) / 1024;
-    const int lo = min(t * per, total), hi = min(lo + per, total);
-    unsigned sum = 0;
-    for (int k = lo; k < hi; ++k) sum += hist[k];
-    part[t] = sum;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {  // inclusive scan of the partial sums
-        const unsigned add = t >= off ? part[t - off] : 0u;
-        __syncthreads();
-        part[t] += add;
-        __syncthreads();
-    }
-    unsigned run = part[t] - sum;
-    for (int k = lo; k < hi; ++k) {
-        const unsigned c = hist[k];
-        hist[k] = run;
-        run += c;
+    constexpr int kQuads = 4;
+    __shared__ unsigned wave_sum[2][16];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    unsigned carry = 0;
+    int turn = 0;
+    for (int base = 0; base < total; base += 1024 * 4 * kQuads, turn ^= 1) {
+        const int at = base + w * 256 * kQuads + lane * 4;
+        uint4 c[kQuads];
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k)
+            c[k] = at + k * 256 < total ? *reinterpret_cast<const uint4*>(hist + at + k * 256) : make_uint4(0, 0, 0, 0);
+        unsigned incl[kQuads];  // of the lanes up to this one, per quad
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) incl[k] = c[k].x + c[k].y + c[k].z + c[k].w;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+            for (int k = 0; k < kQuads; ++k) {
+                const unsigned add = (unsigned)__shfl_up((int)incl[k], off);
+                incl[k] += lane >= off ? add : 0u;
+            }
+        unsigned before[kQuads], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) {
+            before[k] = sum;
+            sum += (unsigned)__shfl((int)incl[k], 63);
+        }
+        if (lane == 0) wave_sum[turn][w] = sum;
+        __syncthreads();  // two buffers: the next tile's sums may be written while these are read
+        unsigned run = carry;
+        for (int k = 0; k < 16; ++k) {
+            run += k < w ? wave_sum[turn][k] : 0u;
+            carry += wave_sum[turn][k];
+        }
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) {
+            if (at + k * 256 >= total) continue;
+            uint4 o;
+            o.x = run + before[k] + incl[k] - (c[k].x + c[k].y + c[k].z + c[k].w);
+            o.y = o.x + c[k].x;
+            o.z = o.y + c[k].y;
+            o.w = o.z + c[k].z;
+            *reinterpret_cast<uint4*>(hist + at + k * 256) = o;
+        }
     }
 }
 
@@ -404,7 +450,7 @@ __global__ __launch_bounds__(1024) void k_sort_scan(unsigned* __restrict__ hist,
 template <class G>
 __global__ __launch_bounds__(NT) void k_sort_scatter(const unsigned long long* __restrict__ in,
                                                      unsigned long long* __restrict__ out, long long N, int shift,
-                                                     const unsigned* __restrict__ offs, int chunks, G gate) {
+                                                     const unsigned* __restrict__ offs, int chunks, int ipt, G gate) {
     if (!gate.sorted()) return;
     __shared__ unsigned run[ND];           // items of each digit placed by earlier passes
     __shared__ unsigned wcnt[NT / 64][ND];  // items of each digit in each wave of this pass
@@ -412,11 +458,11 @@ __global__ __launch_bounds__(NT) void k_sort_scatter(const unsigned long long* _
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));  // lanes below this one
     for (int c = blockIdx.x; c < chunks; c += gridDim.x) {
         for (int d = t; d < ND; d += NT) run[d] = offs[d * chunks + c];
-        for (int q = 0; q < IPT; ++q) {
+        for (int q = 0; q < ipt; ++q) {
             for (int d = t; d < ND; d += NT)
                 for (int k = 0; k < NT / 64; ++k) wcnt[k][d] = 0u;
             __syncthreads();
-            const long long i = (long long)c * CH + q * NT + t;
+            const long long i = ((long long)c * ipt + q) * NT + t;
             const bool valid = i < N;
             const unsigned long long item = valid ? in[i] : 0ull;
             const unsigned dg = (unsigned)(item >> (32 + shift)) & (ND - 1);
@@ -458,9 +504,58 @@ __global__ __launch_bounds__(NT) void k_sort_bounds(const unsigned long long* __
     }
 }
 
-// Each destination merges, in source order, the sources of the four target
-// cells whose shares reach it: (di, dj) takes s1 s3 from target (di, dj),
-// s1 s2 from (di - 1, dj), s0 s3 from (di, dj - 1), s0 s2 from (di - 1, dj - 1).
+// Destination (di, dj) of a grid merges, in source order, the sources of the four
+// target cells whose shares reach it: it takes s1 s3 from target (di, dj), s1 s2 from
+// (di - 1, dj), s0 s3 from (di, dj - 1), s0 s2 from (di - 1, dj - 1).  base: the
+// sources' number of the grid's first cell.  The four lists' next sources stay in
+// registers, so a list's next entry is loaded beside the source it follows.
+__device__ __forceinline__ float merge_shares(const float* __restrict__ rho0, const float* __restrict__ u,
+                                              const float* __restrict__ v, const unsigned long long* __restrict__ items,
+                                              const int2* __restrict__ bounds, unsigned base, int R, int P, float dt0,
+                                              int di, int dj) {
+    constexpr unsigned kNone = 0xffffffffu;
+    const unsigned n = R - 2;
+    const float hi = (float)R - 1.5f;
+    const int ti[4] = {di, di - 1, di, di - 1}, tj[4] = {dj, dj, dj - 1, dj - 1};
+    int cur[4], end[4];
+    unsigned head[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int2 b = bounds[(size_t)ti[k] * (R - 1) + tj[k]];
+        cur[k] = b.x;
+        end[k] = b.y;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) head[k] = cur[k] < end[k] ? (unsigned)items[cur[k]] : kNone;
+    float acc = 0.f;
+    for (;;) {
+        const unsigned bs = min(min(head[0], head[1]), min(head[2], head[3]));
+        if (bs == kNone) break;
+        const int best = head[0] == bs ? 0 : (head[1] == bs ? 1 : (head[2] == bs ? 2 : 3));
+        const unsigned src = bs - base;
+        const int si = 1 + (int)(src / n), sj = 1 + (int)(src % n);
+        const size_t o = (size_t)si * P + sj;
+        const float uu = u[o], vv = v[o], r0 = rho0[o];
+        int next = 0, last = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            cur[k] += best == k;
+            next = best == k ? cur[k] : next;
+            last = best == k ? end[k] : last;
+        }
+        const unsigned h = next < last ? (unsigned)items[next] : kNone;
+        int i0, j0;
+        float s0, s2;
+        source_lands(si, sj, uu, vv, dt0, hi, i0, j0, s0, s2);
+        const float s1 = 1.0f - s0, s3 = 1.0f - s2;
+        const float sh = (best == 0) ? s1 * s3 * r0 : (best == 1) ? s1 * s2 * r0 : (best == 2) ? s0 * s3 * r0 : s0 * s2 * r0;
+        acc = acc + sh;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) head[k] = best == k ? h : head[k];
+    }
+    return acc;
+}
+
 __global__ __launch_bounds__(NT) void k_scatter_merge(float* __restrict__ out, const float* __restrict__ rho0,
                                                       const float* __restrict__ u, const float* __restrict__ v,
                                                       const unsigned long long* __restrict__ items,
@@ -468,40 +563,9 @@ __global__ __launch_bounds__(NT) void k_scatter_merge(float* __restrict__ out, c
                                                       const unsigned* __restrict__ max_bits) {
     if (scatter_radius(max_bits, dt0, R) <= kWindow) return;
     const int n = R - 2;
-    const float hi = (float)R - 1.5f;
     for (long long c = (long long)blockIdx.x * NT + threadIdx.x; c < (long long)n * n; c += (long long)gridDim.x * NT) {
         const int di = 1 + (int)(c / n), dj = 1 + (int)(c % n);
-        int cur[4], end[4];
-        const int ti[4] = {di, di - 1, di, di - 1}, tj[4] = {dj, dj, dj - 1, dj - 1};
-        for (int k = 0; k < 4; ++k) {
-            const int2 b = bounds[(size_t)ti[k] * (R - 1) + tj[k]];
-            cur[k] = b.x;
-            end[k] = b.y;
-        }
-        float acc = 0.f;
-        for (;;) {
-            int best = -1;
-            unsigned bs = 0xffffffffu;
-            for (int k = 0; k < 4; ++k) {
-                if (cur[k] >= end[k]) continue;
-                const unsigned s = (unsigned)items[cur[k]];
-                if (s < bs) {
-                    bs = s;
-                    best = k;
-                }
-            }
-            if (best < 0) break;
-            ++cur[best];
-            const int si = 1 + (int)(bs / (unsigned)n), sj = 1 + (int)(bs % (unsigned)n);
-            const size_t o = (size_t)si * P + sj;
-            int i0, j0;
-            float s0, s2;
-            source_lands(si, sj, u[o], v[o], dt0, hi, i0, j0, s0, s2);
-            const float s1 = 1.0f - s0, s3 = 1.0f - s2;
-            const float r0 = rho0[o];
-            const float sh = (best == 0) ? s1 * s3 * r0 : (best == 1) ? s1 * s2 * r0 : (best == 2) ? s0 * s3 * r0 : s0 * s2 * r0;
-            acc = acc + sh;
-        }
+        const float acc = merge_shares(rho0, u, v, items, bounds, 0u, R, P, dt0, di, dj);
         out[(size_t)di * P + dj] = acc;
         cells::write_ring(out, di, dj, acc, R, P, Ring{false, false});
     }
@@ -566,7 +630,7 @@ __device__ __forceinline__ int sim_of_cell(const ScatterSim* __restrict__ sims, 
 __global__ __launch_bounds__(NT) void k_bsort_keys(unsigned long long* __restrict__ items, unsigned* __restrict__ hist,
                                                    int2* __restrict__ bounds, const float* __restrict__ u,
                                                    const float* __restrict__ v, const ScatterSim* __restrict__ sims,
-                                                   int count, long long N, unsigned nb, int chunks,
+                                                   int count, long long N, unsigned nb, int chunks, int ipt,
                                                    const unsigned* __restrict__ max_bits, FlagGate gate) {
     if (!gate.sorted()) return;
     __shared__ unsigned cnt[ND];
@@ -575,8 +639,8 @@ __global__ __launch_bounds__(NT) void k_bsort_keys(unsigned long long* __restric
     for (int c = blockIdx.x; c < chunks; c += gridDim.x) {
         for (int d = threadIdx.x; d < ND; d += NT) cnt[d] = 0u;
         __syncthreads();
-        for (int q = 0; q < IPT; ++q) {
-            const long long g = (long long)c * CH + q * NT + threadIdx.x;
+        for (int q = 0; q < ipt; ++q) {
+            const long long g = ((long long)c * ipt + q) * NT + threadIdx.x;
             if (g >= N) break;
             const int s = sim_of_cell(sims, count, (unsigned)g);
             const ScatterSim S = sims[s];
@@ -613,41 +677,10 @@ __global__ __launch_bounds__(NT) void k_bscatter_merge(float* __restrict__ out, 
         const ScatterSim S = sims[s];
         if (scatter_radius(max_bits + s, S.dt0, S.R) <= kWindow) continue;
         const int n = S.R - 2, R = S.R, P = S.P;
-        const float hi = (float)R - 1.5f;
         const int local = (int)((unsigned)g - S.cells);
         const int di = 1 + local / n, dj = 1 + local % n;
-        int cur[4], end[4];
-        const int ti[4] = {di, di - 1, di, di - 1}, tj[4] = {dj, dj, dj - 1, dj - 1};
-        for (int k = 0; k < 4; ++k) {
-            const int2 b = bounds[(size_t)S.targets + (size_t)ti[k] * (R - 1) + tj[k]];
-            cur[k] = b.x;
-            end[k] = b.y;
-        }
-        float acc = 0.f;
-        for (;;) {
-            int best = -1;
-            unsigned bs = 0xffffffffu;
-            for (int k = 0; k < 4; ++k) {
-                if (cur[k] >= end[k]) continue;
-                const unsigned src = (unsigned)items[cur[k]];
-                if (src < bs) {
-                    bs = src;
-                    best = k;
-                }
-            }
-            if (best < 0) break;
-            ++cur[best];
-            const int sl = (int)(bs - S.cells);
-            const int si = 1 + sl / n, sj = 1 + sl % n;
-            const size_t o = S.off + (size_t)si * P + sj;
-            int i0, j0;
-            float s0, s2;
-            source_lands(si, sj, u[o], v[o], S.dt0, hi, i0, j0, s0, s2);
-            const float s1 = 1.0f - s0, s3 = 1.0f - s2;
-            const float r0 = rho0[o];
-            const float sh = (best == 0) ? s1 * s3 * r0 : (best == 1) ? s1 * s2 * r0 : (best == 2) ? s0 * s3 * r0 : s0 * s2 * r0;
-            acc = acc + sh;
-        }
+        const float acc = merge_shares(rho0 + S.off, u + S.off, v + S.off, items, bounds + S.targets, S.cells, R, P,
+                                       S.dt0, di, dj);
         float* o = out + S.off;
         o[(size_t)di * P + dj] = acc;
         cells::write_ring(o, di, dj, acc, R, P, Ring{false, false});
@@ -665,6 +698,11 @@ static int key_bits(unsigned long long nb) {
 // Targets 0 .. (R - 1)^2 of one grid.
 static int sort_key_bits(int R) { return key_bits((unsigned long long)(R - 1) * (unsigned long long)(R - 1)); }
 
+// The histograms lie after the bounds, 16-byte aligned (within the scratch's slack).
+static unsigned* sort_hist(void* after) {
+    return reinterpret_cast<unsigned*>((reinterpret_cast<uintptr_t>(after) + 15) & ~static_cast<uintptr_t>(15));
+}
+
 int scatter_launches(int R) {
     const int passes = (sort_key_bits(R) + DB - 1) / DB;
     return 3 + 3 * passes;  // window, keys, (passes - 1) histograms, passes x (scan, scatter), bounds, merge
@@ -673,7 +711,7 @@ int scatter_launches(int R) {
 size_t scatter_sort_bytes(int R) {
     const size_t n = static_cast<size_t>(R - 2);
     const size_t N = n * n;
-    const size_t chunks = std::max<size_t>((N + CH - 1) / CH, 1);
+    const size_t chunks = sort_chunks(static_cast<long long>(N));
     return 2 * N * sizeof(unsigned long long) + static_cast<size_t>(R - 1) * (R - 1) * sizeof(int2) +
            ND * chunks * sizeof(unsigned) + 4096;
 }
@@ -690,16 +728,16 @@ hipError_t launch_scatter_density(hipStream_t s, float* out, const float* rho0, 
     if (!sort_scratch) return hipGetLastError();
     // sorted path (returns at once while the window path is active)
     const long long N = (long long)n * n;
-    const int chunks = static_cast<int>(std::max<long long>((N + CH - 1) / CH, 1));
+    const int chunks = sort_chunks(N), ipt = sort_rounds(N);
     auto* items0 = static_cast<unsigned long long*>(sort_scratch);
     auto* items1 = items0 + N;
     auto* bounds = reinterpret_cast<int2*>(items1 + N);
     const long long nb = (long long)(R - 1) * (R - 1);
-    auto* hist = reinterpret_cast<unsigned*>(bounds + nb);
+    auto* hist = sort_hist(bounds + nb);
     const unsigned chunk_blocks = static_cast<unsigned>(std::min(chunks, kSortBlocks));
     const unsigned cell_blocks = static_cast<unsigned>(std::min<long long>((N + NT - 1) / NT, kSortBlocks));
     hipLaunchKernelGGL(k_sort_keys, dim3(chunk_blocks), dim3(NT), 0, s, items0, hist, bounds, u, v, R, P, dt0, chunks,
-                       max_bits);
+                       ipt, max_bits);
     const int bits = sort_key_bits(R);
     const GridGate gate{max_bits, dt0, R};
     unsigned long long* src = items0;
@@ -707,10 +745,10 @@ hipError_t launch_scatter_density(hipStream_t s, float* out, const float* rho0, 
     for (int shift = 0; shift < bits; shift += DB) {
         if (shift > 0)
             hipLaunchKernelGGL(k_sort_hist<GridGate>, dim3(chunk_blocks), dim3(NT), 0, s, src, N, shift, hist, chunks,
-                               gate);
+                               ipt, gate);
         hipLaunchKernelGGL(k_sort_scan<GridGate>, dim3(1), dim3(1024), 0, s, hist, ND * chunks, gate);
         hipLaunchKernelGGL(k_sort_scatter<GridGate>, dim3(chunk_blocks), dim3(NT), 0, s, src, dst, N, shift, hist,
-                           chunks, gate);
+                           chunks, ipt, gate);
         std::swap(src, dst);
     }
     hipLaunchKernelGGL(k_sort_bounds<GridGate>, dim3(cell_blocks), dim3(NT), 0, s, src, N, bounds, (unsigned)nb, gate);
@@ -721,7 +759,7 @@ hipError_t launch_scatter_density(hipStream_t s, float* out, const float* rho0, 
 
 size_t batch_scatter_bytes(long long cells, long long targets) {
     const size_t N = static_cast<size_t>(cells);
-    const size_t chunks = std::max<size_t>((N + CH - 1) / CH, 1);
+    const size_t chunks = sort_chunks(cells);
     return 2 * N * sizeof(unsigned long long) + static_cast<size_t>(targets) * sizeof(int2) +
            ND * chunks * sizeof(unsigned) + 4096;
 }
@@ -741,27 +779,27 @@ hipError_t launch_batch_scatter(hipStream_t s, const BatchScatter& B, float* out
     hipLaunchKernelGGL(k_bsort_gate, dim3(1), dim3(256), 0, s, B.flag, B.sims, B.count, max_bits);
     // sorted path (returns at once unless the gate is set)
     const long long N = B.cells;
-    const int chunks = static_cast<int>(std::max<long long>((N + CH - 1) / CH, 1));
+    const int chunks = sort_chunks(N), ipt = sort_rounds(N);
     auto* items0 = static_cast<unsigned long long*>(B.scratch);
     auto* items1 = items0 + N;
     auto* bounds = reinterpret_cast<int2*>(items1 + N);
-    auto* hist = reinterpret_cast<unsigned*>(bounds + B.targets);
+    auto* hist = sort_hist(bounds + B.targets);
     const unsigned nb = static_cast<unsigned>(B.targets);
     const unsigned chunk_blocks = static_cast<unsigned>(std::min(chunks, kSortBlocks));
     const unsigned cell_blocks = static_cast<unsigned>(std::min<long long>((N + NT - 1) / NT, kSortBlocks));
     const FlagGate gate{B.flag};
     hipLaunchKernelGGL(k_bsort_keys, dim3(chunk_blocks), dim3(NT), 0, s, items0, hist, bounds, u, v, B.sims, B.count,
-                       N, nb, chunks, max_bits, gate);
+                       N, nb, chunks, ipt, max_bits, gate);
     const int bits = key_bits(nb);
     unsigned long long* src = items0;
     unsigned long long* dst = items1;
     for (int shift = 0; shift < bits; shift += DB) {
         if (shift > 0)
             hipLaunchKernelGGL(k_sort_hist<FlagGate>, dim3(chunk_blocks), dim3(NT), 0, s, src, N, shift, hist, chunks,
-                               gate);
+                               ipt, gate);
         hipLaunchKernelGGL(k_sort_scan<FlagGate>, dim3(1), dim3(1024), 0, s, hist, ND * chunks, gate);
         hipLaunchKernelGGL(k_sort_scatter<FlagGate>, dim3(chunk_blocks), dim3(NT), 0, s, src, dst, N, shift, hist,
-                           chunks, gate);
+                           chunks, ipt, gate);
         std::swap(src, dst);
     }
     hipLaunchKernelGGL(k_sort_bounds<FlagGate>, dim3(cell_blocks), dim3(NT), 0, s, src, N, bounds, nb, gate);
