@@ -392,7 +392,9 @@ bool forms_rhs(const fs2d_handle* h) {
     return h->prm.sweep_order == FS2D_ORDER_JACOBI && h->jacobi_kernel == FS2D_JACOBI_WAVE;
 }
 
-int project(fs2d_handle* h, int K) {
+// speed: the largest speed of the result, which the next density scatter reads, is
+// wanted too (a step's first projection is followed by the velocity's advection).
+int project(fs2d_handle* h, int K, bool speed = true) {
     const Scalars s = scalars(h->R, 1.0f);
     const bool fill = K > 0 && pressure_needs_fill(h);
     JacobiFirst first;
@@ -411,8 +413,8 @@ int project(fs2d_handle* h, int K) {
     if (rc) return rc;
     h->pressure_zero = (K <= 0);
     FS2D_HIP(h, launch_gradient(h->stream, h->u(), h->v(), h->f[F_P], h->R, h->P, s.h, h->pressure_zero ? 1 : 0,
-                                h->max_bits, h->speed_slots));
-    h->speed_valid = true;
+                                speed ? h->max_bits : nullptr, h->speed_slots));
+    h->speed_valid = speed;
     return FS2D_OK;
 }
 
@@ -604,9 +606,9 @@ int step_shared_diffuse(fs2d_handle* h, float diff, float visc, float dt) {
             std::swap(h->u(), h->f[F_UN]);
             std::swap(h->v(), h->f[F_VN]);
             h->pressure_zero = false;
-            FS2D_HIP(h, launch_gradient(h->stream, h->u(), h->v(), h->f[F_P], R, P, scalars(R, 1.0f).h, 0,
-                                        h->max_bits, h->speed_slots));
-            h->speed_valid = true;
+            FS2D_HIP(h, launch_gradient(h->stream, h->u(), h->v(), h->f[F_P], R, P, scalars(R, 1.0f).h, 0, nullptr,
+                                        nullptr));
+            h->speed_valid = false;
             if ((rc = advect_velocity(h, dt))) return rc;
             // the second projection from a stored divergence: its units then
             // read one right-hand side field instead of two (faster than the
@@ -634,7 +636,7 @@ int step_shared_diffuse(fs2d_handle* h, float diff, float visc, float dt) {
     std::swap(h->u(), h->f[F_UN]);
     std::swap(h->v(), h->f[F_VN]);
     h->speed_valid = false;
-    if ((rc = project(h, Kp))) return rc;
+    if ((rc = project(h, Kp, false))) return rc;
     if ((rc = advect_velocity(h, dt))) return rc;
     return project(h, Kp);
 }
@@ -663,7 +665,7 @@ int step(fs2d_handle* h, float diff, float visc, float dt) {
     FS2D_HIP(h, launch_add_sources(h->stream, h->v(), h->f[F_X0], h->f[F_VS], R, P, dt));
     if ((rc = diffuse(h, h->v(), BND_OPP_V, visc, dt, Kd))) return rc;
     // project, self-advect, project (:25-30)
-    if ((rc = project(h, Kp))) return rc;
+    if ((rc = project(h, Kp, false))) return rc;
     if ((rc = advect_velocity(h, dt))) return rc;
     return project(h, Kp);
 }

@@ -151,7 +151,7 @@ __global__ __launch_bounds__(CBX* CBY) void kb_gradient(const BatchSim* __restri
             const size_t o = S.off;
             m = cells::gradient(r.a[A_U] + o, r.a[A_V] + o, r.a[A_P] + o, S.R, S.P, S.h, false, i, j);
         }
-        speed_to_slot(m, slots, s, blk);
+        if (slots) speed_to_slot(m, slots, s, blk);
     }
 }
 
@@ -383,13 +383,15 @@ int solve(fs2d_batch* b, int kind) {
 
 hipError_t cell_launch_check() { return hipGetLastError(); }
 
-int project(fs2d_batch* b) {
+// speed: the largest speeds of the result are wanted too.
+int project(fs2d_batch* b, bool speed) {
     const dim3 grid = cell_grid(b), blk(CBX, CBY);
     int rc = solve(b, SWEEP_PRESSURE);
     if (rc) return rc;
     hipLaunchKernelGGL(kb_gradient, grid, blk, 0, b->stream, b->sims, b->cell_work, b->cell_blocks, b->roles,
-                       b->slots);
-    hipLaunchKernelGGL(kb_fold_speed, dim3(b->count), dim3(64), 0, b->stream, b->max_bits, b->slots);
+                       speed ? b->slots : nullptr);
+    if (speed)
+        hipLaunchKernelGGL(kb_fold_speed, dim3(b->count), dim3(64), 0, b->stream, b->max_bits, b->slots);
     FS2D_BHIP(b, cell_launch_check());
     return FS2D_OK;
 }
@@ -411,13 +413,13 @@ int step(fs2d_batch* b) {
     std::swap(b->roles.a[A_RHO], b->roles.a[A_T1]);
     std::swap(b->roles.a[A_U], b->roles.a[A_UN]);
     std::swap(b->roles.a[A_V], b->roles.a[A_VN]);
-    if ((rc = project(b))) return rc;
+    if ((rc = project(b, false))) return rc;
     hipLaunchKernelGGL(kb_gather_velocity, cell_grid(b), blk, 0, b->stream, b->sims, b->cell_work, b->cell_blocks,
                        b->roles);
     FS2D_BHIP(b, cell_launch_check());
     std::swap(b->roles.a[A_U], b->roles.a[A_T1]);
     std::swap(b->roles.a[A_V], b->roles.a[A_T2]);
-    return project(b);
+    return project(b, true);
 }
 
 constexpr size_t kMaxBatchGraphs = 16;

@@ -199,7 +199,9 @@ int fs2d_hip_copy_bandwidth(long long bytes, int reps, float* gb_per_s);
 /* Number of kernel launches one step enqueues (for per-launch averages).  In
  * the Jacobi order a launch that serves density, u and v together counts as
  * three, and the sources' and divergence's passes count although a solve's first
- * launch makes them: the figure is that of one field and one stage per launch. */
+ * launch makes them; each gradient counts with a reduction of the largest speed,
+ * which a step's first does without: the figure is that of one field and one stage
+ * per launch. */
 int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches);
 
 /* ---- projection without allocation -------------------------------------
@@ -266,7 +268,7 @@ int fs2d_hip_batch_sync(fs2d_batch* b);
  * multiple of (a fixed jacobi_block, else 1: a simulation's sweeps are spread evenly
  * over its launches), tile_rows, the rows an inner Jacobi tile writes after 8 sweeps,
  * passes per step (launches, counting the sources' and the divergences' passes that
- * a solve's first launch makes), captured step graphs, total interior cells. */
+ * a solve's first launch makes, and a speed reduction for each gradient), captured step graphs, total interior cells. */
 int fs2d_hip_batch_info(fs2d_batch* b, int* jacobi_depth, int* tile_rows, int* launches_per_step, int* graphs,
                         long long* interior_cells);
 /* The persistent launches' grid: blocks per compute unit for the Jacobi launches (8
