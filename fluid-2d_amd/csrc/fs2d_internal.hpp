@@ -290,13 +290,24 @@ struct JacobiFirst {
     float scale = 0.f;
     float* b[3] = {};
 };
+// A pressure solve's last launch, if it is not its first, can subtract the pressure's
+// gradient from u and v in place (JACOBI_WAVE); done says that it has.  slots: the
+// largest speed is reduced into them (kSpeedSlots, to be folded by launch_fold_speed).
+struct JacobiLast {
+    float *u = nullptr, *v = nullptr;
+    float h = 0.f;
+    unsigned* slots = nullptr;
+    bool done = false;
+};
 hipError_t launch_jacobi_solve(hipStream_t s, const SweepSet& set, float* const* scratch, int block, int kernel,
-                               const JacobiFirst* first = nullptr);
+                               const JacobiFirst* first = nullptr, JacobiLast* last = nullptr);
+hipError_t launch_fold_speed(hipStream_t s, unsigned* max_bits, unsigned* speed_slots);
 // One launch (JACOBI_LDS: one per field) of m fused sweeps, m in 1..8, from src[f] into dst[f].
 hipError_t launch_jacobi_pass(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
-                              int zero_src, int m, int kernel, const JacobiFirst* first = nullptr);
+                              int zero_src, int m, int kernel, const JacobiFirst* first = nullptr,
+                              const JacobiLast* last = nullptr);
 hipError_t launch_jacobi_tiles(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
-                               int zero_src, int m, const JacobiFirst* first);
+                               int zero_src, int m, const JacobiFirst* first, const JacobiLast* last);
 int jacobi_launches(int K, int block);
 
 }  // namespace fs2d

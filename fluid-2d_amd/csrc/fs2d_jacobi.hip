@@ -12,6 +12,7 @@ struct TileSet {
     const float* src[3];
     float* dst[3];
     JacobiFirst first;
+    JacobiLast last;
     int m, zero, tiles_x, tiles_y;
 };
 
@@ -36,7 +37,13 @@ __global__ __launch_bounds__(64 * NW) void k_jacobi_tile(TileSet S) {
     t.s1 = S.first.s1;
     t.scale = S.first.scale;
     t.b_out = S.first.b[f];
+    t.gu = S.last.u;
+    t.gv = S.last.v;
+    t.h = S.last.h;
+    t.speed_slot = S.last.slots ? S.last.slots + (blockIdx.x % kSpeedSlots) * kSlotStride : nullptr;
+    t.m += LOAD == TILE_GRADIENT;
     tile_place(t, NW * RPW, b / S.tiles_x, b % S.tiles_x, S.tiles_y, S.tiles_x);
+    t.m = S.m;
     jacobi_tile_any<RPW, NW, KIND, LOAD>(t, ex);
 }
 
@@ -49,10 +56,12 @@ void launch_kind(hipStream_t s, const TileSet& S, dim3 grid, dim3 block) {
 template <int RPW, int NW>
 hipError_t launch(hipStream_t s, TileSet& S, int fields, int kind) {
     const int R = S.a[0].R;
-    S.tiles_y = tile_count(R, NW * RPW, S.m);
-    S.tiles_x = tile_count(R, kTileCols, S.m);
+    const int margin = S.m + (S.last.u != nullptr);
+    S.tiles_y = tile_count(R, NW * RPW, margin);
+    S.tiles_x = tile_count(R, kTileCols, margin);
     const dim3 grid(S.tiles_x * S.tiles_y, fields), block(64 * NW);
-    if (kind == TILE_PRESSURE) launch_kind<RPW, NW, TILE_PRESSURE, TILE_DIVERGENCE>(s, S, grid, block);
+    if (S.last.u) hipLaunchKernelGGL((k_jacobi_tile<RPW, NW, TILE_PRESSURE, TILE_GRADIENT>), grid, block, 0, s, S);
+    else if (kind == TILE_PRESSURE) launch_kind<RPW, NW, TILE_PRESSURE, TILE_DIVERGENCE>(s, S, grid, block);
     else if (kind == TILE_DIFFUSE_CHECKED) launch_kind<RPW, NW, TILE_DIFFUSE_CHECKED, TILE_SOURCES>(s, S, grid, block);
     else launch_kind<RPW, NW, TILE_DIFFUSE, TILE_SOURCES>(s, S, grid, block);
     return hipGetLastError();
@@ -78,7 +87,8 @@ hipError_t launch(hipStream_t s, TileSet& S, int fields, int kind) {
 static int tile_rows(long cells) { return cells < 500000 ? 32 : (cells < 8000000 ? 48 : 96); }
 
 hipError_t launch_jacobi_tiles(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
-                               int zero_src, int m, const JacobiFirst* first) {
+                               int zero_src, int m, const JacobiFirst* first, const JacobiLast* last) {
+    if (last && (first || zero_src || set.count != 1 || set.a[0].kind != SWEEP_PRESSURE)) return hipErrorInvalidValue;
     if (m < 1 || m > kTileMaxSweeps || set.count < 1 || set.count > 3) return hipErrorInvalidValue;
     TileSet S{};
     bool checked = true;
@@ -89,6 +99,7 @@ hipError_t launch_jacobi_tiles(hipStream_t s, const SweepSet& set, const float* 
         S.dst[f] = dst[f];
     }
     if (first) S.first = *first;
+    if (last) S.last = *last;
     S.m = m;
     S.zero = zero_src;
     const int kind = set.a[0].kind == SWEEP_PRESSURE ? TILE_PRESSURE : (checked ? TILE_DIFFUSE_CHECKED : TILE_DIFFUSE);

@@ -3,6 +3,7 @@
 // the diffuse division, the relaxation of one cell, and the Jacobi block tile.
 #pragma once
 
+#include "fs2d_cells.hpp"
 #include "fs2d_internal.hpp"
 
 namespace fs2d {
@@ -134,7 +135,12 @@ constexpr int kTileMaxSweeps = 8, kTileCols = 64;
 //   TILE_DIVERGENCE  b is the divergence scale (((s0E - s0W) + s1S) - s1N) of a velocity
 //                    s0, s1; the iterate starts as zero
 // A cell of the halo is formed by every tile that holds it, the same each time.
-enum TileLoad : int { TILE_STORED = 0, TILE_SOURCES = 1, TILE_DIVERGENCE = 2 };
+//   TILE_GRADIENT    stored, and after the sweeps (a pressure solve's last) the tile
+//                    subtracts the pressure's gradient from gu and gv in place, as
+//                    cells::gradient, which saves the pass that would read the pressure
+//                    back.  Tiles are placed for m + 1 sweeps then.  Never in a launch
+//                    that also reads the velocity's halo (TILE_DIVERGENCE).
+enum TileLoad : int { TILE_STORED = 0, TILE_SOURCES = 1, TILE_DIVERGENCE = 2, TILE_GRADIENT = 3 };
 
 struct TileJob {
     const float *src, *b;
@@ -142,6 +148,9 @@ struct TileJob {
     const float *s0, *s1;  // TILE_SOURCES, TILE_DIVERGENCE
     float scale;
     float* b_out;
+    float *gu, *gv;        // TILE_GRADIENT
+    float h;
+    unsigned* speed_slot;  // takes the largest speed of the result if not null (cells::fold_speed)
     int R, P, m;
     bool zero;  // the iterate starts as zero (src is not read)
     float a;
@@ -200,7 +209,7 @@ __device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict_
     const int R = t.R, P = t.P, n = R - 2, i0 = t.gi0 + wave * RPW, gj = t.gj0 + lane;
     const int cj = min(gj, R - 1);  // a grid narrower than the region
     float X[RPW + 1], B[RPW];
-    if constexpr (LOAD == TILE_STORED) {
+    if constexpr (LOAD == TILE_STORED || LOAD == TILE_GRADIENT) {
 #pragma unroll
         for (int r = 0; r < RPW; ++r) X[r + 1] = t.zero ? 0.f : t.src[(size_t)min(i0 + r, R - 1) * P + cj];
 #pragma unroll
@@ -296,6 +305,44 @@ __device__ __forceinline__ void jacobi_tile(const TileJob& t, float* __restrict_
         down(s);
 #pragma unroll
         for (int r = RPW - 1; r >= 0; --r) X[r + 1] = X[r];
+    }
+
+    if constexpr (LOAD == TILE_GRADIENT) {
+        float above, below, speed = 0.f;
+        exchange(t.m, X[1], X[RPW], above, below);
+        const bool own = gj >= t.jlo && gj <= t.jhi;
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+            const int gi = i0 + r;
+            if (gi < t.ilo || gi > t.ihi) continue;  // the same in all lanes
+            const float c = X[r + 1];
+            float pn = r > 0 ? X[r] : above, ps = r + 1 < RPW ? X[r + 2 <= RPW ? r + 2 : RPW] : below;
+            float pw = lane_west(c), pe = lane_east(c);
+            if (ROWS) {  // the pressure's ring continues it
+                pn = gi == 1 ? c : pn;
+                ps = gi == n ? c : ps;
+            }
+            if (COLS) {
+                pw = gj == 1 ? c : pw;
+                pe = gj == n ? c : pe;
+            }
+            if (own) {
+                const size_t g = (size_t)gi * P + gj;
+                const float un = t.gu[g] - 0.5f * (pe - pw) / t.h;
+                const float vn = t.gv[g] - 0.5f * (ps - pn) / t.h;
+                t.gu[g] = un;
+                t.gv[g] = vn;
+                if (ROWS || COLS) {
+                    cells::write_ring(t.gu, gi, gj, un, R, P, Ring{false, true});
+                    cells::write_ring(t.gv, gi, gj, vn, R, P, Ring{true, false});
+                }
+                speed = cells::fold_speed(speed, un, vn);
+            }
+        }
+        if (t.speed_slot) {
+            for (int off = 32; off > 0; off >>= 1) speed = fmaxf(speed, __shfl_xor(speed, off));
+            if (lane == 0) atomicMax(t.speed_slot, __float_as_uint(speed));
+        }
     }
 
     if (gj < t.jlo || gj > t.jhi) return;

@@ -296,7 +296,11 @@ hipError_t launch_gradient(hipStream_t s, float* u, float* v, const float* p, in
                            int p_is_zero, unsigned* max_bits, unsigned* speed_slots) {
     hipLaunchKernelGGL(k_gradient, dim3((R + 1023) / 1024, R - 2), dim3(256), 0, s, u, v, p, R, P, h, p_is_zero,
                        max_bits ? speed_slots : nullptr);
-    if (max_bits) hipLaunchKernelGGL(k_fold_speed, dim3(1), dim3(kSpeedSlots), 0, s, max_bits, speed_slots);
+    return max_bits ? launch_fold_speed(s, max_bits, speed_slots) : hipGetLastError();
+}
+
+hipError_t launch_fold_speed(hipStream_t s, unsigned* max_bits, unsigned* speed_slots) {
+    hipLaunchKernelGGL(k_fold_speed, dim3(1), dim3(kSpeedSlots), 0, s, max_bits, speed_slots);
     return hipGetLastError();
 }
 

@@ -1339,9 +1339,10 @@ hipError_t launch_gs_solve(hipStream_t s, const GsPlan& plan, const SweepArgs& a
 int jacobi_launches(int K, int block) { return (K + block - 1) / block; }
 
 hipError_t launch_jacobi_pass(hipStream_t s, const SweepSet& set, const float* const* src, float* const* dst,
-                              int zero_src, int m, int kernel, const JacobiFirst* first) {
-    if (kernel != JACOBI_LDS) return launch_jacobi_tiles(s, set, src, dst, zero_src, m, first);
-    if (first) return hipErrorInvalidValue;
+                              int zero_src, int m, int kernel, const JacobiFirst* first,
+                              const JacobiLast* last) {
+    if (kernel != JACOBI_LDS) return launch_jacobi_tiles(s, set, src, dst, zero_src, m, first, last);
+    if (first || last) return hipErrorInvalidValue;
     for (int f = 0; f < set.count; ++f) {
         const hipError_t e = launch_jacobi_block(s, set.a[f], src[f], dst[f], zero_src, m);
         if (e != hipSuccess) return e;
@@ -1350,7 +1351,7 @@ hipError_t launch_jacobi_pass(hipStream_t s, const SweepSet& set, const float* c
 }
 
 hipError_t launch_jacobi_solve(hipStream_t s, const SweepSet& set, float* const* scratch, int block, int kernel,
-                               const JacobiFirst* first) {
+                               const JacobiFirst* first, JacobiLast* last) {
     // Sweep order: x -> scratch -> x -> ...; an odd launch count ends in
     // scratch, and the caller swaps the two buffers.
     const float* src[SweepSet::kMax];
@@ -1363,8 +1364,11 @@ hipError_t launch_jacobi_solve(hipStream_t s, const SweepSet& set, float* const*
     bool zero = set.a[0].zero_start != 0;
     while (done < set.a[0].K) {
         const int m = std::min(block, set.a[0].K - done);
-        hipError_t e = launch_jacobi_pass(s, set, src, dst, zero ? 1 : 0, m, kernel, done == 0 ? first : nullptr);
+        const bool ends = last && done > 0 && done + m == set.a[0].K;
+        hipError_t e = launch_jacobi_pass(s, set, src, dst, zero ? 1 : 0, m, kernel, done == 0 ? first : nullptr,
+                                          ends ? last : nullptr);
         if (e != hipSuccess) return e;
+        if (ends) last->done = true;
         zero = false;
         done += m;
         for (int f = 0; f < set.count; ++f) {

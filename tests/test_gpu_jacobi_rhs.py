@@ -1,6 +1,7 @@
 """Jacobi solves whose first launch forms the right-hand sides (the source terms, the
-divergence), against the oracle, bit for bit: one launch a solve (the result is in the
-scratch field) and several, sizes at the tiles' edges, source rings that must not be
+divergence) and whose last one subtracts the gradient, against the oracle, bit for bit: one launch a solve (the result is in the
+scratch field, the gradient a pass of its own) and several, sizes at the tiles' edges
+and at both sides of where the gradient's place changes, source rings that must not be
 read, and no sweeps at all (the separate passes).
 """
 from __future__ import annotations
@@ -14,8 +15,11 @@ import oracle
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("R", [3, 4, 32, 33, 48, 63, 64, 65, 97, 128, 129, 410, 1640])
-@pytest.mark.parametrize("kd,kp", [(1, 1), (8, 3), (9, 17), (0, 5), (5, 0)])
+SIZES = [3, 4, 32, 33, 48, 63, 64, 65, 97, 128, 129, 410, 1640]
+SWEEPS = [(1, 1), (8, 3), (9, 17), (0, 5), (5, 0)]
+
+
+@pytest.mark.parametrize("R,kd,kp", [(R, *k) for R in SIZES for k in SWEEPS] + [(3162, 1, 9), (3163, 1, 9)])
 def test_step(R, kd, kp, oracle_lib):
     rng = np.random.default_rng(1000 * R + 10 * kd + kp)
     x = rng.standard_normal((6, R, R), dtype=np.float32) * np.float32(0.02)
