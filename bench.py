@@ -133,7 +133,7 @@ def solve_roofline(order: int, n: int, K: int, ms: float, kind: str, fields: int
     elif order == 0:
         name = f"k_gs_unit<{policy['tile_cols']},{policy['sweeps_per_unit']},{policy['lag']},{kind}>"
     else:
-        name = f"k_jacobi_wave ({kind})"
+        name = f"k_jacobi_tile ({kind})"
     r = {"kernel": name, "bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
          "frac": round(gbs / HBM_PEAK_GBS, 4) if gbs <= HBM_PEAK_GBS else None,
          "traffic": int(traffic) if traffic else None,

@@ -165,7 +165,10 @@ __global__ __launch_bounds__(CBX* CBY) void kb_gradient(const BatchSim* __restri
 // launch's time.  256 simulations of sides 64 to 512 (19.3 M cells, 20 or 40 sweeps),
 // one step's diffuse solves / one pressure solve: one wave per 16-row tile, 4 sweeps
 // a launch 1.50 / 0.45 ms; block tiles of 48 rows, at most 8 sweeps a launch 1.41 /
-// 0.40 ms; of 96 rows 1.21 / 0.38 ms.
+// 0.40 ms; of 96 rows 1.21 / 0.38 ms; with known ring rows and lanes, and the right-hand
+// sides formed by the first launches, 1.12 / 0.33 ms (the sources' pass of 0.25 ms and a
+// divergence's 0.06 ms are in these and were not before).  The gradient stays a pass:
+// made by the last launch, 40 steps and their read-back took 106.0 ms against 101.9.
 constexpr int JB_WAVES = 8;
 
 // A solve's first launch (FIRST, j = 0) forms its right-hand sides: the sources' terms

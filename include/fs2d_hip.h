@@ -77,7 +77,7 @@ typedef struct fs2d_params {
                               * on the first solve, by timing the candidates (64/128 columns, 4/8
                               * sweeps, lag 4/8) on scratch fields; cached per process.  All choices
                               * give identical results.                                             */
-    int jacobi_kernel;       /* enum fs2d_jacobi_kernel; 0 = default (register strips)                   */
+    int jacobi_kernel;       /* enum fs2d_jacobi_kernel; 0 = default (block tiles in registers)          */
     int launch_mode;         /* enum fs2d_launch_mode; 0 = graph replay                                  */
 } fs2d_params;
 
