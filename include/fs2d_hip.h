@@ -200,7 +200,8 @@ int fs2d_hip_copy_bandwidth(long long bytes, int reps, float* gb_per_s);
  * the Jacobi order a launch that serves density, u and v together counts as
  * three, and the sources' and divergence's passes count although a solve's first
  * launch makes them; each gradient counts with a reduction of the largest speed,
- * which a step's first does without: the figure is that of one field and one stage
+ * which a step's first does without, each sort pass of the density scatter with its scan:
+ * the figure is that of one field and one stage
  * per launch. */
 int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches);
 
