@@ -82,6 +82,8 @@ hipError_t launch(hipStream_t s, TileSet& S, int fields, int kind) {
 // sweeps, so taller is better until too few blocks are left.  At 4098 x 4098 the
 // three fields' launch issues 7.6 VALU operations a cell-sweep (138 us at the halo's
 // 0.62) and moves 0.75 GB (150 us of a copy's rate): both at once take 176.
+// (These were taken before tiles at the grid's edge knew their ring rows and lanes,
+// which took 3 % off a step at 4098 and at 203 and moves no line.)
 // Two or four columns a lane (less halo) measured slower at every size: 184 and
 // 183 us here, 25 and 31 against 19 us at 1026.
 static int tile_rows(long cells) { return cells < 500000 ? 32 : (cells < 8000000 ? 48 : 96); }

@@ -14,9 +14,9 @@
 //    destination adds the shares of a source row in column order to
 //    accumulators for the 2W + 1 rows it reaches.
 //  * W > kWindow: the sources are sorted by target cell with a stable LSD
-//    radix sort of 9-bit digits (k_sort_keys, k_sort_hist, k_sort_scan on
-//    large grids, k_sort_scatter), so each target's sources stay in row-major order; each
-//    destination then merges, in source order, the four target cells whose
+//    radix sort of 9-bit digits (k_sort_keys, k_sort_hist, k_sort_scan on large
+//    grids, k_sort_scatter), so each target's sources stay in row-major order;
+//    each destination then merges, in source order, the four target cells whose
 //    shares reach it (k_sort_bounds, k_scatter_merge).  Work is O(R^2)
 //    whatever the speeds.
 //

@@ -196,13 +196,12 @@ int fs2d_division_plan(float denom, float* inv, float* inv_lo, float* two_hi, fl
  * counted), timed with HIP events over `reps` copies; the achievable HBM
  * figure beside the 8 TB/s peak. */
 int fs2d_hip_copy_bandwidth(long long bytes, int reps, float* gb_per_s);
-/* Number of kernel launches one step enqueues (for per-launch averages).  In
- * the Jacobi order a launch that serves density, u and v together counts as
- * three, and the sources' and divergence's passes count although a solve's first
- * launch makes them; each gradient counts with a reduction of the largest speed,
- * which a step's first does without, each sort pass of the density scatter with its scan:
- * the figure is that of one field and one stage
- * per launch. */
+/* Number of kernel passes of one step (for per-launch averages): one field, one
+ * stage and one sort pass a launch.  Where a launch serves more it counts as often:
+ * the Jacobi order's density, u and v together as three, the sources' and the
+ * divergence's passes although a solve's first launch makes them, a gradient with a
+ * reduction of the largest speed, which a step's first does without, and a sort pass
+ * of the density scatter with its scan. */
 int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches);
 
 /* ---- projection without allocation -------------------------------------
