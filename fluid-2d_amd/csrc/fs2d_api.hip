@@ -1344,7 +1344,7 @@ int fs2d_division_plan(float denom, float* inv, float* inv_lo, float* two_hi, fl
     *inv_lo = A.inv_denom_lo;
     *two_hi = A.inv_hi2;
     *two_lo = A.inv_lo2;
-    *lo = A.div_lo;
+    *lo = A.div_checked ? A.div_lo2 : A.div_lo;
     *checked = A.div_checked;
     return FS2D_OK;
 }

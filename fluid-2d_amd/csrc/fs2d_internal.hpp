@@ -57,6 +57,7 @@ struct SweepArgs {
     float inv_denom_lo;  // RN(1 / denom - inv_denom)
     int div_checked;     // the two-product quotient is exact for this divisor (two_product_quotient)
     float inv_hi2, inv_lo2;  // its pair: inv_hi2 <= 1 / denom, inv_lo2 = RN(1 / denom - inv_hi2) > 0
+    float div_lo2;           // smallest |dividend| it takes; div_lo stays the corrected quotient's own
 };
 
 // Lower end of the dividends the FMA-corrected division handles (zero aside):
@@ -83,7 +84,7 @@ inline SweepArgs sweep_args(float* x, const float* b, int R, int P, int kind, fl
 // Whether q = RN(x y2 + RN(x y2_lo)) equals RN(x / d) for every finite
 // dividend from the division floor up, with y2 the largest float <= 1/d and
 // y2_lo = RN(1/d - y2) > 0; if so, sets A.div_checked, A.inv_hi2 and
-// A.inv_lo2, and raises A.div_lo to where RN(x y2_lo) stays normal.  The tail
+// A.inv_lo2, and A.div_lo2 to where RN(x y2_lo) stays normal.  The tail
 // being positive, +-inf dividends come out +-inf as well.  Decided from the few
 // significands of one binade whose quotients lie next to a midpoint of two floats
 // (the quotients of the other binades are exact power-of-two scalings of those).
@@ -93,7 +94,7 @@ void two_product_quotient(SweepArgs& A);
 // two_product_quotient, and for a power of two (d = 1 when a = 0) the pair (1 / d,
 // 2^-149): x / d is then x y2 rounded once, and the tail, too small to change a
 // finite quotient, keeps infinite dividends infinite, so the quotient is exact for
-// every dividend and div_lo is 0.  What the kernels' launchers use.
+// every dividend and div_lo2 is 0.  What the kernels' launchers use.
 void known_quotient(SweepArgs& A);
 
 // Up to three independent solves with the same sweep count, relaxed by the

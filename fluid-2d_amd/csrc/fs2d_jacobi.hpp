@@ -13,15 +13,17 @@ __device__ __forceinline__ float sgn(bool neg, float x) { return neg ? -x : x; }
 
 // The divisor of a diffuse solve: d = 1 + 4a, y = RN(1/d), y_lo = RN(1/d - y)
 // (so y + y_lo is 1/d to about 2^-48), and lo, the smallest nonzero
-// |dividend| the FMA-based quotients take (the host's division_floor:
-// max(2^-100, d 2^-124), or +inf when d > 2^100; raised where the two-product
-// quotient is in use, see two_product_quotient).
+// |dividend| the corrected quotient takes (the host's division_floor:
+// max(2^-100, d 2^-124), or +inf when d > 2^100).  y2, y2_lo and lo2 are the same
+// of the checked quotient (known_quotient): lo2 is 0 for a power of two, whose pair
+// is exact for every dividend, but Markstein's step turns -0 into +0, so a field
+// with such a divisor that shares a launch with an unchecked one needs its own lo.
 struct Divisor {
-    float d, y, lo, y_lo, y2, y2_lo;
+    float d, y, lo, y_lo, y2, y2_lo, lo2;
 };
 
 __host__ __device__ __forceinline__ Divisor divisor_of(const SweepArgs& A) {
-    return Divisor{A.denom, A.inv_denom, A.div_lo, A.inv_denom_lo, A.inv_hi2, A.inv_lo2};
+    return Divisor{A.denom, A.inv_denom, A.div_lo, A.inv_denom_lo, A.inv_hi2, A.inv_lo2, A.div_lo2};
 }
 
 // Dividends outside [lo, 2^100] (zero, tiny, huge, inf, NaN) take the IEEE
@@ -46,15 +48,15 @@ __device__ __forceinline__ float div_rn(float x, Divisor v) {
 }
 
 // x / d for a divisor whose two-product quotient RN(x y2 + RN(x y2_lo)) the
-// host has checked to be correctly rounded for every finite dividend from lo
+// host has checked to be correctly rounded for every finite dividend from lo2
 // up (Brisebarre, Muller and Raina, "Accelerating correctly rounded
 // floating-point division when the divisor is known in advance", IEEE Trans.
 // Computers 53(8), 2004; the check is two_product_quotient).  With y2_lo > 0
 // an infinite dividend gives the infinity IEEE division gives, so one test,
-// |x| >= lo (false for zero, tiny, subnormal and NaN), guards it.
+// |x| >= lo2 (false for tiny, subnormal and NaN), guards it.
 __device__ __forceinline__ float div_rn_checked(float x, Divisor v) {
     float q = __builtin_fmaf(x, v.y2, x * v.y2_lo);
-    const bool out = !(fabsf(x) >= v.lo);
+    const bool out = !(fabsf(x) >= v.lo2);
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(out) != 0, 0)) q = out ? x / v.d : q;
     return q;
 }
@@ -87,7 +89,7 @@ __device__ __forceinline__ float relax_fast(float b, float n, float s, float w, 
     if (KIND == SWEEP_DIFFUSE) {
         const float x = b + a * (((n + s) + w) + e);
         if (CHECKED) {
-            bad |= __builtin_amdgcn_ballot_w64(!(fabsf(x) >= dv.lo));
+            bad |= __builtin_amdgcn_ballot_w64(!(fabsf(x) >= dv.lo2));
             return __builtin_fmaf(x, dv.y2, x * dv.y2_lo);
         }
         const float ax = fabsf(x);
@@ -188,7 +190,7 @@ __device__ __forceinline__ float relax_tile(float b, float n, float s, float w, 
     const float x = b + a * (((n + s) + w) + e);
     if constexpr (KIND == TILE_DIFFUSE) return div_rn(x, dv);
     float q = __builtin_fmaf(x, dv.y2, x * dv.y2_lo);
-    const bool low = !(fabsf(x) >= dv.lo);
+    const bool low = !(fabsf(x) >= dv.lo2);
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(low) != 0, 0)) {
         const bool bad = low && x != 0.f;
         if (__builtin_amdgcn_ballot_w64(bad) != 0) q = bad ? x / dv.d : q;

@@ -1052,7 +1052,7 @@ void two_product_quotient(SweepArgs& A) {
     const int E = std::max(0, std::ilogb(tf) + 1);
     if (two_product_exact(d, y, yl, E)) {
         A.div_checked = 1;
-        A.div_lo = lo;
+        A.div_lo2 = lo;
         A.inv_hi2 = y;
         A.inv_lo2 = yl;
     }
@@ -1064,7 +1064,7 @@ void known_quotient(SweepArgs& A) {
     int e = 0;
     if (!(A.denom >= 1.f && A.denom <= 0x1p100f) || std::frexp(A.denom, &e) != 0.5f) return;
     A.div_checked = 1;
-    A.div_lo = 0.f;
+    A.div_lo2 = 0.f;
     A.inv_hi2 = 1.0f / A.denom;
     A.inv_lo2 = 0x1p-149f;
 }
