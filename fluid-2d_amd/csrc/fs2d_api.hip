@@ -943,7 +943,7 @@ static int fs2d_hip_upload_device_impl(fs2d_handle* h, const float* rho, const f
     c.add(u, h->u());
     c.add(v, h->v());
     h->speed_valid = false;
-    FS2D_HIP(h, launch_copy_rows(h->stream, c, h->R, h->R, h->P));
+    FS2D_HIP(h, copy_rows_in_order(h->stream, c, h->R, h->P, true));
     return FS2D_OK;
 }
 
@@ -1022,7 +1022,7 @@ static int fs2d_hip_download_device_impl(fs2d_handle* h, float* rho, float* u, f
     if (rho) c.add(h->rho(), rho);
     if (u) c.add(h->u(), u);
     if (v) c.add(h->v(), v);
-    FS2D_HIP(h, copy_rows_in_order(h->stream, c, h->R, h->P, h->R));
+    FS2D_HIP(h, copy_rows_in_order(h->stream, c, h->R, h->P, false));
     return FS2D_OK;
 }
 

@@ -177,10 +177,9 @@ hipError_t launch_set_boundary(hipStream_t s, float* x, int R, int P, Ring ring)
 hipError_t launch_copy4(hipStream_t s, float4* dst, const float4* src, size_t n4);
 hipError_t launch_fill(hipStream_t s, void* p, uint32_t value, size_t n_words);
 
-// Rows of unpadded R x R arrays and of pitched fields (fs2d_transfer.hip):
-// `count` copies of R rows of R floats, source pitch sp, destination pitch dp
-// (floats), in one launch; copy_rows_in_order splits it where destinations
-// overlap.
+// Rows between callers' unpadded R x R device arrays and pitched fields
+// (fs2d_transfer.hip): `count` copies of R rows of R floats into fields of pitch P
+// (`in`) or out of them, a later one winning where destinations overlap.
 struct RowCopies {
     static constexpr int kMax = 6;
     const float* src[kMax] = {};
@@ -191,8 +190,7 @@ struct RowCopies {
         dst[count++] = d;
     }
 };
-hipError_t launch_copy_rows(hipStream_t s, const RowCopies& c, int R, int sp, int dp);
-hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int sp, int dp);
+hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int P, bool in);
 // Host arrays (src, unpadded) into fields (dst, pitch P), and fields (src) out
 // to host arrays (dst).  The buffers are grown on demand and belong to one
 // stream.  stage_in enqueues: the stream is synchronised before the next use of

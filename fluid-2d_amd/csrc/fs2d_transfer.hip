@@ -16,6 +16,12 @@
 //     device buffer of one array.  The two ways cost the same at about 4 MB
 //     an array; the line lies below that, at 8 MB a call, which also bounds
 //     what a handle pins.
+// A caller's pointer is dereferenced here, by the host or a kernel, only where that
+// is known to be good: pageable memory by the host, and an array that lies whole in
+// an allocation of the stream's own device by a kernel.  Any other (pinned or managed
+// memory, another device's, a device array given as a host one, one that its allocation
+// is too short for) is left to hipMemcpy2DAsync, which orders it on the stream, reaches
+// peers, and refuses what it cannot copy.
 #include "fs2d_internal.hpp"
 
 #include <cstring>
@@ -48,6 +54,58 @@ struct OnDeviceOf {
     }
 };
 
+// Whether the runtime has p: device, pinned or managed memory.
+bool registered(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
+// Whether [p, p + bytes) lies in one allocation of the stream's device.
+bool on_device_of(hipStream_t s, const void* p, size_t bytes) {
+    hipPointerAttribute_t a{};
+    hipDevice_t dev = 0;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipStreamGetDevice(s, &dev) != hipSuccess ||
+        a.type != hipMemoryTypeDevice || a.device != dev ||
+        hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t at = static_cast<const char*>(p) - static_cast<const char*>(base);
+    return at <= size && bytes <= size - at;
+}
+
+hipError_t pitched_copy(hipStream_t s, const RowCopies& c, int k, int R, int sp, int dp, hipMemcpyKind kind) {
+    const size_t f = sizeof(float);
+    return hipMemcpy2DAsync(c.dst[k], f * dp, c.src[k], f * sp, f * R, R, kind, s);
+}
+
+hipError_t launch_copy_rows(hipStream_t s, const RowCopies& c, int R, int sp, int dp) {
+    if (c.count <= 0) return hipSuccess;
+    const dim3 grid((R + 255) / 256, R, c.count);
+    hipLaunchKernelGGL(k_copy_rows, grid, dim3(256), 0, s, c, R, sp, dp);
+    return hipGetLastError();
+}
+
+// Arrays of host memory: those that the runtime has are copied by it (at once: a later
+// array wins where two overlap, and host arrays follow), the others are left in `rest`.
+hipError_t copy_registered(hipStream_t s, const RowCopies& c, int R, int sp, int dp, hipMemcpyKind kind, RowCopies* rest) {
+    for (int k = 0; k < c.count; ++k) {
+        if (registered(kind == hipMemcpyHostToDevice ? c.src[k] : c.dst[k])) {
+            const hipError_t e = pitched_copy(s, c, k, R, sp, dp, kind);
+            if (e != hipSuccess) return e;
+        } else {
+            rest->add(c.src[k], c.dst[k]);
+        }
+    }
+    return hipSuccess;
+}
+
 hipError_t grow(float** p, size_t* have, size_t floats, hipStream_t s, bool pinned) {
     if (*have >= floats) return hipSuccess;
     hipError_t e = hipStreamSynchronize(s);  // the old buffer may be in use
@@ -65,35 +123,38 @@ hipError_t grow(float** p, size_t* have, size_t floats, hipStream_t s, bool pinn
 
 }  // namespace
 
-hipError_t launch_copy_rows(hipStream_t s, const RowCopies& c, int R, int sp, int dp) {
-    if (c.count <= 0) return hipSuccess;
-    const OnDeviceOf device(s);
-    const dim3 grid((R + 255) / 256, R, c.count);
-    hipLaunchKernelGGL(k_copy_rows, grid, dim3(256), 0, s, c, R, sp, dp);
-    return hipGetLastError();
-}
-
 // A later array wins where two destinations overlap, as with copies made one
-// after the other: such a set is copied by one launch per array.
-hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int sp, int dp) {
+// after the other: such a set is copied array by array.
+hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int P, bool in) {
+    const int sp = in ? R : P, dp = in ? P : R;
+    const OnDeviceOf device(s);
     const size_t span = (size_t)(R - 1) * dp + R;
+    const size_t bytes = sizeof(float) * R * R;  // of a caller's array
     bool apart = true;
     for (int a = 0; a < c.count; ++a)
         for (int b = 0; b < a; ++b) apart = apart && (c.dst[a] + span <= c.dst[b] || c.dst[b] + span <= c.dst[a]);
-    if (apart) return launch_copy_rows(s, c, R, sp, dp);
+    RowCopies together;
+    hipError_t e;
     for (int a = 0; a < c.count; ++a) {
         RowCopies one;
         one.add(c.src[a], c.dst[a]);
-        const hipError_t e = launch_copy_rows(s, one, R, sp, dp);
+        if (!on_device_of(s, in ? c.src[a] : c.dst[a], bytes)) e = pitched_copy(s, c, a, R, sp, dp, hipMemcpyDeviceToDevice);
+        else if (!apart) e = launch_copy_rows(s, one, R, sp, dp);
+        else {
+            together.add(c.src[a], c.dst[a]);
+            e = hipSuccess;
+        }
         if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    return launch_copy_rows(s, together, R, sp, dp);
 }
 
-hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P) {
+hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& all, int R, int P) {
     const OnDeviceOf device(s);
     const size_t n = (size_t)R * R, bytes = n * sizeof(float);
-    hipError_t e;
+    RowCopies c;
+    hipError_t e = copy_registered(s, all, R, R, P, hipMemcpyHostToDevice, &c);
+    if (e != hipSuccess || c.count == 0) return e;
     if (c.count * bytes <= kPinnedStage) {
         if ((e = grow(&h.pin, &h.pin_floats, c.count * n, s, true)) != hipSuccess) return e;
         RowCopies d = c;
@@ -113,10 +174,13 @@ hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& c, int R, int 
     return hipSuccess;
 }
 
-hipError_t stage_out(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P) {
+hipError_t stage_out(HostStage& h, hipStream_t s, const RowCopies& all, int R, int P) {
     const OnDeviceOf device(s);
     const size_t n = (size_t)R * R, bytes = n * sizeof(float);
-    hipError_t e;
+    RowCopies c;
+    hipError_t e = copy_registered(s, all, R, P, R, hipMemcpyDeviceToHost, &c);
+    if (e != hipSuccess) return e;
+    if (c.count == 0) return hipStreamSynchronize(s);
     if (c.count * bytes <= kPinnedStage) {
         if ((e = grow(&h.pin, &h.pin_floats, c.count * n, s, true)) != hipSuccess) return e;
         RowCopies d = c;
