@@ -393,7 +393,7 @@ int load_samples(fs2d_net* net, Acts& a, const float* d, const float* prev, cons
     const size_t bytes = sizeof(float) * npix;
     NHIP(net, hipMemcpyAsync(dd, d, bytes, hipMemcpyHostToDevice, net->stream));
     NHIP(net, hipMemcpyAsync(a.f("prev"), prev, bytes, hipMemcpyHostToDevice, net->stream));
-    hipLaunchKernelGGL(k_sumsq_samples, dim3(G, a.N), dim3(256), 0, net->stream, dd, a.f("prev"), hw, sums);
+    hipLaunchKernelGGL(k_sumsq_samples, dim3(a.N, G), dim3(256), 0, net->stream, dd, a.f("prev"), hw, sums);
     hipLaunchKernelGGL(k_scale_samples, dim3(a.N), dim3(64), 0, net->stream, sums, G, hw, a.f("scale"), a.f("inv"));
     if (target) NHIP(net, hipMemcpyAsync(a.f("tgt"), target, bytes, hipMemcpyHostToDevice, net->stream));
     hipLaunchKernelGGL(k_pack_samples, dim3(blocks_for(npix)), dim3(256), 0, net->stream, dd, a.f("prev"),

@@ -653,13 +653,13 @@ __global__ __launch_bounds__(1024) void k_reduce_adam(LayerSpans<NL> S, const fl
 }
 
 // Host samples on the device: sums of squares of prev and d, per sample, in
-// FP64 (blocks (G, N): partial sums [n][G][2]) ...
+// FP64 (blocks (N, G), as N may pass the grid's second dimension: partial sums [n][G][2]) ...
 __global__ __launch_bounds__(256) void k_sumsq_samples(const float* __restrict__ d, const float* __restrict__ prev,
                                                       long hw, double* __restrict__ part) {
-    const float4_t* a = reinterpret_cast<const float4_t*>(d + blockIdx.y * hw);
-    const float4_t* b = reinterpret_cast<const float4_t*>(prev + blockIdx.y * hw);
+    const float4_t* a = reinterpret_cast<const float4_t*>(d + blockIdx.x * hw);
+    const float4_t* b = reinterpret_cast<const float4_t*>(prev + blockIdx.x * hw);
     double sd = 0, sp = 0;
-    for (long t = static_cast<long>(blockIdx.x) * 256 + threadIdx.x; t < hw / 4; t += static_cast<long>(gridDim.x) * 256) {
+    for (long t = static_cast<long>(blockIdx.y) * 256 + threadIdx.x; t < hw / 4; t += static_cast<long>(gridDim.y) * 256) {
         const float4_t x = a[t], y = b[t];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -678,7 +678,7 @@ __global__ __launch_bounds__(256) void k_sumsq_samples(const float* __restrict__
     }
     __syncthreads();
     if (threadIdx.x < 2)
-        part[(static_cast<long>(blockIdx.y) * gridDim.x + blockIdx.x) * 2 + threadIdx.x] =
+        part[(static_cast<long>(blockIdx.x) * gridDim.y + blockIdx.y) * 2 + threadIdx.x] =
             (w[threadIdx.x][0] + w[threadIdx.x][1]) + (w[threadIdx.x][2] + w[threadIdx.x][3]);
 }
 
