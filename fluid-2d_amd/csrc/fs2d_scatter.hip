@@ -112,23 +112,48 @@ __device__ __forceinline__ Shares shift_shares(const Shares& x) {
 }
 
 // Layout of one launch for radius W: strips of 64 - 2W destination columns,
-// bands of `band` rows, one wave per (band, strip); `band` is the smallest
-// (at least kMinBand) that keeps every wave resident at once (`slots` waves).
-// A wave is a chain of band + 2W rows, so a grid that leaves the chip idle takes
-// short bands although neighbours then read more rows twice: at 200 x 200, 12.3 us with
-// bands of 16 rows and 6.0 with 4; from about 2500 x 2500 up the bands are as before.
-constexpr int kMinBand = 4;
+// bands of `band` rows (window_band_rows), one wave per (band, strip).
 struct WindowLayout {
     int strips, band, waves;
 };
-__host__ __device__ inline WindowLayout window_layout(int R, int W, int slots) {
+__host__ __device__ inline WindowLayout window_layout(int R, int W, int band) {
     const int n = R - 2, sw = 64 - 2 * W;
     const int strips = (n + sw - 1) / sw;
-    const int maxb = slots / strips > 1 ? slots / strips : 1;
-    int band = (n + maxb - 1) / maxb;
-    band = band < kMinBand ? kMinBand : band;
-    band = band > n ? n : band;
     return WindowLayout{strips, band, strips * ((n + band - 1) / band)};
+}
+
+// The band of every radius, W - 1 first.
+struct WindowBands {
+    int rows[kWindow];
+};
+
+// Rows of a band for radius W: at least enough to keep every wave resident at once
+// (`slots` waves).  A wave is a chain of band + 2W rows, so a grid that leaves the chip
+// idle takes short bands although neighbours then read more rows twice: radius 1 at
+// 200 x 200, 12.3 us with bands of 16 rows and 6.0 with 4.  Two waves on a SIMD cost
+// radius 3 and 4 no more than one (a row of radius 4 is 1.8 us of latency and 0.9 of
+// issue), more share its issue, and 2W rows of each are read twice, so there the time
+// goes as (band + 2W) max(2, waves per SIMD).  A whole advection with bands of 4, 16 and
+// by this rule, us: radius 4 at 514 44 / 63 / 44, 1026 71 / 69 / 57, 1280 98 / 71 / 69,
+// 2050 135 / 130 / 125; radius 3 at 1280 67 / 54 / 53.  Radius 1 and 2 take 4 rows
+// everywhere (16 is never faster by more than a run differs from the next).
+constexpr int kMinBand = 4, kMaxBand = 16;
+inline int window_band_rows(int R, int W, int slots, int simds) {
+    const int n = R - 2, strips = window_layout(R, W, n).strips;
+    const int most = std::max(slots / strips, 1), least = std::max((n + most - 1) / most, kMinBand);
+    int band = least;
+    if (W > 2) {
+        long best = 0;
+        for (int b = least; b <= std::max(least, kMaxBand); b += 2) {
+            const int share = (window_layout(R, W, b).waves + simds - 1) / simds;
+            const long cost = (long)(b + 2 * W) * std::max(share, 2);
+            if (b == least || cost < best) {
+                best = cost;
+                band = b;
+            }
+        }
+    }
+    return std::min(band, n);
 }
 
 struct Row {
@@ -257,16 +282,21 @@ __device__ __forceinline__ void window_band(float* __restrict__ out, const float
 }
 
 // One wave per (band, strip), strip fastest; a block holds kStripWaves
-// consecutive waves, and block b runs block-item (b mod 8) * per + b / 8, so
-// each XCD (blocks are dealt to the 8 XCDs in turn) walks a contiguous run of
-// strips and bands and shares their overlapping lines in its L2.
+// consecutive waves, and block b runs block-item (b mod 8) * per + b / 8 of the
+// 8 per that the radius takes, so each XCD (blocks are dealt to the 8 XCDs in turn)
+// walks a contiguous run of strips and bands and shares their overlapping lines in its
+// L2.  (The grid is sized for the radius with the most waves; a per of the grid's
+// would leave whole XCDs idle for the others.)
 __global__ __launch_bounds__(NT, 6) void k_scatter_window(float* __restrict__ out, const float* __restrict__ rho0,
                                                           const float* __restrict__ u, const float* __restrict__ v,
                                                           int R, int P, float dt0,
-                                                          const unsigned* __restrict__ max_bits, int slots, int per) {
+                                                          const unsigned* __restrict__ max_bits, WindowBands bands) {
     const int W = scatter_radius(max_bits, dt0, R);
     if (W > kWindow) return;
-    const WindowLayout L = window_layout(R, W, slots);
+    const int band = W == 1 ? bands.rows[0] : (W == 2 ? bands.rows[1] : (W == 3 ? bands.rows[2] : bands.rows[3]));
+    const WindowLayout L = window_layout(R, W, band);
+    const int per = (L.waves + 8 * kStripWaves - 1) / (8 * kStripWaves);
+    if ((int)(blockIdx.x >> 3) >= per) return;
     const int item = ((int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3)) * kStripWaves + (int)(threadIdx.x >> 6);
     if (item >= L.waves) return;  // whole waves leave; no block-wide barrier follows
     const int lane = threadIdx.x & 63;
@@ -282,22 +312,29 @@ __global__ __launch_bounds__(NT, 6) void k_scatter_window(float* __restrict__ ou
     }
 }
 
-// Waves of k_scatter_window resident at once on the current device (queried
-// once per device).
-int window_slots() {
+// Waves of k_scatter_window resident at once on the current device, and the device's
+// SIMDs (queried once per device).
+void window_slots(int* slots, int* simds) {
     constexpr int kMaxDev = 64;
-    static int slots[kMaxDev] = {};
+    static int known_slots[kMaxDev] = {}, known_simds[kMaxDev] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) dev = -1;
-    if (dev >= 0 && slots[dev] > 0) return slots[dev];
+    if (dev >= 0 && known_slots[dev] > 0 && known_simds[dev] > 0) {
+        *slots = known_slots[dev];
+        *simds = known_simds[dev];
+        return;
+    }
     int cus = 0, blocks = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev < 0 ? 0 : dev) != hipSuccess || cus < 1)
         cus = 256;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_scatter_window, NT, 0) != hipSuccess || blocks < 1)
         blocks = 1;
-    const int n = cus * blocks * kStripWaves;
-    if (dev >= 0) slots[dev] = n;
-    return n;
+    *slots = cus * blocks * kStripWaves;
+    *simds = cus * 4;
+    if (dev >= 0) {
+        known_slots[dev] = *slots;
+        known_simds[dev] = *simds;
+    }
 }
 
 // ---- sorted path ---------------------------------------------------------------
@@ -762,12 +799,16 @@ size_t scatter_sort_bytes(int R) {
 hipError_t launch_scatter_density(hipStream_t s, float* out, const float* rho0, const float* u, const float* v, int R,
                                   int P, float dt0, const unsigned* max_bits, void* sort_scratch) {
     const int n = R - 2;
-    const int slots = window_slots();
+    int slots = 0, simds = 0;
+    window_slots(&slots, &simds);
+    WindowBands bands;
     int waves = 0;  // the most any radius of the window path takes
-    for (int W = 1; W <= kWindow; ++W) waves = std::max(waves, window_layout(R, W, slots).waves);
-    const int blocks = (waves + kStripWaves - 1) / kStripWaves, per = (blocks + 7) / 8;
-    hipLaunchKernelGGL(k_scatter_window, dim3(8 * per), dim3(NT), 0, s, out, rho0, u, v, R, P, dt0, max_bits, slots,
-                       per);
+    for (int W = 1; W <= kWindow; ++W) {
+        bands.rows[W - 1] = window_band_rows(R, W, slots, simds);
+        waves = std::max(waves, window_layout(R, W, bands.rows[W - 1]).waves);
+    }
+    const int per = (waves + 8 * kStripWaves - 1) / (8 * kStripWaves);
+    hipLaunchKernelGGL(k_scatter_window, dim3(8 * per), dim3(NT), 0, s, out, rho0, u, v, R, P, dt0, max_bits, bands);
     if (!sort_scratch) return hipGetLastError();
     // sorted path (returns at once while the window path is active)
     const long long N = (long long)n * n;
