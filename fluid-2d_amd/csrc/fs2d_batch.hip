@@ -171,6 +171,49 @@ __global__ __launch_bounds__(CBX* CBY) void kb_gradient(const BatchSim* __restri
 // made by the last launch, 40 steps and their read-back took 106.0 ms against 101.9.
 constexpr int JB_WAVES = 8;
 
+// Launch j's job of one field: what it reads and writes, and the divisor; whether that
+// is a checked one.
+template <int KIND, bool FIRST>
+__device__ __forceinline__ bool batch_job(const BatchSim& S, const Roles& r, int f, int j, jac::TileJob& t) {
+    const size_t o = S.off;
+    t.R = S.R;
+    t.P = S.P;
+    bool checked = false;
+    float *home, *s1, *s2;
+    if (KIND == SWEEP_PRESSURE) {
+        home = r.a[A_P] + o;
+        t.b = r.a[A_D] + o;
+        s1 = r.a[A_S1A] + o;
+        s2 = r.a[A_S2A] + o;
+        t.rg = ring_of(BND_CONT);
+        t.a = 0.f;
+        t.dv = jac::Divisor{};
+        t.s0 = r.a[A_U] + o;
+        t.s1 = r.a[A_V] + o;
+        t.scale = S.neg_half_h;
+        t.b_out = r.a[A_D] + o;
+    } else {
+        home = r.a[f == 0 ? A_RHO : (f == 1 ? A_UN : A_VN)] + o;
+        t.b = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
+        s1 = r.a[f == 0 ? A_S1A : (f == 1 ? A_S1B : A_S1C)] + o;
+        s2 = r.a[f == 0 ? A_S2A : (f == 1 ? A_S2B : A_S2C)] + o;
+        t.rg = ring_of(f == 0 ? BND_CONT : (f == 1 ? BND_OPP_H : BND_OPP_V));
+        t.a = f == 0 ? S.a_rho : S.a_vel;
+        t.dv = f == 0 ? S.dv_rho : S.dv_vel;
+        checked = (f == 0 ? S.checked_rho : S.checked_vel) != 0;
+        // u and v go to fresh iterates: the density scatter reads the pre-step
+        // velocity (:16-24)
+        t.src = r.a[f == 0 ? A_RHO : (f == 1 ? A_U : A_V)] + o;
+        t.s0 = r.a[f == 0 ? A_RS : (f == 1 ? A_US : A_VS)] + o;
+        t.scale = S.dt;
+        t.b_out = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
+    }
+    if (!FIRST) t.src = ((j - 1) & 1) ? s2 : s1;
+    t.dst = (j == S.launches - 1) ? home : ((j & 1) ? s2 : s1);
+    t.zero = false;
+    return checked;
+}
+
 // A solve's first launch (FIRST, j = 0) forms its right-hand sides: the sources' terms
 // of density, u and v, or the divergence.
 template <int RPW, int KIND, bool FIRST>
@@ -182,43 +225,8 @@ __global__ __launch_bounds__(64 * JB_WAVES) void kb_jacobi(const BatchSim* __res
         const int2 w = work[e];
         const int s = w.x & 0xffffff, f = w.x >> 24;
         const BatchSim& S = sims[s];
-        const size_t o = S.off;
         jac::TileJob t;
-        t.R = S.R;
-        t.P = S.P;
-        bool checked = false;
-        float *home, *s1, *s2;
-        if (KIND == SWEEP_PRESSURE) {
-            home = r.a[A_P] + o;
-            t.b = r.a[A_D] + o;
-            s1 = r.a[A_S1A] + o;
-            s2 = r.a[A_S2A] + o;
-            t.rg = ring_of(BND_CONT);
-            t.a = 0.f;
-            t.dv = jac::Divisor{};
-            t.s0 = r.a[A_U] + o;
-            t.s1 = r.a[A_V] + o;
-            t.scale = S.neg_half_h;
-            t.b_out = r.a[A_D] + o;
-        } else {
-            home = r.a[f == 0 ? A_RHO : (f == 1 ? A_UN : A_VN)] + o;
-            t.b = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
-            s1 = r.a[f == 0 ? A_S1A : (f == 1 ? A_S1B : A_S1C)] + o;
-            s2 = r.a[f == 0 ? A_S2A : (f == 1 ? A_S2B : A_S2C)] + o;
-            t.rg = ring_of(f == 0 ? BND_CONT : (f == 1 ? BND_OPP_H : BND_OPP_V));
-            t.a = f == 0 ? S.a_rho : S.a_vel;
-            t.dv = f == 0 ? S.dv_rho : S.dv_vel;
-            checked = (f == 0 ? S.checked_rho : S.checked_vel) != 0;
-            // u and v go to fresh iterates: the density scatter reads the pre-step
-            // velocity (:16-24)
-            t.src = r.a[f == 0 ? A_RHO : (f == 1 ? A_U : A_V)] + o;
-            t.s0 = r.a[f == 0 ? A_RS : (f == 1 ? A_US : A_VS)] + o;
-            t.scale = S.dt;
-            t.b_out = r.a[f == 0 ? A_X0 : (f == 1 ? A_X0U : A_X0V)] + o;
-        }
-        if (!FIRST) t.src = ((j - 1) & 1) ? s2 : s1;
-        t.dst = (j == S.launches - 1) ? home : ((j & 1) ? s2 : s1);
-        t.zero = false;
+        const bool checked = batch_job<KIND, FIRST>(S, r, f, j, t);
         // tiles are placed for the longest launch
         t.m = S.sweeps + (S.longer > 0);
         const int tiles_y = jac::tile_count(t.R, RPW * JB_WAVES, t.m), tiles_x = jac::tile_count(t.R, jac::kTileCols, t.m);
@@ -233,6 +241,93 @@ __global__ __launch_bounds__(64 * JB_WAVES) void kb_jacobi(const BatchSim* __res
             jac::jacobi_tile_any<RPW, JB_WAVES, jac::TILE_DIFFUSE, FIRST ? jac::TILE_SOURCES : jac::TILE_STORED>(t, ex);
         __syncthreads();  // the next tile's first exchange may take the buffer of this one's last
     }
+}
+
+// A launch of M = 1 or 2 sweeps that is not a solve's first, one wave a strip: lane l
+// holds column gj0 + l of a 64-column region and its kStripRows + 2M rows in registers.
+// Each sweep leaves one more row and lane a side stale; rows M .. and lanes M .. 63 - M
+// are written.  Region cells outside the grid hold clamped values that reach only other
+// outside cells or the ring, which is rebuilt from the new interior after a sweep.
+//
+// What bounds it: memory, at one or two sweeps a pass.  A block tile's waves wait for
+// each other each sweep and its rows past the grid's are relaxed in vain, which so few
+// sweeps do not pay back.  A step by tiles and by strips, us: 300 grids of 66 x 66, 20
+// sweeps, 1 a launch 1099 and 711, 2 a launch 632 and 511; 512 of 98 x 98, 16 sweeps,
+// 1940 and 1349, 1166 and 934; 256 of sides 64 to 512 9292 and 8669, 5007 and 4846; one
+// of 4098 x 4098 4277 and 4065, 2430 and 2419.  From 4 sweeps a launch on tiles win
+// (256 grids: 2941 us).  Strips of 32 rows take the same time.
+constexpr int kStripRows = 16, kStripWaves = 4;
+
+__host__ __device__ inline int strip_count(int R, int m) {
+    const int n = R - 2, cols = 64 - 2 * m;
+    return ((n + cols - 1) / cols) * ((n + kStripRows - 1) / kStripRows);
+}
+
+template <int M, int KIND, bool EDGE>
+__device__ __forceinline__ void batch_strip(const jac::TileJob& t, int gi0, int gj0, int lane) {
+    constexpr int H = kStripRows + 2 * M;
+    const int R = t.R, P = t.P, n = R - 2, gj = gj0 + lane;
+    float X[H], B[H];
+    if (EDGE) {
+        const int cj = min(max(gj, 0), R - 1), bj = min(max(gj, 1), n);
+#pragma unroll
+        for (int q = 0; q < H; ++q) X[q] = t.src[(size_t)min(max(gi0 + q, 0), R - 1) * P + cj];
+#pragma unroll
+        for (int q = 1; q < H - 1; ++q) B[q] = t.b[(size_t)min(max(gi0 + q, 1), n) * P + bj];
+    } else {
+        const size_t o = (size_t)gi0 * P + gj;
+#pragma unroll
+        for (int q = 0; q < H; ++q) X[q] = t.src[o + (size_t)q * P];
+#pragma unroll
+        for (int q = 1; q < H - 1; ++q) B[q] = t.b[o + (size_t)q * P];
+    }
+    const bool cols_ring = EDGE && (gj0 <= 0 || gj0 + 63 >= R - 1);  // the same in all lanes
+#pragma unroll
+    for (int s = 1; s <= M; ++s) {
+        float north = X[s - 1];
+#pragma unroll
+        for (int q = s; q < H - s; ++q) {
+            const float c = X[q];
+            float v = jac::relax_k<KIND>(B[q], north, X[q + 1], jac::lane_west(c), jac::lane_east(c), t.a, t.dv);
+            north = c;
+            if (EDGE && s < M) {
+                const int gi = gi0 + q;
+                if (gi == R - 1) v = jac::sgn(t.rg.neg_tb, X[q - 1]);
+                if (cols_ring) {
+                    const float e = jac::sgn(t.rg.neg_lr, jac::lane_east(v)), w = jac::sgn(t.rg.neg_lr, jac::lane_west(v));
+                    v = gj == 0 ? e : (gj == R - 1 ? w : v);
+                }
+                if (gi == 1) X[q - 1] = jac::sgn(t.rg.neg_tb, v);
+            }
+            X[q] = v;
+        }
+    }
+    if (lane < M || lane >= 64 - M || gj > n) return;  // gj >= 1: a strip starts at column 1 - M
+#pragma unroll
+    for (int q = M; q < M + kStripRows; ++q) {
+        const int gi = gi0 + q;
+        if (EDGE && gi > n) continue;
+        t.dst[(size_t)gi * P + gj] = X[q];
+        if (EDGE) cells::write_ring(t.dst, gi, gj, X[q], R, P, t.rg);
+    }
+}
+
+// Entries as kb_jacobi's, the strips of a field row-major.
+template <int M, int KIND>
+__global__ __launch_bounds__(64 * kStripWaves) void kb_strip(const BatchSim* __restrict__ sims,
+                                                             const int2* __restrict__ work, int n_work, Roles r, int j) {
+    const int e = xcd_block(blockIdx.x, gridDim.x) * kStripWaves + (threadIdx.x >> 6);
+    if (e >= n_work) return;  // whole wave; no barrier follows
+    const int2 w = work[e];
+    const BatchSim& S = sims[w.x & 0xffffff];
+    jac::TileJob t;
+    batch_job<KIND, false>(S, r, w.x >> 24, j, t);
+    constexpr int cols = 64 - 2 * M;
+    const int across = (t.R - 2 + cols - 1) / cols, ty = w.y / across;
+    const int gi0 = 1 + kStripRows * ty - M, gj0 = 1 + cols * (w.y - ty * across) - M, lane = threadIdx.x & 63;
+    const bool plain = gi0 >= 1 && gi0 + kStripRows + 2 * M - 1 <= t.R - 2 && gj0 >= 1 && gj0 + 63 <= t.R - 2;
+    if (plain) batch_strip<M, KIND, false>(t, gi0, gj0, lane);
+    else batch_strip<M, KIND, true>(t, gi0, gj0, lane);
 }
 
 __global__ __launch_bounds__(256) void kb_fill(uint32_t* __restrict__ p, size_t n) {
@@ -274,6 +369,15 @@ hipError_t launch_kb_jacobi(hipStream_t st, int rows, int kind, const BatchSim* 
     return hipGetLastError();
 }
 
+template <int M>
+hipError_t launch_kb_strip(hipStream_t st, int kind, const BatchSim* sims, const int2* w, int n, Roles r, int j) {
+    if (n <= 0) return hipSuccess;
+    const dim3 grid((n + kStripWaves - 1) / kStripWaves), block(64 * kStripWaves);
+    if (kind == SWEEP_DIFFUSE) hipLaunchKernelGGL((kb_strip<M, SWEEP_DIFFUSE>), grid, block, 0, st, sims, w, n, r, j);
+    else hipLaunchKernelGGL((kb_strip<M, SWEEP_PRESSURE>), grid, block, 0, st, sims, w, n, r, j);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 // The work lists of the diffuse (3 fields) and pressure (1 field) solves with,
@@ -283,6 +387,11 @@ struct JacobiWork {
     int2* diffuse = nullptr;
     int2* pressure = nullptr;
     std::vector<int> diffuse_count, pressure_count;  // per launch j
+    // the same for the launches after a solve's first where they take strips
+    int strip_sweeps = 0;  // 0: they take tiles
+    int2* diffuse_strips = nullptr;
+    int2* pressure_strips = nullptr;
+    std::vector<int> diffuse_strip_count, pressure_strip_count;
 };
 
 struct BatchGraph {
@@ -345,42 +454,63 @@ float cells_of(int R) { return static_cast<float>(static_cast<size_t>(R) * stati
 int jac_limit(const fs2d_batch* b) { return b->jac_per_cu > 0 ? b->cus * b->jac_per_cu : 0; }
 dim3 cell_grid(const fs2d_batch* b) { return dim3(persistent_grid(b->cell_blocks, 1, b->cell_per_cu > 0 ? b->cus * b->cell_per_cu : 0)); }
 
-// Work lists of the Jacobi launches.  Entries are ordered by the simulation's
-// launch count (descending), so launch j takes a prefix.  Rows of a tile's region:
-// as for one grid (fs2d_jacobi.hip), by the cells of a diffuse launch.
+// One solve kind's work list (`fields` fields a simulation, tiles(S) entries a field),
+// and the prefix of it that launch j takes: entries are ordered by the simulation's
+// launch count (descending).
+template <class F>
+hipError_t build_work(const fs2d_batch* b, int fields, F&& tiles, int2** list, std::vector<int>* counts) {
+    std::vector<int2> w;
+    for (int s : b->order) {
+        const BatchSim& S = b->host_sims[s];
+        const int n = tiles(S);
+        for (int f = 0; f < fields; ++f)
+            for (int t = 0; t < n; ++t) w.push_back(make_int2(s | (f << 24), t));
+        if (counts->empty()) counts->assign(S.launches, 0);  // the first has the most launches
+        for (int j = 0; j < S.launches; ++j) (*counts)[j] += fields * n;
+    }
+    const hipError_t e = hipMalloc(list, sizeof(int2) * w.size());
+    return e != hipSuccess ? e : hipMemcpy(*list, w.data(), sizeof(int2) * w.size(), hipMemcpyHostToDevice);
+}
+
+// Tiles of one field of a simulation whose regions are `rows` high.
+int tiles_of(const BatchSim& S, int rows) {
+    const int m = S.sweeps + (S.longer > 0);
+    return jac::tile_count(S.R, rows, m) * jac::tile_count(S.R, jac::kTileCols, m);
+}
+
+// Work lists of the Jacobi launches.  Rows of a tile's region: as for one grid
+// (fs2d_jacobi.hip), by the cells of a diffuse launch.  Fixed launches of 1 or 2 sweeps
+// take strips after a solve's first one.
 hipError_t build_jacobi_work(fs2d_batch* b) {
     JacobiWork& c = b->jacobi;
     c.rows = 3 * b->interior < 500000 ? 32 : (3 * b->interior < 8000000 ? 48 : 96);
-    std::vector<int2> dw, pw;
-    for (int s : b->order) {
-        const BatchSim& S = b->host_sims[s];
-        const int m = S.sweeps + (S.longer > 0);
-        const int tiles = jac::tile_count(S.R, c.rows, m) * jac::tile_count(S.R, jac::kTileCols, m);
-        for (int f = 0; f < 3; ++f)
-            for (int t = 0; t < tiles; ++t) dw.push_back(make_int2(s | (f << 24), t));
-        for (int t = 0; t < tiles; ++t) pw.push_back(make_int2(s, t));
-        if (c.diffuse_count.empty()) {  // the first has the most launches
-            c.diffuse_count.assign(S.launches, 0);
-            c.pressure_count.assign(S.launches, 0);
-        }
-        for (int j = 0; j < S.launches; ++j) {
-            c.diffuse_count[j] += 3 * tiles;
-            c.pressure_count[j] += tiles;
-        }
-    }
+    const auto tiles = [&](const BatchSim& S) { return tiles_of(S, c.rows); };
     hipError_t e;
-    if ((e = hipMalloc(&c.diffuse, sizeof(int2) * dw.size())) != hipSuccess) return e;
-    if ((e = hipMalloc(&c.pressure, sizeof(int2) * pw.size())) != hipSuccess) return e;
-    if ((e = hipMemcpy(c.diffuse, dw.data(), sizeof(int2) * dw.size(), hipMemcpyHostToDevice)) != hipSuccess) return e;
-    return hipMemcpy(c.pressure, pw.data(), sizeof(int2) * pw.size(), hipMemcpyHostToDevice);
+    if ((e = build_work(b, 3, tiles, &c.diffuse, &c.diffuse_count)) != hipSuccess) return e;
+    if ((e = build_work(b, 1, tiles, &c.pressure, &c.pressure_count)) != hipSuccess) return e;
+    const int m = b->prm.jacobi_block;
+    if (m != 1 && m != 2) return hipSuccess;
+    c.strip_sweeps = m;
+    const auto strips = [&](const BatchSim& S) { return strip_count(S.R, m); };
+    if ((e = build_work(b, 3, strips, &c.diffuse_strips, &c.diffuse_strip_count)) != hipSuccess) return e;
+    return build_work(b, 1, strips, &c.pressure_strips, &c.pressure_strip_count);
 }
 
 int solve(fs2d_batch* b, int kind) {
     const JacobiWork& c = b->jacobi;
-    const auto& counts = kind == SWEEP_DIFFUSE ? c.diffuse_count : c.pressure_count;
-    const int2* w = kind == SWEEP_DIFFUSE ? c.diffuse : c.pressure;
-    for (int j = 0; j < static_cast<int>(counts.size()); ++j)
-        FS2D_BHIP(b, launch_kb_jacobi(b->stream, c.rows, kind, b->sims, w, counts[j], b->roles, j, jac_limit(b)));
+    const bool diffuse = kind == SWEEP_DIFFUSE;
+    const auto& counts = diffuse ? c.diffuse_count : c.pressure_count;
+    const auto& strips = diffuse ? c.diffuse_strip_count : c.pressure_strip_count;
+    const int2* w = diffuse ? c.diffuse : c.pressure;
+    const int2* ws = diffuse ? c.diffuse_strips : c.pressure_strips;
+    for (int j = 0; j < static_cast<int>(counts.size()); ++j) {
+        if (j == 0 || !c.strip_sweeps)
+            FS2D_BHIP(b, launch_kb_jacobi(b->stream, c.rows, kind, b->sims, w, counts[j], b->roles, j, jac_limit(b)));
+        else if (c.strip_sweeps == 1)
+            FS2D_BHIP(b, launch_kb_strip<1>(b->stream, kind, b->sims, ws, strips[j], b->roles, j));
+        else
+            FS2D_BHIP(b, launch_kb_strip<2>(b->stream, kind, b->sims, ws, strips[j], b->roles, j));
+    }
     return FS2D_OK;
 }
 
@@ -504,6 +634,8 @@ int fs2d_hip_batch_destroy(fs2d_batch* b) {
     drop_graphs(b);
     if (b->jacobi.diffuse) (void)hipFree(b->jacobi.diffuse);
     if (b->jacobi.pressure) (void)hipFree(b->jacobi.pressure);
+    if (b->jacobi.diffuse_strips) (void)hipFree(b->jacobi.diffuse_strips);
+    if (b->jacobi.pressure_strips) (void)hipFree(b->jacobi.pressure_strips);
     for (float* p : b->roles.a)
         if (p) (void)hipFree(p);
     if (b->sims) (void)hipFree(b->sims);
