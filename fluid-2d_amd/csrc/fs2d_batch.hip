@@ -478,12 +478,30 @@ int tiles_of(const BatchSim& S, int rows) {
     return jac::tile_count(S.R, rows, m) * jac::tile_count(S.R, jac::kTileCols, m);
 }
 
-// Work lists of the Jacobi launches.  Rows of a tile's region: as for one grid
-// (fs2d_jacobi.hip), by the cells of a diffuse launch.  Fixed launches of 1 or 2 sweeps
-// take strips after a solve's first one.
+// Rows of a tile's region: as for one grid (fs2d_jacobi.hip), by the cells of a diffuse
+// launch.  But many grids a little over one region high leave most of their second tile
+// of 96 rows to the first: where regions of 48 rows hold less than 0.85 of the rows those
+// of 96 do, they are the faster ones.  512 grids of 98 x 98, 16 sweeps, a step with 48
+// and 96 rows (0.75): 554 and 619 us; at equal rows 400 of 130 x 130 961 and 886, 50 of
+// 258 x 258 406 and 357, 700 of 66 x 66 604 and 628 us.
+int jacobi_rows(const fs2d_batch* b) {
+    const long long cells = 3 * b->interior;
+    if (cells < 500000) return 32;
+    if (cells < 8000000) return 48;
+    double low = 0, high = 0;  // rows of regions relaxed in a solve
+    for (const BatchSim& S : b->host_sims) {
+        const double sweeps = static_cast<double>(S.launches) * S.sweeps + S.longer;
+        low += sweeps * tiles_of(S, 48) * 48;
+        high += sweeps * tiles_of(S, 96) * 96;
+    }
+    return low < 0.85 * high ? 48 : 96;
+}
+
+// Work lists of the Jacobi launches.  Fixed launches of 1 or 2 sweeps take strips after
+// a solve's first one.
 hipError_t build_jacobi_work(fs2d_batch* b) {
     JacobiWork& c = b->jacobi;
-    c.rows = 3 * b->interior < 500000 ? 32 : (3 * b->interior < 8000000 ? 48 : 96);
+    c.rows = jacobi_rows(b);
     const auto tiles = [&](const BatchSim& S) { return tiles_of(S, c.rows); };
     hipError_t e;
     if ((e = build_work(b, 3, tiles, &c.diffuse, &c.diffuse_count)) != hipSuccess) return e;

@@ -1,6 +1,7 @@
 """Batched Jacobi launches of one and two sweeps, which take strips of 16 rows and 62 or
 60 columns a wave after a solve's first launch, against the oracle, bit for bit: sizes
-at the strips' edges, the fewest sweeps, divisors of every kind, -0 and subnormal cells.
+at the strips' edges, the fewest sweeps, divisors of every kind, -0 and subnormal cells;
+and the height of the tiles of many equal grids.
 """
 from __future__ import annotations
 
@@ -41,3 +42,16 @@ def test_strips(block, oracle_lib):
         b.step_n(2)
         for k, (R, K, dt, diff, visc) in enumerate(sims):
             compare(b.download(k), starts[k], R, K, dt, diff, visc, 2, oracle_lib)
+
+
+@pytest.mark.parametrize("R, count, rows", [(98, 300, 32), (130, 180, 80)])
+def test_height_of_many_equal_grids(R, count, rows, oracle_lib):
+    """9 and 8 million cells of three fields: regions of 48 rows (32 written after 8 sweeps) and of 96."""
+    st = special_values(R, R)
+    with fs2d_amd.Batch([(R, 16, 0.05, 1e-5, 1e-6)] * count) as b:
+        for k in (0, count // 2, count - 1):
+            b.upload(k, *st)
+        b.step_n(1)
+        assert b.info()["tile_rows"] == rows
+        for k in (0, count // 2, count - 1):
+            compare(b.download(k), st, R, 16, 0.05, 1e-5, 1e-6, 1, oracle_lib)
