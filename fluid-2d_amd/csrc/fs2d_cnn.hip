@@ -68,7 +68,8 @@ struct Layer {
 
 // Activation and gradient buffers of one (N, H, W) shape, and how many blocks
 // share each layer's weight gradient (partial sums at `part` of the buffer
-// "part", for training).
+// "part", which the shape's first training step allocates: up to 116 MB that a
+// prediction has no use for).
 struct Acts {
     int N = 0, H = 0, W = 0;
     int splits[kNumLayers] = {};
@@ -273,7 +274,7 @@ int acts_for(fs2d_net* n, int N, int H, int W, Acts** out) {
         {"d3", p3 * 64, 2},  {"c2", p2 * 96, 2},  {"b2", p2 * 32, 2},  {"d2", p2 * 32, 2},
         {"c1", p1 * 48, 2},  {"b1", p1 * 16, 2},  {"d1", p1 * 16, 2},  {"o", p1, 4},
         {"prev", p1, 4},     {"tgt", p1, 4},      {"scale", N, 4},      {"inv", N, 4},
-        {"sums", static_cast<long>(N) * kSumBlocks * 2, 8},             {"part", a->part_floats, 4},
+        {"sums", static_cast<long>(N) * kSumBlocks * 2, 8},
         // gradients
         {"dO", p1 * 16, 2},  {"gA", p1 * 48, 2},  {"gB", p1 * 48, 2},  {"gS1", p1 * 16, 2}, {"gS2", p2 * 32, 2},
         {"gS3", p3 * 64, 2},
@@ -673,6 +674,14 @@ static int fs2d_net_train_step_impl(fs2d_net* net, int n, int h, int w, const fl
     if (!d || !prev || !target || !loss) return nfail(net, FS2D_ERR_ARGUMENT, "fs2d_net_train_step: NULL argument");
     Acts* a = nullptr;
     if ((rc = acts_for(net, n, h, w, &a))) return rc;
+    if (!a->buf.count("part")) {
+        void*& part = a->buf["part"];  // null until it is there: freed like the others
+        const hipError_t e = hipMalloc(&part, sizeof(float) * a->part_floats);
+        if (e != hipSuccess) {
+            a->buf.erase("part");
+            return nfail(net, FS2D_ERR_HIP, std::string("hipMalloc(weight gradients): ") + hipGetErrorString(e));
+        }
+    }
     const long npix = static_cast<long>(n) * h * w;
     if ((rc = load_samples(net, *a, d, prev, target))) return rc;
     if ((rc = forward(net, *a))) return rc;
