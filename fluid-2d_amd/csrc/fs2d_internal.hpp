@@ -198,7 +198,7 @@ hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int P, b
 // in place).
 struct HostStage {
     float* pin = nullptr;  // pinned host memory
-    float* dev = nullptr;  // one unpadded array
+    float* dev = nullptr;  // rows of one unpadded array
     size_t pin_floats = 0, dev_floats = 0;
 };
 hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& c, int R, int P);

@@ -11,9 +11,11 @@
 //     between that buffer, read and written over PCIe, and the fields: one
 //     launch and one wait per call.  Measured: a 256 x 256 array in, 18 us
 //     alone with its launch and wait; 1026 x 1026, 55 us of host copy and 86 us of kernel.
-//   * Larger transfers take hipMemcpyAsync on each whole array (31-35 GB/s in
-//     and 18 GB/s out of pageable memory from 1026 x 1026 up: 134 us in) and a
-//     device buffer of one array.  The two ways cost the same at about 4 MB
+//   * Larger transfers take hipMemcpyAsync on ranges of whole rows (31-35 GB/s in
+//     and 18 GB/s out of pageable memory from 1026 x 1026 up: 134 us in) through a
+//     device buffer of at most kDeviceStage bytes, which bounds what a handle holds
+//     (one array, up to 4 GB, otherwise).  Where no buffer can be had, pitched
+//     copies, which need none.  The two ways cost the same at about 4 MB
 //     an array; the line lies below that, at 8 MB a call, which also bounds
 //     what a handle pins.
 // A caller's pointer is dereferenced here, by the host or a kernel, only where that
@@ -24,12 +26,13 @@
 // peers, and refuses what it cannot copy.
 #include "fs2d_internal.hpp"
 
+#include <algorithm>
 #include <cstring>
 
 namespace fs2d {
 namespace {
 
-constexpr size_t kPinnedStage = size_t(8) << 20;
+constexpr size_t kPinnedStage = size_t(8) << 20, kDeviceStage = size_t(128) << 20;
 
 // Field blockIdx.z, row blockIdx.y.
 __global__ __launch_bounds__(256) void k_copy_rows(RowCopies c, int R, int sp, int dp) {
@@ -85,9 +88,10 @@ hipError_t pitched_copy(hipStream_t s, const RowCopies& c, int k, int R, int sp,
     return hipMemcpy2DAsync(c.dst[k], f * dp, c.src[k], f * sp, f * R, R, kind, s);
 }
 
-hipError_t launch_copy_rows(hipStream_t s, const RowCopies& c, int R, int sp, int dp) {
+// `rows` rows of R floats.
+hipError_t launch_copy_rows(hipStream_t s, const RowCopies& c, int rows, int R, int sp, int dp) {
     if (c.count <= 0) return hipSuccess;
-    const dim3 grid((R + 255) / 256, R, c.count);
+    const dim3 grid((R + 255) / 256, rows, c.count);
     hipLaunchKernelGGL(k_copy_rows, grid, dim3(256), 0, s, c, R, sp, dp);
     return hipGetLastError();
 }
@@ -121,6 +125,20 @@ hipError_t grow(float** p, size_t* have, size_t floats, hipStream_t s, bool pinn
     return hipSuccess;
 }
 
+// grow, as a question.
+bool grown(float** p, size_t* have, size_t floats, hipStream_t s, bool pinned) {
+    if (grow(p, have, floats, s, pinned) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+// Rows of R floats that the device buffer takes; 0 where there is none to be had.
+int stage_rows(HostStage& h, hipStream_t s, int R) {
+    const size_t most = std::max<size_t>(kDeviceStage / sizeof(float) / R, 1);
+    const int rows = static_cast<int>(std::min<size_t>(most, R));
+    return grown(&h.dev, &h.dev_floats, (size_t)rows * R, s, false) ? rows : 0;
+}
+
 }  // namespace
 
 // A later array wins where two destinations overlap, as with copies made one
@@ -139,14 +157,14 @@ hipError_t copy_rows_in_order(hipStream_t s, const RowCopies& c, int R, int P, b
         RowCopies one;
         one.add(c.src[a], c.dst[a]);
         if (!on_device_of(s, in ? c.src[a] : c.dst[a], bytes)) e = pitched_copy(s, c, a, R, sp, dp, hipMemcpyDeviceToDevice);
-        else if (!apart) e = launch_copy_rows(s, one, R, sp, dp);
+        else if (!apart) e = launch_copy_rows(s, one, R, R, sp, dp);
         else {
             together.add(c.src[a], c.dst[a]);
             e = hipSuccess;
         }
         if (e != hipSuccess) return e;
     }
-    return launch_copy_rows(s, together, R, sp, dp);
+    return launch_copy_rows(s, together, R, R, sp, dp);
 }
 
 hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& all, int R, int P) {
@@ -155,21 +173,26 @@ hipError_t stage_in(HostStage& h, hipStream_t s, const RowCopies& all, int R, in
     RowCopies c;
     hipError_t e = copy_registered(s, all, R, R, P, hipMemcpyHostToDevice, &c);
     if (e != hipSuccess || c.count == 0) return e;
-    if (c.count * bytes <= kPinnedStage) {
-        if ((e = grow(&h.pin, &h.pin_floats, c.count * n, s, true)) != hipSuccess) return e;
+    if (c.count * bytes <= kPinnedStage && grown(&h.pin, &h.pin_floats, c.count * n, s, true)) {
         RowCopies d = c;
         for (int k = 0; k < c.count; ++k) {
             std::memcpy(h.pin + k * n, c.src[k], bytes);
             d.src[k] = h.pin + k * n;
         }
-        return launch_copy_rows(s, d, R, R, P);
+        return launch_copy_rows(s, d, R, R, R, P);
     }
-    if ((e = grow(&h.dev, &h.dev_floats, n, s, false)) != hipSuccess) return e;
+    const int rows = stage_rows(h, s, R);
     for (int k = 0; k < c.count; ++k) {
-        RowCopies one;
-        one.add(h.dev, c.dst[k]);
-        if ((e = hipMemcpyAsync(h.dev, c.src[k], bytes, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
-        if ((e = launch_copy_rows(s, one, R, R, P)) != hipSuccess) return e;
+        if (rows == 0 && (e = pitched_copy(s, c, k, R, R, P, hipMemcpyHostToDevice)) != hipSuccess) return e;
+        for (int r = 0; rows && r < R; r += rows) {
+            const int m = std::min(rows, R - r);
+            RowCopies one;
+            one.add(h.dev, c.dst[k] + (size_t)r * P);
+            if ((e = hipMemcpyAsync(h.dev, c.src[k] + (size_t)r * R, sizeof(float) * m * R, hipMemcpyHostToDevice, s)) !=
+                hipSuccess)
+                return e;
+            if ((e = launch_copy_rows(s, one, m, R, R, P)) != hipSuccess) return e;
+        }
     }
     return hipSuccess;
 }
@@ -181,21 +204,26 @@ hipError_t stage_out(HostStage& h, hipStream_t s, const RowCopies& all, int R, i
     hipError_t e = copy_registered(s, all, R, P, R, hipMemcpyDeviceToHost, &c);
     if (e != hipSuccess) return e;
     if (c.count == 0) return hipStreamSynchronize(s);
-    if (c.count * bytes <= kPinnedStage) {
-        if ((e = grow(&h.pin, &h.pin_floats, c.count * n, s, true)) != hipSuccess) return e;
+    if (c.count * bytes <= kPinnedStage && grown(&h.pin, &h.pin_floats, c.count * n, s, true)) {
         RowCopies d = c;
         for (int k = 0; k < c.count; ++k) d.dst[k] = h.pin + k * n;
-        if ((e = launch_copy_rows(s, d, R, P, R)) != hipSuccess) return e;
+        if ((e = launch_copy_rows(s, d, R, R, P, R)) != hipSuccess) return e;
         if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
         for (int k = 0; k < c.count; ++k) std::memcpy(c.dst[k], h.pin + k * n, bytes);
         return hipSuccess;
     }
-    if ((e = grow(&h.dev, &h.dev_floats, n, s, false)) != hipSuccess) return e;
+    const int rows = stage_rows(h, s, R);
     for (int k = 0; k < c.count; ++k) {
-        RowCopies one;
-        one.add(c.src[k], h.dev);
-        if ((e = launch_copy_rows(s, one, R, P, R)) != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(c.dst[k], h.dev, bytes, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+        if (rows == 0 && (e = pitched_copy(s, c, k, R, P, R, hipMemcpyDeviceToHost)) != hipSuccess) return e;
+        for (int r = 0; rows && r < R; r += rows) {
+            const int m = std::min(rows, R - r);
+            RowCopies one;
+            one.add(c.src[k] + (size_t)r * P, h.dev);
+            if ((e = launch_copy_rows(s, one, m, R, P, R)) != hipSuccess) return e;
+            if ((e = hipMemcpyAsync(c.dst[k] + (size_t)r * R, h.dev, sizeof(float) * m * R, hipMemcpyDeviceToHost, s)) !=
+                hipSuccess)
+                return e;
+        }
     }
     return hipStreamSynchronize(s);
 }

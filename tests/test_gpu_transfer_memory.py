@@ -86,3 +86,24 @@ def test_batch_memory():
             assert all(np.array_equal(a, c) for a, c in zip(x, b.download(1)))
             assert L.fs2d_hip_batch_download(b._h, 1, *(t.data_ptr() for t in dst)) == 0
             assert all(np.array_equal(a, t.cpu().numpy()) for a, t in zip(x, dst))
+
+
+def test_a_large_transfer_goes_by_ranges_of_rows():
+    """Arrays past the device buffer's 128 MB (a range of 5592 rows of 6000 and the rest),
+    and what a handle holds for them."""
+    R = 6000
+    rng = np.random.default_rng(3)
+    x = [rng.integers(0, 1 << 20, (R, R), dtype=np.int32).astype(np.float32) for _ in range(3)]
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    with fs2d_amd.Solver(900) as s:  # whatever the runtime allocates for itself is there afterwards
+        s.upload(*(a[:900, :900].copy() for a in x))
+        s.download()
+    with fs2d_amd.Solver(R) as s:
+        before = free()
+        s.upload(*x)
+        assert all(np.array_equal(a, b) for a, b in zip(x, s.download()))
+        assert before - free() <= 132 << 20
