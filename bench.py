@@ -108,7 +108,7 @@ def run_gpu(order: int, n: int, kd: int, kp: int, steps: int, warmup: int, state
     elapsed = time.perf_counter() - t0
     # the step's two relaxations, each timed with HIP events on the solver's
     # own stream around repeated solves (the kernels of the timed steps)
-    out = {"sec_step": elapsed / steps, "launches": s.launches_per_step()}
+    out = {"sec_step": elapsed / steps, "launches": s.step_launches()}
     if time_solve:
         reps = max(3, min(20, int(0.5 / max(elapsed / steps / 5, 1e-4))))
         out["ms_pressure"] = s.time_pressure_sweeps(reps)
@@ -171,11 +171,12 @@ def run_batch(count: int, steps: int, warmup: int):
         b.sync()
         sec = (time.perf_counter() - t0) / steps
         info = b.info()
+        launched = b.step_launches()
     cells = info["interior_cells"]
     return {"simulations": count, "interior_cells": cells, "steps": steps, "value": round(1.0 / sec, 2),
             "unit": "steps/s (all simulations)", "ms_per_step": round(sec * 1e3, 3),
-            "cell_updates_per_s": round(cells / sec, 1), "jacobi_depth": info["jacobi_depth"],
-            "tile_rows": info["tile_rows"], "launches_per_step": info["launches_per_step"],
+            "cell_updates_per_s": round(cells / sec, 1), "sweeps_per_launch": [launched["fewest_sweeps"], launched["most_sweeps"]],
+            "tile_rows": info["tile_rows"], "launches_per_step": launched["launches"],
             "persistent_blocks_per_cu": {"jacobi": info["jacobi_blocks_per_cu"], "stages": info["stage_blocks_per_cu"],
                                          "note": "8 waves per Jacobi block, 4 per stage block; 0 = one block per work entry"},
             "graph_replayed": info["graphs"] > 0,

@@ -1415,6 +1415,34 @@ int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches) {
     return guarded(h, "fs2d_hip_launches_per_step", [&] { return fs2d_hip_launches_per_step_impl(h, launches); });
 }
 
+// The next step is captured and dropped, so that the count is of what a step enqueues.
+static int fs2d_hip_step_launches_impl(fs2d_handle* h, int* launches) {
+    if (!h || !launches) return fail(h, FS2D_ERR_ARGUMENT, "fs2d_hip_step_launches: bad argument");
+    if (h->steps_done == 0)  // it builds plans and tunes, which a capture cannot hold
+        return fail(h, FS2D_ERR_STATE, "fs2d_hip_step_launches: only after the first step");
+    float* kept[F_COUNT];
+    std::memcpy(kept, h->f, sizeof kept);
+    const bool speed = h->speed_valid, pzero = h->pressure_zero;
+    FS2D_HIP(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
+    const int rc = step(h, 1e-5f, 1e-6f, 0.01f);
+    hipGraph_t graph = nullptr;
+    size_t n = 0;
+    hipError_t e = hipStreamEndCapture(h->stream, &graph);
+    if (e == hipSuccess) e = hipGraphGetNodes(graph, nullptr, &n);
+    if (graph) (void)hipGraphDestroy(graph);
+    std::memcpy(h->f, kept, sizeof kept);  // nothing of it has run
+    h->speed_valid = speed;
+    h->pressure_zero = pzero;
+    if (rc) return rc;
+    FS2D_HIP(h, e);
+    *launches = static_cast<int>(n);
+    return FS2D_OK;
+}
+
+int fs2d_hip_step_launches(fs2d_handle* h, int* launches) {
+    return guarded(h, "fs2d_hip_step_launches", [&] { return fs2d_hip_step_launches_impl(h, launches); });
+}
+
 // ---- the seeded projection (include/fs2d_cnn.h) ---------------------------
 static int residual_of(fs2d_handle* h, double* rel) {
     if (!h->res_sums) FS2D_HIP(h, hipMalloc(&h->res_sums, 2 * kResidualBlocks * sizeof(double)));

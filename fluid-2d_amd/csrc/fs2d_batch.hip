@@ -917,6 +917,40 @@ static int fs2d_hip_batch_info_impl(fs2d_batch* b, int* depth, int* tile_rows, i
     return FS2D_OK;
 }
 
+// As fs2d_hip_step_launches.
+static int fs2d_hip_batch_step_launches_impl(fs2d_batch* b, int* launches, int* fewest, int* most) {
+    if (!b) return bfail(b, FS2D_ERR_ARGUMENT, "fs2d_hip_batch_step_launches: NULL batch");
+    if (launches) {
+        float* kept[A_COUNT];
+        std::memcpy(kept, b->roles.a, sizeof kept);
+        const bool speed = b->speed_valid;
+        FS2D_BHIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+        const int rc = step(b);
+        hipGraph_t graph = nullptr;
+        size_t n = 0;
+        hipError_t e = hipStreamEndCapture(b->stream, &graph);
+        if (e == hipSuccess) e = hipGraphGetNodes(graph, nullptr, &n);
+        if (graph) (void)hipGraphDestroy(graph);
+        std::memcpy(b->roles.a, kept, sizeof kept);  // nothing of it has run
+        b->speed_valid = speed;
+        if (rc) return rc;
+        FS2D_BHIP(b, e);
+        *launches = static_cast<int>(n);
+    }
+    int lo = b->host_sims[0].sweeps, hi = 0;
+    for (const BatchSim& S : b->host_sims) {
+        lo = std::min(lo, S.sweeps);
+        hi = std::max(hi, S.sweeps + (S.longer > 0));
+    }
+    if (fewest) *fewest = lo;
+    if (most) *most = hi;
+    return FS2D_OK;
+}
+
+int fs2d_hip_batch_step_launches(fs2d_batch* b, int* launches, int* fewest_sweeps, int* most_sweeps) {
+    return guarded(b, "fs2d_hip_batch_step_launches", [&] { return fs2d_hip_batch_step_launches_impl(b, launches, fewest_sweeps, most_sweeps); });
+}
+
 int fs2d_hip_batch_set_occupancy(fs2d_batch* b, int jacobi_blocks_per_cu, int stage_blocks_per_cu) {
     if (!b || jacobi_blocks_per_cu < 0 || jacobi_blocks_per_cu > 64 || stage_blocks_per_cu < 0 ||
         stage_blocks_per_cu > 64)

@@ -103,6 +103,8 @@ def library() -> ctypes.CDLL:
         "fs2d_division_plan": (_i, [_f] + [ctypes.POINTER(_f)] * 5 + [ctypes.POINTER(_i)]),
         "fs2d_hip_gs_policy": (_i, [H, _i, ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_i)]),
         "fs2d_hip_launches_per_step": (_i, [H, ctypes.POINTER(_i)]),
+        "fs2d_hip_step_launches": (_i, [H, ctypes.POINTER(_i)]),
+        "fs2d_hip_batch_step_launches": (_i, [H, ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_i)]),
         "fs2d_hip_last_error": (ctypes.c_char_p, [H]),
         "fs2d_hip_abi_version": (_i, []),
         "fs2d_hip_project_noalloc": (_i, [_i, ctypes.POINTER(Params), _p, _p, _p, _p]),
@@ -286,8 +288,15 @@ class Solver:
         return a.value, b.value
 
     def launches_per_step(self) -> int:
+        """Passes of one step (a launch may serve several, see step_launches)."""
         n = _i()
         self._ck(self._L.fs2d_hip_launches_per_step(self._h, ctypes.byref(n)))
+        return int(n.value)
+
+    def step_launches(self) -> int:
+        """Launches that the next step enqueues (after the first step)."""
+        n = _i()
+        self._ck(self._L.fs2d_hip_step_launches(self._h, ctypes.byref(n)))
         return int(n.value)
 
 
@@ -305,6 +314,7 @@ EXPORTED_SYMBOLS = (
     "fs2d_hip_stage_diffuse", "fs2d_hip_stage_advect_density", "fs2d_hip_stage_advect_velocity",
     "fs2d_hip_stage_project", "fs2d_hip_stage_set_boundary", "fs2d_hip_download_pressure",
     "fs2d_hip_stream", "fs2d_hip_time_pressure_sweeps", "fs2d_hip_time_diffuse_sweeps", "fs2d_hip_time_joint_sweeps", "fs2d_hip_gs_policy", "fs2d_gs_pipeline_offset", "fs2d_division_plan", "fs2d_hip_launches_per_step",
+    "fs2d_hip_step_launches", "fs2d_hip_batch_step_launches",
     "fs2d_hip_last_error", "fs2d_hip_abi_version",
     "fs2d_hip_render_density", "fs2d_hip_render_density_device", "fs2d_hip_render_velocity",
     "fs2d_hip_render_velocity_device", "fs2d_hip_time_render", "fs2d_hip_project_noalloc",
@@ -400,6 +410,12 @@ class Batch:
     def set_occupancy(self, jacobi_blocks_per_cu: int, stage_blocks_per_cu: int) -> None:
         """Fix the persistent launches' blocks per CU (before the first step)."""
         self._ck(self._L.fs2d_hip_batch_set_occupancy(self._h, jacobi_blocks_per_cu, stage_blocks_per_cu))
+
+    def step_launches(self) -> dict:
+        """Launches that the next step enqueues, and the fewest and most sweeps of a Jacobi launch."""
+        n, lo, hi = _i(), _i(), _i()
+        self._ck(self._L.fs2d_hip_batch_step_launches(self._h, ctypes.byref(n), ctypes.byref(lo), ctypes.byref(hi)))
+        return {"launches": n.value, "fewest_sweeps": lo.value, "most_sweeps": hi.value}
 
     def info(self) -> dict:
         d, t, l, g = _i(), _i(), _i(), _i()

@@ -196,13 +196,17 @@ int fs2d_division_plan(float denom, float* inv, float* inv_lo, float* two_hi, fl
  * counted), timed with HIP events over `reps` copies; the achievable HBM
  * figure beside the 8 TB/s peak. */
 int fs2d_hip_copy_bandwidth(long long bytes, int reps, float* gb_per_s);
-/* Number of kernel passes of one step (for per-launch averages): one field, one
- * stage and one sort pass a launch.  Where a launch serves more it counts as often:
- * the Jacobi order's density, u and v together as three, the sources' and the
- * divergence's passes although a solve's first launch makes them, a gradient with a
+/* Number of passes of one step: one field, one stage and one sort pass each.  It is
+ * not the number of launches, since a launch may serve several passes: the Jacobi
+ * order's density, u and v together count as three, the sources' and the divergence's
+ * passes count although a solve's first launch makes them, a gradient with a
  * reduction of the largest speed, which a step's first does without, and a sort pass
- * of the density scatter with its scan. */
+ * of the density scatter with its scan.  For launches, and averages over them, see
+ * fs2d_hip_step_launches. */
 int fs2d_hip_launches_per_step(fs2d_handle* h, int* launches);
+/* Number of launches that the handle's next step enqueues (after the first step only;
+ * nothing runs and nothing changes). */
+int fs2d_hip_step_launches(fs2d_handle* h, int* launches);
 
 /* ---- projection without allocation -------------------------------------
  * No counterpart in the reference; for callers that cannot allocate device
@@ -264,13 +268,17 @@ int fs2d_hip_batch_step_n(fs2d_batch* b, int n);
 /* Wait for the batch's stream, then copy one simulation out (any pointer may be NULL). */
 int fs2d_hip_batch_download(fs2d_batch* b, int sim, float* density, float* u, float* v);
 int fs2d_hip_batch_sync(fs2d_batch* b);
-/* The configuration in use: jacobi_depth, the sweeps every Jacobi launch takes a
- * multiple of (a fixed jacobi_block, else 1: a simulation's sweeps are spread evenly
- * over its launches), tile_rows, the rows an inner Jacobi tile writes after 8 sweeps,
- * passes per step (launches, counting the sources' and the divergences' passes that
- * a solve's first launch makes, and a speed reduction for each gradient), captured step graphs, total interior cells. */
+/* The configuration in use: jacobi_depth, the fixed jacobi_block, else 1 (a
+ * simulation's sweeps are then spread evenly over its launches, see
+ * fs2d_hip_batch_step_launches); tile_rows, the rows an inner Jacobi tile writes after 8
+ * sweeps; passes per step, counted as fs2d_hip_launches_per_step does (0 before the
+ * first step); captured step graphs; total interior cells. */
 int fs2d_hip_batch_info(fs2d_batch* b, int* jacobi_depth, int* tile_rows, int* launches_per_step, int* graphs,
                         long long* interior_cells);
+/* Number of launches that the batch's next step enqueues, and the fewest and the most
+ * sweeps that one of its Jacobi launches takes a simulation through (any pointer may be
+ * NULL; nothing runs and nothing changes). */
+int fs2d_hip_batch_step_launches(fs2d_batch* b, int* launches, int* fewest_sweeps, int* most_sweeps);
 /* The persistent launches' grid: blocks per compute unit for the Jacobi launches (8
  * waves each) and for the single-pass stages (4 waves each; 0: one block per work
  * entry), and the compute units. */
