@@ -405,13 +405,11 @@ struct BatchGraph {
 struct fs2d_batch {
     int count = 0;
     fs2d_params prm{};
-    std::vector<fs2d_batch_sim> spec;
     std::vector<BatchSim> host_sims;
     std::vector<int> order;           // simulations by Jacobi launch count, descending
     size_t arena_floats = 0;
     long long interior = 0;
     hipStream_t stream = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
     HostStage stage;  // host transfers (fs2d_transfer.hip)
     Roles roles{};
     BatchSim* sims = nullptr;     // device copy of host_sims
@@ -665,8 +663,6 @@ int fs2d_hip_batch_destroy(fs2d_batch* b) {
     if (b->scatter_scratch) (void)hipFree(b->scatter_scratch);
     if (b->scatter_flag) (void)hipFree(b->scatter_flag);
     stage_free(b->stage);
-    if (b->ev0) (void)hipEventDestroy(b->ev0);
-    if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
     return FS2D_OK;
@@ -705,7 +701,6 @@ static int fs2d_hip_batch_create_impl(int count, const fs2d_batch_sim* sims, con
     fs2d_batch* b = new fs2d_batch();
     b->count = count;
     b->prm = prm;
-    b->spec.assign(sims, sims + count);
     b->host_sims.resize(count);
     size_t off = 0;
     std::vector<int2> cw, sw;  // single-pass stage blocks; the scatter's window-path waves
@@ -769,8 +764,6 @@ static int fs2d_hip_batch_create_impl(int count, const fs2d_batch_sim* sims, con
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
             b->cus = cus;
     }
-    if ((e = hipEventCreate(&b->ev0)) != hipSuccess) return bail(e, "hipEventCreate");
-    if ((e = hipEventCreate(&b->ev1)) != hipSuccess) return bail(e, "hipEventCreate");
     const size_t bytes = sizeof(float) * off;
     const size_t fill_blocks = std::max<size_t>(1, std::min<size_t>((off + 255) / 256, 4096));
     for (int a = 0; a < A_COUNT; ++a) {

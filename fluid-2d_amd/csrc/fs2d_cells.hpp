@@ -42,28 +42,6 @@ __device__ __forceinline__ void add_sources(float* __restrict__ x, float* __rest
     if (x0) x0[o] = v;
 }
 
-// The same update written to a fresh iterate: out = x + dt*s (interior),
-// x0 = out, and out's ring copied from x (the stale ring the first sweep reads).
-__device__ __forceinline__ void add_sources_split(float* __restrict__ out, float* __restrict__ x0,
-                                                  const float* __restrict__ x, const float* __restrict__ s, int R,
-                                                  int P, float dt, int i, int j) {
-    const size_t o = (size_t)i * P + j;
-    const float v = x[o] + dt * s[o];
-    out[o] = v;
-    x0[o] = v;
-    if (i == 1) out[o - P] = x[o - P];
-    if (i == R - 2) out[o + P] = x[o + P];
-    if (j == 1) out[o - 1] = x[o - 1];
-    if (j == R - 2) out[o + 1] = x[o + 1];
-    if (i == 1 && j == 1) {
-        const size_t last = (size_t)(R - 1) * P;
-        out[0] = x[0];
-        out[R - 1] = x[R - 1];
-        out[last] = x[last];
-        out[last + R - 1] = x[last + R - 1];
-    }
-}
-
 // Largest finite magnitude of a and b folded into m (inf and NaN are skipped).
 __device__ __forceinline__ float fold_speed(float m, float a, float b) {
     a = fabsf(a);

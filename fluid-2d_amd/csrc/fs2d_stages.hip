@@ -30,13 +30,6 @@ __global__ __launch_bounds__(BX* BY) void k_add_sources(float* __restrict__ x, f
     if (interior(R, i, j)) cells::add_sources(x, x0, s, P, dt, i, j);
 }
 
-__global__ __launch_bounds__(BX* BY) void k_add_sources_split(float* __restrict__ out, float* __restrict__ x0,
-                                                              const float* __restrict__ x, const float* __restrict__ s,
-                                                              int R, int P, float dt) {
-    int i, j;
-    if (interior(R, i, j)) cells::add_sources_split(out, x0, x, s, R, P, dt, i, j);
-}
-
 // The step's first stage in one pass (src/fluid_solver_cpu.cpp:16, :21-22 with
 // the copies diffuse takes, :102): density in place, rho += dt * rs, with its
 // copy; u and v into fresh iterates, un = u + dt * us, with their copies, and
@@ -258,12 +251,6 @@ __global__ __launch_bounds__(256) void k_fill(uint32_t* __restrict__ p, uint32_t
 
 hipError_t launch_add_sources(hipStream_t s, float* x, float* x0, const float* src, int R, int P, float dt) {
     hipLaunchKernelGGL(k_add_sources, grid2d(R), dim3(BX, BY), 0, s, x, x0, src, R, P, dt);
-    return hipGetLastError();
-}
-
-hipError_t launch_add_sources_split(hipStream_t s, float* out, float* x0, const float* x, const float* src, int R,
-                                    int P, float dt) {
-    hipLaunchKernelGGL(k_add_sources_split, grid2d(R), dim3(BX, BY), 0, s, out, x0, x, src, R, P, dt);
     return hipGetLastError();
 }
 
