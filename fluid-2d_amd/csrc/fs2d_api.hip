@@ -1577,7 +1577,9 @@ static int fs2d_hip_project_seeded_impl(fs2d_handle* h, fs2d_net* net, int seed,
                     "fs2d_hip_project_seeded: seed 2 needs a network and a side n = rows - 2 that is a multiple of 32");
     const Scalars s = scalars(h->R, 1.0f);
     FS2D_HIP(h, launch_divergence(h->stream, h->f[F_D], h->u(), h->v(), h->R, h->P, s.neg_half_h, nullptr));
-    if (seed == 0 || seed == 3 || h->pressure_zero) FS2D_HIP(h, launch_fill(h->stream, h->f[F_P], 0u, h->field_bytes / 4));
+    // (a multigrid seed's first cycle starts from zero without reading the field)
+    if (seed == 0 || (seed != 3 && h->pressure_zero))
+        FS2D_HIP(h, launch_fill(h->stream, h->f[F_P], 0u, h->field_bytes / 4));
     const bool keep_prev = seed == 2 && fallback;
     if (keep_prev)  // the previous pressure, for the fallback
         FS2D_HIP(h, hipMemcpyAsync(h->f[F_T1], h->f[F_P], h->field_bytes, hipMemcpyDeviceToDevice, h->stream));
