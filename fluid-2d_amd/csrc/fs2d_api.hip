@@ -1232,20 +1232,25 @@ static int fs2d_hip_time_diffuse_sweeps_impl(fs2d_handle* h, float diff, float v
                                  reinterpret_cast<const float4*>(h->f[pr[1]]), n4));
     const float ad = dt * cells(R) * diff, av = dt * cells(R) * visc;
     const float dd = 1.f + 4.f * ad, dv = 1.f + 4.f * av;
-    // the Jacobi order's third free field, for the timing only
-    const bool spare_needed = h->prm.sweep_order == FS2D_ORDER_JACOBI && shares_diffuses(h);
+    // the Jacobi order's third free field, for the timing only; where there is no memory
+    // for it the fields are timed one after the other
+    const bool jacobi = h->prm.sweep_order == FS2D_ORDER_JACOBI;
     float* spare = nullptr;
-    if (spare_needed) FS2D_HIP(h, hipMalloc(&spare, h->field_bytes));
+    if (jacobi && shares_diffuses(h) && hipMalloc(&spare, h->field_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        spare = nullptr;
+    }
     float* const spare_field = spare;
+    const bool shared = shares_diffuses(h) && (!jacobi || spare_field);
     auto once = [&]() -> int {
         if (Kd <= 0) return FS2D_OK;
-        if (shares_diffuses(h)) {  // as the step relaxes them
+        if (shared) {  // as the step relaxes them
             SweepSet set{};
             set.count = 3;
             set.a[0] = sweep_args(h->f[F_T1], h->f[F_X0], R, P, SWEEP_DIFFUSE, ad, dd, BND_CONT, Kd, 0);
             set.a[1] = sweep_args(h->f[F_UN], h->f[F_X0U], R, P, SWEEP_DIFFUSE, av, dv, BND_OPP_H, Kd, 0);
             set.a[2] = sweep_args(h->f[F_VN], h->f[F_X0V], R, P, SWEEP_DIFFUSE, av, dv, BND_OPP_V, Kd, 0);
-            if (h->prm.sweep_order == FS2D_ORDER_JACOBI) {
+            if (jacobi) {
                 float** const fields[3] = {&h->f[F_T1], &h->f[F_UN], &h->f[F_VN]};
                 float** const scratch[3] = {&h->f[F_SCRATCH], &h->f[F_T2], &spare};
                 return jacobi_solve(h, set, fields, scratch);
@@ -1274,7 +1279,7 @@ static int fs2d_hip_time_diffuse_sweeps_impl(fs2d_handle* h, float diff, float v
         return FS2D_OK;
     };
     const int rc = timed();
-    if (spare_needed) {
+    if (spare_field) {
         (void)hipStreamSynchronize(h->stream);
         if (spare != spare_field) std::swap(h->f[F_VN], spare);  // the handle keeps its own field
         (void)hipFree(spare);
