@@ -11,7 +11,8 @@
 //
 // Each stage is one launch over a work list: the single-pass stages over
 // (simulation, 64 x 4 cell block) entries, the Jacobi sweeps over
-// (simulation, field, tile) entries with the block tile of the one-grid solver.
+// (simulation, field, tile) entries with the block tile of the one-grid solver, or, in
+// fixed launches of one or two sweeps, over (simulation, field, strip) entries.
 // Simulation s runs its K_s sweeps in L_s launches of at most 8 fused sweeps,
 // as evenly as they go; launch j covers the simulations with more than j
 // launches (the work list is ordered by launch count, so that is a prefix of
@@ -312,22 +313,26 @@ __device__ __forceinline__ void batch_strip(const jac::TileJob& t, int gi0, int 
     }
 }
 
-// Entries as kb_jacobi's, the strips of a field row-major.
-template <int M, int KIND>
+// Entries as kb_jacobi's, the strips of a field row-major.  LOOP: persistent by waves,
+// else an entry a wave (the loop's code cost launches of one sweep 5 %).
+template <int M, int KIND, bool LOOP>
 __global__ __launch_bounds__(64 * kStripWaves) void kb_strip(const BatchSim* __restrict__ sims,
                                                              const int2* __restrict__ work, int n_work, Roles r, int j) {
-    const int e = xcd_block(blockIdx.x, gridDim.x) * kStripWaves + (threadIdx.x >> 6);
-    if (e >= n_work) return;  // whole wave; no barrier follows
-    const int2 w = work[e];
-    const BatchSim& S = sims[w.x & 0xffffff];
-    jac::TileJob t;
-    batch_job<KIND, false>(S, r, w.x >> 24, j, t);
-    constexpr int cols = 64 - 2 * M;
-    const int across = (t.R - 2 + cols - 1) / cols, ty = w.y / across;
-    const int gi0 = 1 + kStripRows * ty - M, gj0 = 1 + cols * (w.y - ty * across) - M, lane = threadIdx.x & 63;
-    const bool plain = gi0 >= 1 && gi0 + kStripRows + 2 * M - 1 <= t.R - 2 && gj0 >= 1 && gj0 + 63 <= t.R - 2;
-    if (plain) batch_strip<M, KIND, false>(t, gi0, gj0, lane);
-    else batch_strip<M, KIND, true>(t, gi0, gj0, lane);
+    const int lane = threadIdx.x & 63, waves = (int)gridDim.x * kStripWaves;
+    // (no barrier: a wave leaves when its entries are done)
+    for (int e = xcd_block(blockIdx.x, gridDim.x) * kStripWaves + (threadIdx.x >> 6); e < n_work; e += waves) {
+        const int2 w = work[e];
+        const BatchSim& S = sims[w.x & 0xffffff];
+        jac::TileJob t;
+        batch_job<KIND, false>(S, r, w.x >> 24, j, t);
+        constexpr int cols = 64 - 2 * M;
+        const int across = (t.R - 2 + cols - 1) / cols, ty = w.y / across;
+        const int gi0 = 1 + kStripRows * ty - M, gj0 = 1 + cols * (w.y - ty * across) - M;
+        const bool plain = gi0 >= 1 && gi0 + kStripRows + 2 * M - 1 <= t.R - 2 && gj0 >= 1 && gj0 + 63 <= t.R - 2;
+        if (plain) batch_strip<M, KIND, false>(t, gi0, gj0, lane);
+        else batch_strip<M, KIND, true>(t, gi0, gj0, lane);
+        if (!LOOP) return;
+    }
 }
 
 __global__ __launch_bounds__(256) void kb_fill(uint32_t* __restrict__ p, size_t n) {
@@ -369,12 +374,19 @@ hipError_t launch_kb_jacobi(hipStream_t st, int rows, int kind, const BatchSim* 
     return hipGetLastError();
 }
 
+template <int M, int KIND>
+void launch_kb_strip_kind(hipStream_t st, const BatchSim* sims, const int2* w, int n, Roles r, int j, int limit) {
+    const dim3 grid(persistent_grid(n, kStripWaves, limit)), block(64 * kStripWaves);
+    if (limit > 0) hipLaunchKernelGGL((kb_strip<M, KIND, true>), grid, block, 0, st, sims, w, n, r, j);
+    else hipLaunchKernelGGL((kb_strip<M, KIND, false>), grid, block, 0, st, sims, w, n, r, j);
+}
+
 template <int M>
-hipError_t launch_kb_strip(hipStream_t st, int kind, const BatchSim* sims, const int2* w, int n, Roles r, int j) {
+hipError_t launch_kb_strip(hipStream_t st, int kind, const BatchSim* sims, const int2* w, int n, Roles r, int j,
+                           int limit) {
     if (n <= 0) return hipSuccess;
-    const dim3 grid((n + kStripWaves - 1) / kStripWaves), block(64 * kStripWaves);
-    if (kind == SWEEP_DIFFUSE) hipLaunchKernelGGL((kb_strip<M, SWEEP_DIFFUSE>), grid, block, 0, st, sims, w, n, r, j);
-    else hipLaunchKernelGGL((kb_strip<M, SWEEP_PRESSURE>), grid, block, 0, st, sims, w, n, r, j);
+    if (kind == SWEEP_DIFFUSE) launch_kb_strip_kind<M, SWEEP_DIFFUSE>(st, sims, w, n, r, j, limit);
+    else launch_kb_strip_kind<M, SWEEP_PRESSURE>(st, sims, w, n, r, j, limit);
     return hipGetLastError();
 }
 
@@ -523,9 +535,9 @@ int solve(fs2d_batch* b, int kind) {
         if (j == 0 || !c.strip_sweeps)
             FS2D_BHIP(b, launch_kb_jacobi(b->stream, c.rows, kind, b->sims, w, counts[j], b->roles, j, jac_limit(b)));
         else if (c.strip_sweeps == 1)
-            FS2D_BHIP(b, launch_kb_strip<1>(b->stream, kind, b->sims, ws, strips[j], b->roles, j));
+            FS2D_BHIP(b, launch_kb_strip<1>(b->stream, kind, b->sims, ws, strips[j], b->roles, j, jac_limit(b)));
         else
-            FS2D_BHIP(b, launch_kb_strip<2>(b->stream, kind, b->sims, ws, strips[j], b->roles, j));
+            FS2D_BHIP(b, launch_kb_strip<2>(b->stream, kind, b->sims, ws, strips[j], b->roles, j, jac_limit(b)));
     }
     return FS2D_OK;
 }

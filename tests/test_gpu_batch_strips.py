@@ -30,12 +30,14 @@ def compare(got, st, R, K, dt, diff, visc, steps, O):
 
 
 @pytest.mark.parametrize("block", [1, 2])
-def test_strips(block, oracle_lib):
+@pytest.mark.parametrize("per_cu", [0, 1])  # an entry a wave, and waves that walk many
+def test_strips(block, per_cu, oracle_lib):
     sims = [(R, K * block // 2, 0.05, rate, 0.5 * rate) for R, K, rate in SIMS if K * block // 2 >= 2 * block]
     starts = [special_values(s[0], 1000 * s[0] + s[1]) for s in sims]
     for st in starts:
         st[1][::3, ::2] = -0.0
-    with fs2d_amd.Batch(sims, jacobi_block=block) as b:
+    with fs2d_amd.Batch(sims * 4, jacobi_block=block) as b:
+        b.set_occupancy(per_cu, 8)
         for k, st in enumerate(starts):
             b.upload(k, *st)
             b.set_sources(k)
