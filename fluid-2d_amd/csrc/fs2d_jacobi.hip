@@ -79,9 +79,11 @@ hipError_t launch(hipStream_t s, TileSet& S, int fields, int kind) {
 //   before    85.5 / 18.4 86.1 / 18.6 87.2 / 18.8 87.5 / 19.1 150 / 28.9  373 / 62.7
 // Few cells: the launch is a chain of sweeps, and fewer rows a wave are a shorter
 // one.  Many: each 64-column region spends 16 columns and 16 rows on its halo at 8
-// sweeps, so taller is better until too few blocks are left.  At 4098 x 4098 the
-// three fields' launch issues 7.6 VALU operations a cell-sweep (138 us at the halo's
-// 0.62) and moves 0.75 GB (150 us of a copy's rate): both at once take 176.
+// sweeps, so taller is better until too few blocks are left.  At 4098 x 4098, by
+// counters, the three fields' launch executes 9.2 VALU operations a cell-sweep of its
+// regions, 14.7 a written one, at 82 % of the issue slots, and moves 0.66 GB, 3.6 TB/s:
+// issue bounds it, and the halo in it.  A pressure launch executes 9.6 a written
+// cell-sweep and moves 0.21 GB in 41 to 51 us, about a copy's rate.
 // (These were taken before tiles at the grid's edge knew their ring rows and lanes,
 // which took 3 % off a step at 4098 and at 203 and moves no line.)
 // Two or four columns a lane (less halo) measured slower at every size: 184 and

@@ -25,8 +25,8 @@
 //    coordinates (one wave per sweep, lagged; see its comment).
 //
 //  * Jacobi -- every neighbour from the previous iterate.  M sweeps are fused
-//    per launch (temporal blocking).  The default kernel, k_jacobi_wave, keeps
-//    a tile's rows in registers, one wave per tile (fs2d_jacobi.hpp); the
+//    per launch (temporal blocking).  The default kernel, k_jacobi_tile, keeps
+//    a tile's rows in the registers of a block's 8 waves (fs2d_jacobi.hpp); the
 //    alternative, k_jacobi_block, has a 256-thread block load its tile plus an
 //    M-cell halo into LDS once, relax M times in LDS on a shrinking region
 //    (recomputing the ring in LDS after each sweep), and write only the tile.
@@ -259,8 +259,8 @@ struct UnitLds {
     static constexpr int BH = GS_ROWS - 1 + M, BW = TW - 1 + M;   // right-hand side region
     static constexpr int BP = BW + (BW & 1);
     // Guard space after each array absorbs the operand reads of inactive lanes
-    // (their skewed columns run up to GS_ROWS + TW + M past the cell); lanes
-    // that relax nothing in a step store nothing.
+    // (their skewed columns run up to GS_ROWS + TW + M past the cell), and, after
+    // X, the stores of lanes that relax nothing in a step: GS_ROWS + lag words.
     static constexpr int GUARD = GS_ROWS + TW + 2 * M + 8;
     static constexpr int NXS = XH * XP + GUARD, NBS = BH * BP + GUARD;
 };
@@ -486,6 +486,7 @@ __device__ __forceinline__ void gs_unit_run(const SweepArgs& A, const int2 wk, f
     constexpr int STEPS = GS_ROWS + TW - 1;
     constexpr int INTERVALS = (STEPS + L - 1) / L;  // of one wave
     static_assert(GS_ROWS == 64 && TW % 64 == 0 && 64 % L == 0, "the step phases assume 64-row tiles");
+    static_assert(UnitLds<TW, M>::GUARD >= GS_ROWS + L, "idle lanes store to the guard words r + q, q < L");
     const int me0 = (1 + r + (M - 1 - w)) * XP + ofs - r;   // X index of this lane's cell at step s: me0 + s
     const int bme0 = (r + (M - 1 - w)) * BP + ofs - 1 - r;  // Bs index of its right-hand side: bme0 + s
     using Lds = __attribute__((address_space(3))) float*;
@@ -500,7 +501,9 @@ __device__ __forceinline__ void gs_unit_run(const SweepArgs& A, const int2 wk, f
     auto flip = [](float v, unsigned sign) { return __uint_as_float(__float_as_uint(v) ^ sign); };
     // mask ? a : b, in the encoding that names its mask register: with an
     // implicit vcc one such select took 30 clocks, not 5, with 8 waves on a
-    // compute unit (solves 5 % longer)
+    // compute unit (solves 5 % longer).  The compiler puts no wait states before an asm's
+    // operands, and a vector instruction that writes a mask needs two before it is read
+    // here: masks are made by scalar instructions, or by ballots outside the intervals.
     auto pick = [](unsigned long long mask, auto a, auto b) {
         decltype(a) d;
         asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(d) : "v"(b), "v"(a), "s"(mask));
