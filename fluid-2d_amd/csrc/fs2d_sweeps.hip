@@ -1266,21 +1266,23 @@ int gs_pipeline_offset(const GsPlan& pp, int R, int Kd, int TWd, int Md) {
     // through its adjacent interior cell -- is the unit relaxing sweep Kd - 1
     // there: skewed (i + Kd - 1, j + Kd - 1), so level
     // (i + Kd - 2) / 64 + (j + Kd - 2) / TWd + (Kd - 1) / Md, non-decreasing in
-    // i and j.  A pressure unit reads the velocity one cell beyond the
-    // divergence region it loads (rows up to 64 I' - k_lo + 63, columns up to
-    // TW J' - k_lo + TW - 1, clamped into the interior); its last writer is at
-    // that region's far corner.
+    // i and j.  A pressure unit loads the divergence of rows up to
+    // 64 I' - k_lo + 64 and columns up to TW J' - k_lo + TW, clamped into the
+    // interior, and each reads the velocity of its four neighbours: the last
+    // writer is that of the far corner's south or east neighbour.
     const int n = R - 2;
+    auto last_writer = [&](int i, int j) {
+        return (i + Kd - 2) / GS_ROWS + (j + Kd - 2) / TWd + (Kd - 1) / Md;
+    };
     int off = 0;
     for (int L = 0; L < pp.levels; ++L)
         for (int e = pp.host_offsets[L]; e < pp.host_offsets[L + 1]; ++e) {
             const int2 w = pp.host_work[e];
             const int I = w.x >> 16, J = w.x & 0xffff, k_lo = w.y * pp.M;
-            const int ib = std::min(GS_ROWS * I - k_lo + GS_ROWS - 1, n) + 1;
-            const int jb = std::min(pp.TW * J - k_lo + pp.TW - 1, n) + 1;
-            const int ic = std::min(std::max(ib, 1), n), jc = std::min(std::max(jb, 1), n);
-            const int last_writer = (ic + Kd - 2) / GS_ROWS + (jc + Kd - 2) / TWd + (Kd - 1) / Md;
-            off = std::max(off, last_writer + 1 - pp.level_of[L]);
+            const int i = std::min(std::max(GS_ROWS * I - k_lo + GS_ROWS, 1), n);
+            const int j = std::min(std::max(pp.TW * J - k_lo + pp.TW, 1), n);
+            const int last = std::max(last_writer(std::min(i + 1, n), j), last_writer(i, std::min(j + 1, n)));
+            off = std::max(off, last + 1 - pp.level_of[L]);
         }
     return off;
 }
